@@ -1,8 +1,5 @@
 // ljg_force.hip -- Lennard-Jones 12-6 force kernels for gfx950 (wave64).
 //
-//  * k_force_lc_fp64: the plain FP64 kernel.  One lane per particle (cell order), full shell over the 27
-//    neighbour cells of CellBlock3D with periodic image shifts, FP64 pair term written as LJFunctor.h:
-//    288-320, FP64 sums.  No atomics, no Newton-3.
 //  * k_force_cluster<M, FP32>: cluster-pair tiles.  One wave per i-cluster of M particles; the i-cluster
 //    (positions, types) is wave-uniform and lives in scalar registers, the 64 lanes stream the j-particles
 //    of the i-cluster's neighbour-cluster list (M consecutive lanes hold one j-cluster), and every lane
@@ -60,77 +57,6 @@ __device__ inline void block_partials(double e, double v, int64_t h, double *pe,
     ph[blockIdx.x] = sh[0];
     if (acc) acc_add(acc, (unsigned long long)sh[0]);
   }
-}
-
-// ---- plain FP64 linked-cells kernel ------------------------------------------------------------------
-template <bool MIX>
-__global__ __launch_bounds__(kFThreads) void k_force_lc_fp64(
-    int64_t n, const double *__restrict__ x, const double *__restrict__ y, const double *__restrict__ z,
-    const int32_t *__restrict__ type, const int32_t *__restrict__ cell_of, const int64_t *__restrict__ cell_start,
-    CellGeom g, ForceArgs a, const double *__restrict__ tab, double *__restrict__ fx, double *__restrict__ fy,
-    double *__restrict__ fz, double *__restrict__ pe, double *__restrict__ pv, int64_t *__restrict__ ph,
-    int32_t globals, unsigned long long *__restrict__ acc, SkipIf sk, Owned own) {
-  if (skip_launch(sk)) return;
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  double ax = 0., ay = 0., az = 0., ae = 0., av = 0.;
-  int64_t hits = 0;
-  if (i < n) {
-    const double xi = x[i], yi = y[i], zi = z[i];
-    const int ti = MIX ? type[i] : 0;
-    const int32_t c = cell_of[i];
-    const int cx = c % g.nh[0], cy = (c / g.nh[0]) % g.nh[1], cz = c / (g.nh[0] * g.nh[1]);
-    const int no0 = g.nh[0] - 2, no1 = g.nh[1] - 2, no2 = g.nh[2] - 2;
-    for (int oz = -1; oz <= 1; ++oz) {
-      int jz = cz - 1 + oz;
-      double shz = 0.;
-      if (jz < 0) { jz += no2; shz = -g.L[2]; } else if (jz >= no2) { jz -= no2; shz = g.L[2]; }
-      for (int oy = -1; oy <= 1; ++oy) {
-        int jy = cy - 1 + oy;
-        double shy = 0.;
-        if (jy < 0) { jy += no1; shy = -g.L[1]; } else if (jy >= no1) { jy -= no1; shy = g.L[1]; }
-        for (int ox = -1; ox <= 1; ++ox) {
-          int jx = cx - 1 + ox;
-          double shx = 0.;
-          if (jx < 0) { jx += no0; shx = -g.L[0]; } else if (jx >= no0) { jx -= no0; shx = g.L[0]; }
-          const int64_t cidx = ((int64_t)(jz + 1) * g.nh[1] + (jy + 1)) * g.nh[0] + (jx + 1);
-          const int64_t sb = cell_start[cidx], se = cell_start[cidx + 1];
-          for (int64_t j = sb; j < se; ++j) {
-            const double drx = xi - (x[j] + shx);
-            const double dry = yi - (y[j] + shy);
-            const double drz = zi - (z[j] + shz);
-            const double dr2 = drx * drx + dry * dry + drz * drz;
-            double eps24 = a.eps24, sig2 = a.sig2, shift6 = a.shift6;
-            if (MIX) {
-              const int k = ti * a.ntypes + type[j];
-              eps24 = tab[3 * k];
-              sig2 = tab[3 * k + 1];
-              shift6 = tab[3 * k + 2];
-            }
-            const bool mask = dr2 <= a.rc2 && dr2 > 0.;
-            const double invdr2 = 1. / dr2;
-            const double lj2 = sig2 * invdr2;
-            const double lj6 = lj2 * lj2 * lj2;
-            const double lj12 = lj6 * lj6;
-            const double lj12m6 = lj12 - lj6;
-            const double fac = mask ? eps24 * (lj12 + lj12m6) * invdr2 : 0.;
-            ax += drx * fac;
-            ay += dry * fac;
-            az += drz * fac;
-            if (globals) {
-              ae += mask ? eps24 * lj12m6 + shift6 : 0.;
-              av += drx * (drx * fac) + dry * (dry * fac) + drz * (drz * fac);
-            }
-            hits += mask ? 1 : 0;
-          }
-        }
-      }
-    }
-    fx[i] = ax;
-    fy[i] = ay;
-    fz[i] = az;
-    if (globals && !is_owned(own, i)) ae = av = 0.;
-  }
-  block_partials(ae, av, hits, pe, pv, ph, globals != 0, acc);
 }
 
 // ---- cluster-pair tiles -------------------------------------------------------------------------------
@@ -1002,44 +928,6 @@ static ForceArgs make_args(const Ctx &c) {
   a.sig2 = c.lj.sig2[0];
   a.shift6 = c.lj.shift6[0];
   return a;
-}
-
-void lc_force_launch(hipStream_t st, int64_t n, const double *x, const double *y, const double *z,
-                     const int32_t *type, const int32_t *cell_of, const int64_t *cell_start, const CellGeom &g,
-                     double rc2, int32_t ntypes, const double *tab, double eps24, double sig2, double shift6,
-                     double *fx, double *fy, double *fz, double *pe, double *pv, int64_t *ph, bool globals,
-                     unsigned long long *acc, SkipIf skip, Owned own) {
-  ForceArgs a{};
-  for (int d = 0; d < 3; ++d) a.L[d] = g.L[d];
-  a.rc2 = rc2;
-  a.ntypes = ntypes;
-  a.eps24 = eps24;
-  a.sig2 = sig2;
-  a.shift6 = shift6;
-  const int nb = blocks_for(n, kFThreads);
-  if (ntypes > 1)
-    hipLaunchKernelGGL(k_force_lc_fp64<true>, dim3(nb), dim3(kFThreads), 0, st, n, x, y, z, type, cell_of,
-                       cell_start, g, a, tab, fx, fy, fz, pe, pv, ph, (int32_t)globals, acc, skip, own);
-  else
-    hipLaunchKernelGGL(k_force_lc_fp64<false>, dim3(nb), dim3(kFThreads), 0, st, n, x, y, z, type, cell_of,
-                       cell_start, g, a, tab, fx, fy, fz, pe, pv, ph, (int32_t)globals, acc, skip, own);
-  LJG_HIP(hipGetLastError());
-}
-
-void lc_force(Ctx &c, bool globals) {
-  const bool mix = c.lj.ntypes > 1;
-  const double *tab = mix ? c.tab.p : nullptr;
-  const int nb = blocks_for(c.n, kFThreads);
-  c.part_e.ensure(nb);
-  c.part_v.ensure(nb);
-  c.part_hits.ensure(nb);
-  c.part_items = nb;
-  State &s = c.st[c.cur];
-  if (c.timing) LJG_HIP(hipEventRecord(c.ev0, c.stream));
-  lc_force_launch(c.stream, c.n, s.x.p, s.y.p, s.z.p, s.type.p, c.cell_of.p, c.cell_start.p, c.cg, c.lj.rc2,
-                  c.lj.ntypes, tab, c.lj.eps24[0], c.lj.sig2[0], c.lj.shift6[0], s.fx.p, s.fy.p, s.fz.p, c.part_e.p,
-                  c.part_v.p, c.part_hits.p, globals, c.hits_acc, c.skip, owned_of(c));
-  if (c.timing) LJG_HIP(hipEventRecord(c.ev1, c.stream));
 }
 
 __global__ void k_zero_forces(int64_t n, double *__restrict__ fx, double *__restrict__ fy, double *__restrict__ fz,

@@ -481,13 +481,14 @@ CellGeom make_cell_geom(const double lo[3], const double hi[3], double ilen, int
 void cell_bin_launch(hipStream_t st, int64_t n, const double *x, const double *y, const double *z, const CellGeom &g,
                      int32_t *cell_of, int32_t *rank, int32_t *count, const int64_t *start, int32_t *items,
                      const int64_t *id, int32_t *sorted, int phase);
-// The plain FP64 linked-cells kernel on explicit buffers (ljg_force.hip); block partials into pe/pv/ph
-// (blocks_for(n, 256) of them).
-void lc_force_launch(hipStream_t st, int64_t n, const double *x, const double *y, const double *z,
-                     const int32_t *type, const int32_t *cell_of, const int64_t *cell_start, const CellGeom &g,
-                     double rc2, int32_t ntypes, const double *tab, double eps24, double sig2, double shift6,
-                     double *fx, double *fy, double *fz, double *pe, double *pv, int64_t *ph, bool globals,
-                     unsigned long long *acc, SkipIf skip, Owned owned = Owned{nullptr, 0});
+// The plain FP64 linked-cells kernel on explicit buffers in cell order (ljg_lc.hip); block partials into
+// pe/pv/ph (lc_force_blocks(g) of them).
+int64_t lc_force_blocks(const CellGeom &g);
+void lc_force_launch(hipStream_t st, const double *x, const double *y, const double *z, const int32_t *type,
+                     const int64_t *cell_start, const CellGeom &g, double rc2, int32_t ntypes, const double *tab,
+                     double eps24, double sig2, double shift6, double *fx, double *fy, double *fz, double *pe,
+                     double *pv, int64_t *ph, bool globals, unsigned long long *acc, SkipIf skip,
+                     Owned owned = Owned{nullptr, 0});
 // Exclusive scan on a given stream with caller-provided temporary storage of scan_tmp_len(n) entries.
 int64_t scan_tmp_len(int64_t n);  // ljg_md.hip
 void exclusive_scan_i32_to_i64_on(hipStream_t st, const int32_t *in, int64_t *out, int64_t n, int64_t *tmp,
@@ -495,7 +496,7 @@ void exclusive_scan_i32_to_i64_on(hipStream_t st, const int32_t *in, int64_t *ou
 // Deterministic sum of block partials into out[0] (energy x6), out[1] (virial), out_h[0] (pair hits).
 void reduce_launch(hipStream_t st, int64_t nitems, const double *pe, const double *pv, const int64_t *ph,
                    double *out, int64_t *out_h, bool globals);  // ljg_md.hip
-void lc_force(Ctx &c, bool globals);       // ljg_bin.hip (plain FP64 kernel)
+void lc_force(Ctx &c, bool globals);       // ljg_lc.hip (plain FP64 kernel)
 void vcl_build(Ctx &c);                    // ljg_vcl.hip
 // Reads and checks the list lengths of a j-row build that left them pending (true when none is pending):
 // false when a row overflowed or the vetoed force launch assumed a frame the rows leave, in which case

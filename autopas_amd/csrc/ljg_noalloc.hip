@@ -144,7 +144,7 @@ ljg_status ljg_force_lc_noalloc(const ljg_params *params, int32_t ntypes, const 
   int64_t ncells = 0;
   const CellGeom g = make_cell_geom(params->box_min, params->box_max, ilen, &ncells);
   if (ncells > LJG_NOALLOC_MAX_CELLS) return LJG_ERR_CAPACITY;
-  const int64_t nblocks = blocks_for(n, 256);
+  const int64_t nblocks = lc_force_blocks(g);
   const int64_t slen = scan_tmp_len(ncells);
   const ScratchLayout l = layout_for(n, ncells, ntypes, slen, nblocks);
   if (l.total > (size_t)LJG_NOALLOC_SCRATCH_BYTES) return LJG_ERR_CAPACITY;
@@ -215,8 +215,8 @@ ljg_status ljg_force_lc_noalloc(const ljg_params *params, int32_t ntypes, const 
     LJG_HIP(hipGetLastError());
     // the forces in cell order go where the wrapped caller-order positions were
     double *fs = xw;
-    lc_force_launch(st, n, xs, xs + n, xs + 2 * n, ts, cells, start, g, rc2, ntypes, tab, e24[0], s2[0], sh6[0], fs,
-                    fs + n, fs + 2 * n, pe, pv, ph, globals != nullptr, nullptr, SkipIf{nullptr, 0});
+    lc_force_launch(st, xs, xs + n, xs + 2 * n, ts, start, g, rc2, ntypes, tab, e24[0], s2[0], sh6[0], fs, fs + n,
+                    fs + 2 * n, pe, pv, ph, globals != nullptr, nullptr, SkipIf{nullptr, 0});
     hipLaunchKernelGGL(k_na_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, sorted, fs, fx, fy, fz);
     LJG_HIP(hipGetLastError());
     if (globals) {
