@@ -533,7 +533,7 @@ void verlet_fixed(Ctx &c);                 // ljg_verlet.hip
 void verlet_force(Ctx &c, bool globals);   // ljg_verlet.hip
 void verlet_geometry(Ctx &c);              // ljg_verlet.hip: fixed-point scales of the box
 void verlet_fixed_slots(Ctx &c, int64_t nslots);  // ljg_verlet.hip: posfx for slots [0, nslots)
-void cluster_jrows_force(Ctx &c, bool globals, const IntegArgs *integ = nullptr);  // ljg_force.hip
+void cluster_jrows_force(Ctx &c, bool globals, const IntegArgs *integ = nullptr);  // ljg_jrows.hip
 IntegArgs integ_args(Ctx &c, bool kick, bool drift, double dt, int32_t stamp);    // ljg_md.hip
 void md_kick_drift(Ctx &c, bool kick, bool drift, double dt, int32_t stamp, SkipIf skip = SkipIf{nullptr, 0});  // ljg_md.hip
 void wrap_positions(Ctx &c);               // ljg_md.hip
