@@ -277,10 +277,9 @@ __global__ __launch_bounds__(kLayoutBlock) void k_layout_apply(int64_t ntowers, 
 // One workgroup per tower: bitonic sort of (z, id) in LDS, then the tower's slots of the cluster layout
 // are written: src[new slot] = old slot, -1 for padding; cluster_tower for the tower's clusters.  A tower
 // holds count[t] particles, its items from start[t], its clusters [cstart[t], cstart[t] + ccount[t]).
-// Two instances: CAP = kSortSmall takes the towers up to that size (12 KB of LDS, so many workgroups
-// share a CU), CAP = kTowerSortCap the rare larger ones; each skips the towers of the other.
+// It takes the rare towers that are longer than the register sorts reach (min_n), up to kTowerSortCap.
 constexpr int kSortThreads = 256;
-constexpr int kSortSmall = 1024;
+constexpr int kSortRegisters = 1024;  // towers up to this are sorted in registers
 
 __device__ inline bool zid_less(double za, int32_t sa, double zb, int32_t sb, const int64_t *__restrict__ id) {
   if (sb < 0) return sa >= 0;  // padding sorts last
@@ -290,7 +289,6 @@ __device__ inline bool zid_less(double za, int32_t sa, double zb, int32_t sb, co
   return id[sa] < id[sb];
 }
 
-// Towers of up to min_n particles are left to k_tower_sort_wave (min_n = 0 when it does not run).
 template <int CAP>
 __global__ __launch_bounds__(kSortThreads) void k_tower_sort(
     int64_t ntowers, Segs sg, const int64_t *__restrict__ start, const int32_t *__restrict__ count,
@@ -303,9 +301,7 @@ __global__ __launch_bounds__(kSortThreads) void k_tower_sort(
   const int64_t t = seg_index(sg, blockIdx.x);
   const int64_t b = start[t];
   const int n = count[t];
-  if (n <= min_n) return;                           // sorted in registers by k_tower_sort_wave
-  if (CAP > kSortSmall && n <= kSortSmall) return;  // sorted by the small instance
-  if (CAP == kSortSmall && n > kSortSmall) return;  // left to the large instance
+  if (n <= min_n) return;  // sorted in registers
   if (n > CAP) {
     if (threadIdx.x == 0) err[0] = 1ull;
     return;
@@ -346,11 +342,10 @@ __global__ __launch_bounds__(kSortThreads) void k_tower_sort(
   for (int64_t c = c0 + threadIdx.x; c < c1; c += kSortThreads) cluster_tower[c] = (int32_t)t;
 }
 
-// Short towers (small boxes): one wavefront per tower sorts (z, id) in registers with a bitonic network
+// Towers of up to 64 particles: one wavefront per tower sorts (z, id) in registers with a bitonic network
 // over 64 E elements, element e * 64 + lane in slot e of a lane (padding sorts last), and writes the same
 // cluster layout as k_tower_sort.  Keys are distinct (ids are), so every sorter produces the one sorted
-// order.  The E = 1 instance takes towers of up to 64 particles, E = 4 those of 65 to 256, E = 8 those
-// of 257 to 512.
+// order.
 constexpr int kSortWaveThreads = 256;
 
 // The register sort carries two words per element: its z rounded to FP32 and its index k in the tower's
@@ -421,24 +416,21 @@ __device__ inline void bitonic2_sizes(float (&zv)[E], int32_t (&kv)[E], int lane
   if constexpr (SIZE < kWave * E) bitonic2_sizes<E, SIZE * 2>(zv, kv, lane, ti);
 }
 
-template <int E>
 __global__ __launch_bounds__(kSortWaveThreads) void k_tower_sort_wave(
     int64_t ntowers, Segs sg, const int64_t *__restrict__ start, const int32_t *__restrict__ count,
     const int32_t *__restrict__ items, const double *__restrict__ items_z, const int64_t *__restrict__ items_id,
     const int64_t *__restrict__ cstart, const int32_t *__restrict__ ccount, int32_t M, int32_t *__restrict__ src,
     int32_t *__restrict__ cluster_tower, unsigned long long *__restrict__ over) {
-  constexpr int P = kWave * E;
+  constexpr int E = 1, P = kWave;
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t w = (int64_t)blockIdx.x * (kSortWaveThreads / kWave) + threadIdx.x / kWave;
   if (w >= ntowers) return;
   const int64_t t = seg_index(sg, w);
   const int64_t b = start[t];
   const int n = count[t];
-  constexpr int LO = E == 1 ? 0 : E == 4 ? kWave : 4 * kWave;  // the next shorter instance's reach
-  static_assert(E == 1 || E == 4 || E == 8, "instances cover up to 64, 65-256 and 257-512 particles");
   // (over: the longest instance launched reports a tower beyond its reach, which no launched sort takes)
   if (n > P && over && lane == 0) over[0] = 1ull;
-  if (n > P || n <= LO) return;  // another instance sorts this tower
+  if (n > P) return;  // another instance sorts this tower
   float zv[E];
   int32_t kv[E];
 #pragma unroll
@@ -456,37 +448,37 @@ __global__ __launch_bounds__(kSortWaveThreads) void k_tower_sort_wave(
     const int k = e * kWave + lane;
     if (k < nslot) src[c0 * M + k] = kv[e] >= 0 ? items[b + kv[e]] : -1;
   }
-  if (P + lane < nslot) src[c0 * M + P + lane] = -1;
   for (int64_t c = c0 + lane; c < c1; c += kWave) cluster_tower[c] = (int32_t)t;
 }
 
-// Towers of 65 to 256 (E = 2) and 257 to 512 particles (E = 4): two wavefronts per tower, each sorting
-// one half of up to 64 E in registers as k_tower_sort_wave<E> does, then a merge by rank: an element's
-// place is its index in its half plus the number of the other half's elements before it (a binary
-// search in the other half, held in LDS; equal FP32 z are ordered by the exact z and id).  Twice the
-// wavefronts of a single-wave sort of the tower, each with half the network.
-constexpr int kSortPairThreads = 2 * kWave;
-
-template <int E>
-__global__ __launch_bounds__(kSortPairThreads) void k_tower_sort_pair(
+// Longer towers of up to 1024 particles: W wavefronts per tower, each sorting one W-th of up to 64 E
+// particles in registers as k_tower_sort_wave does, then a merge by rank: an element's place is its index in
+// its part plus the number of the other parts' elements before it (a binary search in each, held in LDS;
+// equal FP32 z are ordered by the exact z and id).  Two wavefronts with half the network each beat one
+// with the whole, and for 513 to 1024 particles four beat the sort in LDS with its 55 barriers: 2500 towers
+// of 800 particles 173 -> 82 us.  Instances: 65 to 256 particles (E = 2, W = 2), 257 to 512
+// (4, 2), 513 to 1024 (4, 4).
+template <int E, int W>
+__global__ __launch_bounds__(W *kWave) void k_tower_sort_parts(
     int64_t ntowers, Segs sg, const int64_t *__restrict__ start, const int32_t *__restrict__ count,
     const int32_t *__restrict__ items, const double *__restrict__ items_z, const int64_t *__restrict__ items_id,
     const int64_t *__restrict__ cstart, const int32_t *__restrict__ ccount, int32_t M, int32_t *__restrict__ src,
     int32_t *__restrict__ cluster_tower, unsigned long long *__restrict__ over) {
-  static_assert(E == 2 || E == 4, "pairs cover 65-256 and 257-512 particles");
-  constexpr int P = kWave * E;             // each half up to 64 E
-  constexpr int LO = E == 2 ? kWave : 4 * kWave;  // the next shorter instance's reach
-  __shared__ float s_z[2][P];
-  __shared__ int32_t s_k[2][P];
-  const int lane = threadIdx.x & (kWave - 1), half = (int)threadIdx.x / kWave;
+  constexpr int P = kWave * E;  // each part up to 64 E
+  constexpr int LO = W * E == 4 ? kWave : W * P / 2;  // the next shorter instance's reach
+  static_assert(W * E == 4 || W * E == 8 || W * E == 16, "instances cover 65-256, 257-512 and 513-1024 particles");
+  __shared__ float s_z[W][P];
+  __shared__ int32_t s_k[W][P];
+  const int lane = threadIdx.x & (kWave - 1), part = (int)threadIdx.x / kWave;
   if ((int64_t)blockIdx.x >= ntowers) return;  // the whole workgroup: one tower
   const int64_t t = seg_index(sg, blockIdx.x);
   const int64_t b = start[t];
   const int n = count[t];
-  if (n > 2 * P && over && threadIdx.x == 0) over[0] = 1ull;
-  if (n > 2 * P || n <= LO) return;  // another instance sorts this tower
-  const int h = (n + 1) / 2;
-  const int first = half ? h : 0, len = half ? n - h : h, olen = half ? h : n - h;
+  if (n > W * P && over && threadIdx.x == 0) over[0] = 1ull;
+  if (n > W * P || n <= LO) return;  // another instance sorts this tower
+  // parts of h particles, the last ones shorter or empty
+  const int h = (n + W - 1) / W;
+  const int first = part * h < n ? part * h : n, len = n - first < h ? n - first : h;
   float zf[E];
   int32_t kv[E];
 #pragma unroll
@@ -499,12 +491,10 @@ __global__ __launch_bounds__(kSortPairThreads) void k_tower_sort_pair(
   bitonic2_sizes<E, 2>(zf, kv, lane, ti);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    s_z[half][e * kWave + lane] = zf[e];
-    s_k[half][e * kWave + lane] = kv[e];
+    s_z[part][e * kWave + lane] = zf[e];
+    s_k[part][e * kWave + lane] = kv[e];
   }
   __syncthreads();
-  const float *oz = s_z[1 - half];
-  const int32_t *ok = s_k[1 - half];
   const int64_t c0 = cstart[t], c1 = c0 + ccount[t];
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -512,24 +502,32 @@ __global__ __launch_bounds__(kSortPairThreads) void k_tower_sort_pair(
     if (idx >= len) continue;
     const float z = zf[e];
     const int32_t k = kv[e];
-    int lo = 0, hi = olen;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      const float zo = oz[mid];
-      bool before = zo < z;
-      if (zo == z) {
-        const int32_t ko = ok[mid];
-        const double da = ti.z[ko], db = ti.z[k];
-        before = (da < db) | ((da == db) & (ti.id[ko] < ti.id[k]));
+    int place = idx;
+#pragma unroll
+    for (int o = 1; o < W; ++o) {
+      const int op = (part + o) % W;
+      const float *oz = s_z[op];
+      const int of = op * h < n ? op * h : n;
+      int lo = 0, hi = n - of < h ? n - of : h;
+      while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        const float zo = oz[mid];
+        bool before = zo < z;
+        if (zo == z) {
+          const int32_t ko = s_k[op][mid];
+          const double da = ti.z[ko], db = ti.z[k];
+          before = (da < db) | ((da == db) & (ti.id[ko] < ti.id[k]));
+        }
+        if (before) lo = mid + 1;
+        else hi = mid;
       }
-      if (before) lo = mid + 1;
-      else hi = mid;
+      place += lo;
     }
-    src[c0 * M + idx + lo] = items[b + k];
+    src[c0 * M + place] = items[b + k];
   }
   const int nslot = (int)((c1 - c0) * M);
-  for (int q = n + (int)threadIdx.x; q < nslot; q += kSortPairThreads) src[c0 * M + q] = -1;
-  for (int64_t c = c0 + threadIdx.x; c < c1; c += kSortPairThreads) cluster_tower[c] = (int32_t)t;
+  for (int q = n + (int)threadIdx.x; q < nslot; q += W * kWave) src[c0 * M + q] = -1;
+  for (int64_t c = c0 + threadIdx.x; c < c1; c += W * kWave) cluster_tower[c] = (int32_t)t;
 }
 
 // One lane per slot, the M lanes of a cluster reduce with shuffles (M divides the wavefront, and the
@@ -680,6 +678,10 @@ __global__ __launch_bounds__(kListThreads * NS, JCL ? 4 : 1) void k_cluster_list
   const double il2 = g.ilen * g.ilen;
   const double zwin = g.ilen * (1.0 + 1e-9) + 1e-9;
   const bool xy_repeats = g.nt[0] < 2 * g.R + 1 || g.nt[1] < 2 * g.R + 1;
+  // Two z images of a j-cluster can both pass the box test only if 2 ilen and the two clusters' z-extents
+  // together reach the box length: below one_image_z no earlier image needs a look (all but the longest
+  // clusters; 184 -> 151 us per pass on the 10^6-particle liquid).
+  const double one_image_z = xy_repeats ? -1. : g.L[2] - 2. * zwin - 1e-9 * g.L[2];
   const int side = 2 * g.R + 1, nvis = side * side;
   const int vbeg = (int)((int64_t)nvis * wv / NS), vend = (int)((int64_t)nvis * (wv + 1) / NS);
   const int32_t subcap = cap / NS;
@@ -780,7 +782,8 @@ __global__ __launch_bounds__(kListThreads * NS, JCL ? 4 : 1) void k_cluster_list
             if (bj[2] > zmax) break;
             if (box_dist2(bi, bj, shx, shy, shz) <= il2) {
               if constexpr (JCL) {
-                if (!passed_earlier(bi, bj, g, tx, ty, oy, ox, sz, xy_repeats, il2)) {
+                if ((bi[5] - bi[2]) + (bj[5] - bj[2]) < one_image_z ||
+                    !passed_earlier(bi, bj, g, tx, ty, oy, ox, sz, xy_repeats, il2)) {
                   if (cnt < subcap) jcl[w0 + cnt] = (int32_t)(jb + k);
                   ++cnt;
                 }
@@ -1001,18 +1004,44 @@ __global__ __launch_bounds__(kListSplitThreads) void k_cluster_lists_split(
 // frame; otherwise it uses exact per-pair differences.
 constexpr int kExpandThreads = 256;
 
-// CUB (cubic boxes): the member test runs in FP32 on the separation in fixed-point units, against ilen^2
-// in those units; tests whose FP32 d^2 lies in a band around it (cut_lo, cut_hi on the bit pattern; the
-// FP32 error of d^2 is ~5 roundings, the band 2^-18 relative) are decided again by the FP64 test above,
-// so the rows are the same.  Otherwise every test is the FP64 one.
-// STAGED: each group first copies its concatenated sub-rows into LDS (ccap int32 per group, dynamic
-// shared memory of the launch), so that entry e of the stream is one LDS read instead of a search over
-// the sub-row offsets.
-template <int M, int NS, int G, bool CUB, bool STAGED>
+// The member test runs in FP32 in the frame of the cluster's first member: members and j enter as their
+// minimum-image fixed-point offsets from it, scaled to units of ilen once per particle, so a test is three
+// subtractions, a square and a minimum over the members.  With qmax the largest member offset, the j of a
+// pair within ilen lies within qmax + ilen, and 2 qmax + ilen < L/2 leaves such a pair no wrap-around; a
+// difference of two offsets is some image of the pair, so none is taken for near that is not.  A cluster
+// that fails that, or is longer than kExpandSpan ilen, takes the FP64 test for every pair.  Of a pair near
+// ilen each offset is rounded twice, the member's below kExpandSpan ilen and j's below (kExpandSpan + 1) ilen;
+// the difference and the scale round once: d^2 is off by at most
+// 2 sqrt(3) (2 (2 kExpandSpan + 1) + 2) 2^-24 + 3 2^-24 = 38 2^-24 relative.  Tests within 2^-17 of ilen^2
+// (cut_lo, cut_hi on the bit pattern) are decided again by the FP64 test, so the rows are its rows.
+// The pass is bound by VALU instructions; it tested every member of a non-cubic box in FP64 (2.0M
+// particles, M 8: 954 us a pass) and formed the exact integer difference per pair in cubic ones (10^6
+// particles: 237 us).  Now 610 and 188 us.
+constexpr double kExpandSpan = 1.5;
+
+// Limits in fixed-point units, per dimension: j: L/2 - ilen; q: the largest member offset that the FP32 test
+// takes, below kExpandSpan ilen and (L/2 - ilen) / 2 (less 1e4 units, far above the rounding of the sums).
+struct ExpandLimits {
+  uint32_t j[3], q[3];
+};
+
+static ExpandLimits expand_limits(const FixGeom &f, double ilen) {
+  ExpandLimits l{};
+  for (int d = 0; d < 3; ++d) {
+    const double il_u = ilen * f.inv_scale[d], room = 2147483648.0 - il_u;  // (the box is longer than 2 ilen)
+    l.j[d] = room > 0. ? (uint32_t)room : 0u;
+    l.q[d] = (uint32_t)std::fmax(0., std::fmin(kExpandSpan * il_u, 0.5 * (room - 1e4)));
+  }
+  return l;
+}
+
+__device__ inline uint32_t abs_u32(int32_t a) { return a < 0 ? 0u - (uint32_t)a : (uint32_t)a; }
+
+template <int M, int NS, int G, bool STAGED>
 __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
     int64_t nclusters, const int4 *__restrict__ posfx, const double4 *__restrict__ c0, int32_t ccap,
-    const int32_t *__restrict__ ccount, const int32_t *__restrict__ jcl, FixGeom f, double ilen, uint32_t cut_lo,
-    uint32_t cut_hi, int32_t cap, int32_t *__restrict__ count, int32_t *__restrict__ jrows,
+    const int32_t *__restrict__ ccount, const int32_t *__restrict__ jcl, FixGeom f, ExpandLimits lim, double ilen,
+    uint32_t cut_lo, uint32_t cut_hi, int32_t cap, int32_t *__restrict__ count, int32_t *__restrict__ jrows,
     unsigned long long *__restrict__ stats) {
   constexpr int LG = kWave / G;  // lanes per i-cluster
   const int lane = threadIdx.x & (kWave - 1);
@@ -1026,27 +1055,32 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
   int4 xi[M];
 #pragma unroll
   for (int q = 0; q < M; ++q) xi[q] = posfx[icl * M + q];
-  // lanes whose cluster has a real member q
-  unsigned long long real_m[M];
-#pragma unroll
-  for (int q = 0; q < M; ++q) real_m[q] = __builtin_amdgcn_ballot_w64(q < nri);
-  // frame limits for the row entries: L/2 - ilen minus the largest member offset
-  int64_t jlim[3];
-  bool frame_bad = false;
+  // frame limits for the row entries: L/2 - ilen minus the largest member offset; the FP32 test's condition
+  uint32_t jlim[3];
+  bool frame_bad = false, exact = false;
+  float fxi[M], fyi[M], fzi[M];  // offsets from the first member (padding: far from every j)
+  const float scx = (float)(f.scale[0] / ilen), scy = (float)(f.scale[1] / ilen), scz = (float)(f.scale[2] / ilen);
   {
-    int64_t qmax[3] = {0, 0, 0};
+    uint32_t qmax[3] = {0, 0, 0};
 #pragma unroll
     for (int q = 0; q < M; ++q) {
+      const int32_t ox = (int32_t)((uint32_t)xi[q].x - (uint32_t)xi[0].x);
+      const int32_t oy = (int32_t)((uint32_t)xi[q].y - (uint32_t)xi[0].y);
+      const int32_t oz = (int32_t)((uint32_t)xi[q].z - (uint32_t)xi[0].z);
       if (q < nri) {
-        qmax[0] = max(qmax[0], llabs((int64_t)(int32_t)((uint32_t)xi[q].x - (uint32_t)xi[0].x)));
-        qmax[1] = max(qmax[1], llabs((int64_t)(int32_t)((uint32_t)xi[q].y - (uint32_t)xi[0].y)));
-        qmax[2] = max(qmax[2], llabs((int64_t)(int32_t)((uint32_t)xi[q].z - (uint32_t)xi[0].z)));
+        qmax[0] = max(qmax[0], abs_u32(ox));
+        qmax[1] = max(qmax[1], abs_u32(oy));
+        qmax[2] = max(qmax[2], abs_u32(oz));
       }
+      fxi[q] = q < nri ? (float)ox * scx : kPadPos32;
+      fyi[q] = q < nri ? (float)oy * scy : kPadPos32;
+      fzi[q] = q < nri ? (float)oz * scz : kPadPos32;
     }
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
-      jlim[d] = (int64_t)(2147483648.0 - ilen * f.inv_scale[d]) - qmax[d];
-      frame_bad = frame_bad || (live && jlim[d] < 0);
+      frame_bad = frame_bad || (live && qmax[d] > lim.j[d]);
+      jlim[d] = qmax[d] > lim.j[d] ? 0u : lim.j[d] - qmax[d];
+      exact = exact || qmax[d] > lim.q[d];
     }
   }
   // the NS sub-rows of the first pass, in order (an overflowed sub-row is rebuilt anyway)
@@ -1074,9 +1108,15 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
   if constexpr (STAGED) {
     // the group's row in LDS (also for a dead group, whose icl is a real cluster: its lanes' clamped
     // prefetches below read real entries); a wavefront reads only its own groups' rows
+    // (the sub-rows' first entries are loaded together: most hold no more than LG)
+    int32_t first[NS];
 #pragma unroll
-    for (int w = 0; w < NS; ++w)
-      for (int k = l; k < pre[w + 1] - pre[w]; k += LG) srow[pre[w] + k] = crow[w * subcap + k];
+    for (int w = 0; w < NS; ++w) first[w] = l < pre[w + 1] - pre[w] ? crow[w * subcap + l] : 0;
+#pragma unroll
+    for (int w = 0; w < NS; ++w) {
+      if (l < pre[w + 1] - pre[w]) srow[pre[w] + l] = first[w];
+      for (int k = l + LG; k < pre[w + 1] - pre[w]; k += LG) srow[pre[w] + k] = crow[w * subcap + k];
+    }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1118,45 +1158,30 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
     }
     bool near = false;
     // the FP64 member test
-    auto near64 = [&](int q, const int4 &pj) {
-      const double dx = (double)(int32_t)((uint32_t)xi[q].x - (uint32_t)pj.x) * f.scale[0];
-      const double dy = (double)(int32_t)((uint32_t)xi[q].y - (uint32_t)pj.y) * f.scale[1];
-      const double dz = (double)(int32_t)((uint32_t)xi[q].z - (uint32_t)pj.z) * f.scale[2];
+    auto near64 = [&](const int4 &pi, const int4 &pj) {
+      const double dx = (double)(int32_t)((uint32_t)pi.x - (uint32_t)pj.x) * f.scale[0];
+      const double dy = (double)(int32_t)((uint32_t)pi.y - (uint32_t)pj.y) * f.scale[1];
+      const double dz = (double)(int32_t)((uint32_t)pi.z - (uint32_t)pj.z) * f.scale[2];
       return dx * dx + dy * dy + dz * dz <= il2;
     };
     if (inrow && xj.w >= 0) {  // padding slots carry type -1
-      if constexpr (CUB) {
-        // per member, the lanes inside and the lanes in the band, as wave masks (scalar unit)
-        unsigned long long in_m = 0ull, band_m = 0ull;
+      const int32_t ox = (int32_t)((uint32_t)xj.x - (uint32_t)xi[0].x);
+      const int32_t oy = (int32_t)((uint32_t)xj.y - (uint32_t)xi[0].y);
+      const int32_t oz = (int32_t)((uint32_t)xj.z - (uint32_t)xi[0].z);
+      const float jx = (float)ox * scx, jy = (float)oy * scy, jz = (float)oz * scz;
+      float dmin = __builtin_inff();
 #pragma unroll
-        for (int q = 0; q < M; ++q) {
-          const float dx = (float)(int32_t)((uint32_t)xi[q].x - (uint32_t)xj.x);
-          const float dy = (float)(int32_t)((uint32_t)xi[q].y - (uint32_t)xj.y);
-          const float dz = (float)(int32_t)((uint32_t)xi[q].z - (uint32_t)xj.z);
-          const uint32_t ub = __float_as_uint(__builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)));
-          const unsigned long long lo = __builtin_amdgcn_ballot_w64(ub < cut_lo) & real_m[q];
-          in_m |= lo;
-          band_m |= __builtin_amdgcn_ballot_w64(ub < cut_hi) & real_m[q] & ~lo;
-        }
-        near = (in_m >> lane) & 1ull;
-        if (band_m != 0ull) {
-          // rare; j passes through an empty asm so that the integer separations above are not kept
-          int4 pj = xj;
-          asm volatile("" : "+v"(pj.x), "+v"(pj.y), "+v"(pj.z));
-          if ((band_m >> lane) & 1ull) {
-#pragma unroll
-            for (int q = 0; q < M; ++q) near = near || (q < nri && near64(q, pj));
-          }
-        }
-      } else {
-#pragma unroll
-        for (int q = 0; q < M; ++q) near = near || (q < nri && near64(q, xj));
+      for (int q = 0; q < M; ++q) {
+        const float dx = fxi[q] - jx, dy = fyi[q] - jy, dz = fzi[q] - jz;
+        dmin = fminf(dmin, __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)));
       }
-      if (near) {
-        frame_bad = frame_bad || llabs((int64_t)(int32_t)((uint32_t)xj.x - (uint32_t)xi[0].x)) > jlim[0] ||
-                    llabs((int64_t)(int32_t)((uint32_t)xj.y - (uint32_t)xi[0].y)) > jlim[1] ||
-                    llabs((int64_t)(int32_t)((uint32_t)xj.z - (uint32_t)xi[0].z)) > jlim[2];
+      near = __float_as_uint(dmin) < cut_lo;
+      if (exact || (!near && __float_as_uint(dmin) < cut_hi)) {
+        // rare: the FP64 test of every member, from positions read again (no integer one is kept for this)
+        near = false;
+        for (int q = 0; q < nri; ++q) near = near || near64(posfx[icl * M + q], xj);
       }
+      if (near) frame_bad = frame_bad || abs_u32(ox) > jlim[0] || abs_u32(oy) > jlim[1] || abs_u32(oz) > jlim[2];
     }
     const unsigned long long ball = __ballot(near) & gmask;
     const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(ball >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ball, 0u));
@@ -1408,10 +1433,8 @@ void fill_i32(Ctx &c, int32_t *p, int64_t n, int32_t v) {
 }
 
 // Average clusters per tower below which the cluster-entry lists use a lane (or a group of lanes) per
-// i-cluster, and average particles per tower up to which the towers of at most 512 particles are sorted in
-// registers.
+// i-cluster.
 constexpr int kLaneListsBelow = 24;
-constexpr int kWaveSortBelow = 448;
 // i-clusters below which those rows are made by a group of lanes per i-cluster: such a build (a few boxes
 // of an ensemble, a small box) is bound by the latency of its dependent loads, ~850 per lane in the lane
 // kernel, ~60 per lane in the group form; above it, by a lane each (the group form scans every visit
@@ -1542,7 +1565,7 @@ void vcl_build(Ctx &c) {
   // permutation then skips, and the build runs again with the readback.
   unsigned long long ts[4] = {0, 0, 0, 0};
   if (guess) {
-    ts[1] = (unsigned long long)(c.seg_max_count < 8 * kWave ? c.seg_max_count : 8 * kWave);
+    ts[1] = (unsigned long long)(c.seg_max_count < kSortRegisters ? c.seg_max_count : kSortRegisters);
   } else {
     stream_spin(c, tmark, 4, ts);
   }
@@ -1554,49 +1577,37 @@ void vcl_build(Ctx &c) {
   c.perm.ensure(new_slots);
   c.cluster_tower.ensure(ncl);
   if (ens) ensemble_region_prep(c, active);  // the regions' tails stay padding
-  // towers of up to 512 particles sort in registers, a wavefront each (three instances by length, each
-  // launched only if some tower is in its range); longer ones in LDS
-  const bool wave_sort = ens || (int64_t)ts[0] <= (int64_t)kWaveSortBelow * ntow;
-  const int32_t min_n = wave_sort ? 8 * kWave : 0;
-  if (wave_sort) {
-    constexpr int per_block = kSortWaveThreads / kWave;
-#define LJG_WAVE_SORT(E, OVER)                                                                                  \
-  if (n_towers > 0) {                                                                                           \
-    hipLaunchKernelGGL(k_tower_sort_wave<E>, dim3(blocks_for(n_towers, per_block)), dim3(kSortWaveThreads), 0,  \
-                       c.stream, n_towers, sg_towers, c.tower_start.p, c.tower_count.p, c.tower_items.p,        \
-                       c.tower_z.p, c.tower_id.p, c.ctow_start.p, c.ctow_count.p, M, c.perm.p, c.cluster_tower.p, \
-                       OVER);                                                                                   \
+  // Towers of up to 1024 particles sort in registers (an instance by length, launched only if some tower is
+  // in its range), longer ones in LDS.  Every tower is sorted by exactly one instance; the longest tower
+  // (ts[1]) and the shortest non-empty one (ts[3], 0 when not known) bound which ones can have work.
+  if (n_towers > 0) {
+#define LJG_SORT(KERNEL, BLOCKS, THREADS, OVER)                                                                  \
+  {                                                                                                             \
+    hipLaunchKernelGGL(KERNEL, dim3(BLOCKS), dim3(THREADS), 0, c.stream, n_towers, sg_towers, c.tower_start.p,  \
+                       c.tower_count.p, c.tower_items.p, c.tower_z.p, c.tower_id.p, c.ctow_start.p,             \
+                       c.ctow_count.p, M, c.perm.p, c.cluster_tower.p, OVER);                                   \
     LJG_HIP(hipGetLastError());                                                                                 \
   }
-    // every tower is sorted by exactly one instance; the longest tower (ts[1]) and the shortest non-empty
-    // one (ts[3], 0 when not known) bound which ones can have work
     unsigned long long *over = guess ? c.list_stats.p + 5 : nullptr;
-    const int top = ts[1] > (unsigned long long)(4 * kWave) ? 8 : ts[1] > (unsigned long long)kWave ? 4 : 1;
-    const unsigned long long shortest = ens ? 0ull : ts[3];
-#define LJG_PAIR_SORT(E, OVER)                                                                                  \
-  if (n_towers > 0) {                                                                                           \
-    hipLaunchKernelGGL(k_tower_sort_pair<E>, dim3((unsigned)n_towers), dim3(kSortPairThreads), 0, c.stream,    \
-                       n_towers, sg_towers, c.tower_start.p, c.tower_count.p, c.tower_items.p, c.tower_z.p,     \
-                       c.tower_id.p, c.ctow_start.p, c.ctow_count.p, M, c.perm.p, c.cluster_tower.p, OVER);     \
-    LJG_HIP(hipGetLastError());                                                                                 \
-  }
-    if (shortest <= (unsigned long long)kWave) LJG_WAVE_SORT(1, top == 1 ? over : nullptr)
-    if (top >= 4 && shortest <= (unsigned long long)(4 * kWave)) LJG_PAIR_SORT(2, top == 4 ? over : nullptr)
-    if (top == 8) LJG_PAIR_SORT(4, over)
-#undef LJG_PAIR_SORT
-#undef LJG_WAVE_SORT
-  }
-  if (ts[1] > (unsigned long long)min_n && n_towers > 0) {
-    hipLaunchKernelGGL(k_tower_sort<kSortSmall>, dim3((unsigned)n_towers), dim3(kSortThreads), 0, c.stream, n_towers,
-                       sg_towers, c.tower_start.p, c.tower_count.p, c.tower_items.p, s.z.p, s.id.p, c.ctow_start.p,
-                       c.ctow_count.p, M, c.perm.p, c.cluster_tower.p, c.list_stats.p + 5, min_n);
-    LJG_HIP(hipGetLastError());
-  }
-  if (ts[1] > (unsigned long long)kSortSmall && n_towers > 0) {
-    hipLaunchKernelGGL(k_tower_sort<kTowerSortCap>, dim3((unsigned)n_towers), dim3(kSortThreads), 0, c.stream,
-                       n_towers, sg_towers, c.tower_start.p, c.tower_count.p, c.tower_items.p, s.z.p, s.id.p,
-                       c.ctow_start.p, c.ctow_count.p, M, c.perm.p, c.cluster_tower.p, c.list_stats.p + 5, min_n);
-    LJG_HIP(hipGetLastError());
+    const unsigned long long longest = ts[1], shortest = ens ? 0ull : ts[3];
+    constexpr unsigned long long r1 = kWave, r2 = 4 * kWave, r3 = 8 * kWave, r4 = kSortRegisters;
+    if (shortest <= r1)
+      LJG_SORT(k_tower_sort_wave, blocks_for(n_towers, kSortWaveThreads / kWave), kSortWaveThreads,
+               longest <= r1 ? over : nullptr)
+    if (longest > r1 && shortest <= r2)
+      LJG_SORT((k_tower_sort_parts<2, 2>), (unsigned)n_towers, 2 * kWave, longest <= r2 ? over : nullptr)
+    if (longest > r2 && shortest <= r3)
+      LJG_SORT((k_tower_sort_parts<4, 2>), (unsigned)n_towers, 2 * kWave, longest <= r3 ? over : nullptr)
+    if (longest > r3 && shortest <= r4)
+      LJG_SORT((k_tower_sort_parts<4, 4>), (unsigned)n_towers, 4 * kWave, over)
+#undef LJG_SORT
+    if (longest > r4) {
+      hipLaunchKernelGGL(k_tower_sort<kTowerSortCap>, dim3((unsigned)n_towers), dim3(kSortThreads), 0, c.stream,
+                         n_towers, sg_towers, c.tower_start.p, c.tower_count.p, c.tower_items.p, s.z.p, s.id.p,
+                         c.ctow_start.p, c.ctow_count.p, M, c.perm.p, c.cluster_tower.p, c.list_stats.p + 5,
+                         (int32_t)r4);
+      LJG_HIP(hipGetLastError());
+    }
   }
   const bool jrows = c.want_jrows;
   if (jrows && ens) throw HipError{hipErrorInvalidValue, "j-particle rows on an ensemble of boxes", -2};
@@ -1693,29 +1704,27 @@ void vcl_build(Ctx &c) {
       // (one i-cluster per wave below 2048 clusters: latency-bound small builds)
       const int eg = c.prm.build_groups > 0 ? c.prm.build_groups
                                              : (M >= 4 ? (ncl <= 2048 ? 1 : 4) : M == 2 ? 4 : 8);
-      // FP32 member test of the cubic variant: ilen^2 in fixed-point units, band 2^-18 relative
+      // FP32 member test (lengths in units of ilen): a band of 128 ulps, 2^-17 below 1 and 2^-16 above
       uint32_t cut_lo = 0, cut_hi = 0;
-      cutoff_band((float)(ilen * ilen * c.fg.inv_scale[0] * c.fg.inv_scale[0]), std::ldexp(1.0, -18), cut_lo, cut_hi);
+      cutoff_band(1.f, std::ldexp(1.0, -16), cut_lo, cut_hi);
+      const ExpandLimits lim = expand_limits(c.fg, ilen);
 // the staged form when the block's rows fit in 64 KiB of LDS (4 G rows of cap int32)
-#define LJG_EXPAND_LAUNCH(MV, GV, CUBV)                                                                           \
+#define LJG_EXPAND_LAUNCH(MV, GV)                                                                                 \
   {                                                                                                               \
     const size_t lds = (size_t)(kExpandThreads / (kWave / GV)) * (size_t)cap * sizeof(int32_t);                   \
     if (lds <= 65536)                                                                                             \
-      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, CUBV, true>), dim3(nb), dim3(kExpandThreads),         \
+      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, true>), dim3(nb), dim3(kExpandThreads),         \
                          (unsigned)lds, c.stream, ncl, c.posfx.p, c.c0.p, cap, c.list_count.p, c.jcl.p, c.fg,     \
-                         ilen, cut_lo, cut_hi, jcap, c.jcount.p, c.jlist.p, c.list_stats.p);                      \
+                         lim, ilen, cut_lo, cut_hi, jcap, c.jcount.p, c.jlist.p, c.list_stats.p);                      \
     else                                                                                                          \
-      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, CUBV, false>), dim3(nb), dim3(kExpandThreads), 0,     \
-                         c.stream, ncl, c.posfx.p, c.c0.p, cap, c.list_count.p, c.jcl.p, c.fg, ilen, cut_lo,      \
+      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, false>), dim3(nb), dim3(kExpandThreads), 0,     \
+                         c.stream, ncl, c.posfx.p, c.c0.p, cap, c.list_count.p, c.jcl.p, c.fg, lim, ilen, cut_lo,      \
                          cut_hi, jcap, c.jcount.p, c.jlist.p, c.list_stats.p);                                    \
   }
 #define LJG_EXPAND(MV, GV)                                                                                        \
   if (M == MV && eg == GV) {                                                                                      \
     const int nb = blocks_for(ncl, (kExpandThreads / kWave) * GV);                                               \
-    if (c.fg.cubic)                                                                                               \
-      LJG_EXPAND_LAUNCH(MV, GV, true)                                                                             \
-    else                                                                                                          \
-      LJG_EXPAND_LAUNCH(MV, GV, false)                                                                            \
+    LJG_EXPAND_LAUNCH(MV, GV)                                                                                     \
     goto expanded;                                                                                                \
   }
       LJG_EXPAND(1, 4) LJG_EXPAND(1, 8) LJG_EXPAND(2, 2) LJG_EXPAND(2, 4) LJG_EXPAND(4, 1) LJG_EXPAND(4, 2)
