@@ -503,7 +503,6 @@ void vcl_build(Ctx &c);                    // ljg_vcl.hip
 // that launch exited without effect and the caller builds again and launches again.  ljg_vcl.hip
 bool vcl_finish_lists(Ctx &c);
 void fill_i32(Ctx &c, int32_t *p, int64_t n, int32_t v);  // ljg_vcl.hip: p[0..n) = v on the stream
-void vcl_pos32(Ctx &c, const int32_t *active = nullptr);  // ljg_vcl.hip (active: ensemble boxes to write)
 // A launch of the FP32 cluster kernel over some i-clusters only (the segments' nitems clusters), with
 // its block partials from part_offset (reserved by the caller).
 // Work queue of a persistent force launch: the tiles (G i-clusters of one wavefront) are taken in chunks
@@ -537,8 +536,8 @@ void cluster_jrows_force(Ctx &c, bool globals, const IntegArgs *integ = nullptr)
 IntegArgs integ_args(Ctx &c, bool kick, bool drift, double dt, int32_t stamp);    // ljg_md.hip
 void md_kick_drift(Ctx &c, bool kick, bool drift, double dt, int32_t stamp, SkipIf skip = SkipIf{nullptr, 0});  // ljg_md.hip
 void wrap_positions(Ctx &c);               // ljg_md.hip
-// Rebuild permutation (also sets the rebuild reference positions; writes posfx when given).
-void permute_state(Ctx &c, const int32_t *src, int64_t new_slots, int4 *posfx = nullptr);  // ljg_md.hip
+// Rebuild permutation of the cell layout (also sets the rebuild reference positions).
+void permute_state(Ctx &c, const int32_t *src, int64_t new_slots);  // ljg_md.hip
 void reduce_partials(Ctx &c, int64_t nitems, ljg_globals *out, bool globals);  // ljg_md.hip
 // Positions (3n: x, y, z in upload order) into the current layout, velocities too when vel != nullptr,
 // the derived FP32 / fixed-point positions refreshed; flag[2] = 1 if a particle moved skin/2 since the
@@ -560,8 +559,11 @@ void stream_wait(Ctx &c, const unsigned long long *src = nullptr, int n = 0, uns
 // queued in between.
 unsigned long long stream_mark(Ctx &c, const unsigned long long *src, int n);
 void stream_spin(Ctx &c, unsigned long long seq, int n, unsigned long long *out);
-// stats[0] += sum(cnt[0..n)), stats[1] = max(stats[1], max(cnt)); a few hundred atomics at most.
-void count_stats(Ctx &c, const int32_t *cnt, int64_t n, unsigned long long *stats);  // ljg_md.hip
+// Sum and maximum of cnt[0..n) into stats[0], [1] (zero before), and of cnt2[0..n2) into stats2.  ljg_md.hip
+void count_stats(Ctx &c, const int32_t *cnt, int64_t n, unsigned long long *stats, const int32_t *cnt2 = nullptr,
+                 int64_t n2 = 0, unsigned long long *stats2 = nullptr);
+// The same of one array, and a stream marker with the first `words` of stats (stream_spin waits for it).
+unsigned long long count_stats_mark(Ctx &c, const int32_t *cnt, int64_t n, unsigned long long *stats, int words);
 // Ensemble (ljg_ensemble.hip): per-box tower grids and fixed regions for cluster size c.M, the tower
 // histogram that wraps each position into its own box, the per-box tower layout inside the regions, the
 // wrap alone, and the per-box reduction of cl_glob into box_glob.  `active` (device, per box; null: every
@@ -587,9 +589,9 @@ void ensemble_edit_regions(Ctx &c, const std::vector<int32_t> &src_box, const st
                            int64_t kept, int64_t added, const double *x, const double *y, const double *z,
                            const double *vx, const double *vy, const double *vz, const int32_t *type,
                            const int64_t *id);
-// The slots of the active boxes' regions gathered from src (old slots of the same regions) in place,
-// through the other state buffer; the other boxes' slots are not touched.  Nothing moves when *skip is
-// set on the device (skip may be null).  ljg_md.hip
+// The slots of the active boxes' regions gathered from src (old slots of the same regions) into the other
+// state buffer; the other boxes' slots are not touched.  Nothing is written when *skip is set on the device
+// (skip may be null).  ljg_md.hip
 void permute_active(Ctx &c, const int32_t *src, const int32_t *active, const unsigned long long *skip = nullptr);
 // The member rows of the FP32 cluster kernel after a cluster-entry build (all clusters, or with `partial`
 // the marked boxes' of an ensemble).

@@ -93,11 +93,10 @@ void exclusive_scan_i32_to_i64(Ctx &c, const int32_t *in, int64_t *out, int64_t 
 
 // ---------------------------------------------------------------------------------------------------
 // State permutation: new slot s takes the particle of old slot src[s]; src[s] < 0 makes a padding slot.
-// Every permutation is a rebuild, so the rebuild reference positions are set to the positions here, and
-// when posfx is given the slots' 32-bit fixed-point positions are written too (type -1 for padding).
+// Every permutation is a rebuild, so the rebuild reference positions are set to the positions here.
 // Inside the step loop the force is recomputed right after a rebuild, so it is not carried.
 __global__ void k_permute(int64_t nnew, const int32_t *__restrict__ src, StateView o, StateView n,
-                          int32_t carry_force, int4 *__restrict__ posfx, FixGeom f) {
+                          int32_t carry_force) {
   const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (s >= nnew) return;
   const int32_t k = src[s];
@@ -110,10 +109,6 @@ __global__ void k_permute(int64_t nnew, const int32_t *__restrict__ src, StateVi
     if (carry_force) { n.fx[s] = o.fx[k]; n.fy[s] = o.fy[k]; n.fz[s] = o.fz[k]; }
     n.ofx[s] = o.ofx[k]; n.ofy[s] = o.ofy[k]; n.ofz[s] = o.ofz[k];
     n.type[s] = t; n.orig[s] = o.orig[k]; n.id[s] = o.id[k];
-    if (posfx)
-      posfx[s] = make_int4((int32_t)(uint32_t)(uint64_t)__double2ll_rn((x - f.min[0]) * f.inv_scale[0]),
-                           (int32_t)(uint32_t)(uint64_t)__double2ll_rn((y - f.min[1]) * f.inv_scale[1]),
-                           (int32_t)(uint32_t)(uint64_t)__double2ll_rn((z - f.min[2]) * f.inv_scale[2]), t);
   } else {
     n.x[s] = kDummyPos; n.y[s] = kDummyPos; n.z[s] = kDummyPos;
     n.vx[s] = 0.; n.vy[s] = 0.; n.vz[s] = 0.;
@@ -121,12 +116,11 @@ __global__ void k_permute(int64_t nnew, const int32_t *__restrict__ src, StateVi
     n.ofx[s] = 0.; n.ofy[s] = 0.; n.ofz[s] = 0.;
     n.rx[s] = kDummyPos; n.ry[s] = kDummyPos; n.rz[s] = kDummyPos;
     n.type[s] = 0; n.orig[s] = -1; n.id[s] = -1;
-    if (posfx) posfx[s] = make_int4(0, 0, 0, -1);
   }
 }
 
 // The same gather over the slots of the marked ensemble boxes only, into the other buffer at the same
-// slots, then copied back: each box's particles stay in the box's region, so the gather reads no slot
+// slots (the cluster build copies them back): each box's particles stay in the box's region, so the gather reads no slot
 // another thread writes, and the unmarked boxes' slots are never touched.
 __global__ void k_permute_boxes(int64_t nitems, Segs sg, int32_t M, const int32_t *__restrict__ src,
                                 const int32_t *__restrict__ cluster_box, const int32_t *__restrict__ box_active,
@@ -156,21 +150,6 @@ __global__ void k_permute_boxes(int64_t nitems, Segs sg, int32_t M, const int32_
   }
 }
 
-__global__ void k_copy_boxes(int64_t nitems, Segs sg, int32_t M, const int32_t *__restrict__ cluster_box,
-                             const int32_t *__restrict__ box_active, StateView from, StateView to,
-                             const unsigned long long *__restrict__ skip) {
-  const int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (it >= nitems || (skip && *skip)) return;
-  const int64_t s = seg_index(sg, it);
-  if (box_active[cluster_box[s / M]] == 0) return;
-  to.x[s] = from.x[s];   to.y[s] = from.y[s];   to.z[s] = from.z[s];
-  to.vx[s] = from.vx[s]; to.vy[s] = from.vy[s]; to.vz[s] = from.vz[s];
-  to.fx[s] = from.fx[s]; to.fy[s] = from.fy[s]; to.fz[s] = from.fz[s];
-  to.ofx[s] = from.ofx[s]; to.ofy[s] = from.ofy[s]; to.ofz[s] = from.ofz[s];
-  to.rx[s] = from.rx[s]; to.ry[s] = from.ry[s]; to.rz[s] = from.rz[s];
-  to.type[s] = from.type[s]; to.orig[s] = from.orig[s]; to.id[s] = from.id[s];
-}
-
 void permute_active(Ctx &c, const int32_t *src, const int32_t *active, const unsigned long long *skip) {
   const int other = 1 - c.cur;
   c.st[other].ensure((size_t)c.nslots);
@@ -179,16 +158,13 @@ void permute_active(Ctx &c, const int32_t *src, const int32_t *active, const uns
   hipLaunchKernelGGL(k_permute_boxes, dim3(blocks_for(ni, 256)), dim3(256), 0, c.stream, ni, c.seg_slots, c.M, src,
                      c.cluster_box.p, active, view(c.st[c.cur]), view(c.st[other]), (int32_t)c.carry_force, skip);
   LJG_HIP(hipGetLastError());
-  hipLaunchKernelGGL(k_copy_boxes, dim3(blocks_for(ni, 256)), dim3(256), 0, c.stream, ni, c.seg_slots, c.M,
-                     c.cluster_box.p, active, view(c.st[other]), view(c.st[c.cur]), skip);
-  LJG_HIP(hipGetLastError());
 }
 
-void permute_state(Ctx &c, const int32_t *src, int64_t new_slots, int4 *posfx) {
+void permute_state(Ctx &c, const int32_t *src, int64_t new_slots) {
   const int other = 1 - c.cur;
   c.st[other].ensure((size_t)new_slots);
   hipLaunchKernelGGL(k_permute, dim3(blocks_for(new_slots, 256)), dim3(256), 0, c.stream, new_slots, src,
-                     view(c.st[c.cur]), view(c.st[other]), (int32_t)c.carry_force, posfx, c.fg);
+                     view(c.st[c.cur]), view(c.st[other]), (int32_t)c.carry_force);
   LJG_HIP(hipGetLastError());
   c.cur = other;
   c.nslots = new_slots;
@@ -439,14 +415,23 @@ __global__ __launch_bounds__(1024) void k_reduce(int64_t n, const double *__rest
 
 constexpr int kStatThreads = 256;
 
+// Sum and maximum of the n counts into stats[0], [1], and of the n2 counts of a second array into stats2: the
+// first nb workgroups take the first array, the others the second.
 __global__ __launch_bounds__(kStatThreads) void k_count_stats(int64_t n, const int32_t *__restrict__ cnt,
-                                                              unsigned long long *__restrict__ stats) {
+                                                              unsigned long long *__restrict__ stats, int32_t nb,
+                                                              int64_t n2, const int32_t *__restrict__ cnt2,
+                                                              unsigned long long *__restrict__ stats2) {
   __shared__ unsigned long long ss[kStatThreads];
   __shared__ int32_t sm[kStatThreads];
+  const bool second = (int32_t)blockIdx.x >= nb;
+  const int64_t m = second ? n2 : n;
+  const int32_t *p = second ? cnt2 : cnt;
+  const int32_t bid = second ? (int32_t)blockIdx.x - nb : (int32_t)blockIdx.x;
+  const int32_t nblk = second ? (int32_t)gridDim.x - nb : nb;
   unsigned long long sum = 0;
   int32_t mx = 0;
-  for (int64_t i = (int64_t)blockIdx.x * kStatThreads + threadIdx.x; i < n; i += (int64_t)gridDim.x * kStatThreads) {
-    const int32_t v = cnt[i];
+  for (int64_t i = (int64_t)bid * kStatThreads + threadIdx.x; i < m; i += (int64_t)nblk * kStatThreads) {
+    const int32_t v = p[i];
     sum += (unsigned long long)v;
     mx = v > mx ? v : mx;
   }
@@ -461,9 +446,55 @@ __global__ __launch_bounds__(kStatThreads) void k_count_stats(int64_t n, const i
     __syncthreads();
   }
   if (threadIdx.x == 0) {
-    atomicAdd(&stats[0], ss[0]);
-    atomicMax(&stats[1], (unsigned long long)sm[0]);
+    unsigned long long *out = second ? stats2 : stats;
+    atomicAdd(&out[0], ss[0]);
+    atomicMax(&out[1], (unsigned long long)sm[0]);
   }
+}
+
+// The same for few counts, in one workgroup that also copies the statistics behind the marker word and writes
+// the marker: a launch less for small builds.
+constexpr int kStatMarkThreads = 1024;
+constexpr int64_t kStatMarkMax = 16384;  // 16 counts per thread: about the cost of the launch saved
+
+__global__ __launch_bounds__(kStatMarkThreads) void k_count_stats_mark(int32_t n, const int32_t *__restrict__ cnt,
+                                                                       unsigned long long *__restrict__ stats,
+                                                                       int32_t words,
+                                                                       unsigned long long *__restrict__ dst,
+                                                                       unsigned long long seq) {
+  constexpr int W = kStatMarkThreads / kWave;
+  __shared__ unsigned long long ss[W];
+  __shared__ int32_t sm[W];
+  unsigned long long sum = 0;
+  int32_t mx = 0;
+  for (int32_t i = threadIdx.x; i < n; i += kStatMarkThreads) {
+    const int32_t v = cnt[i];
+    sum += (unsigned long long)v;
+    mx = v > mx ? v : mx;
+  }
+  for (int off = kWave / 2; off > 0; off >>= 1) {
+    sum += __shfl_xor(sum, off, kWave);
+    const int32_t o = __shfl_xor(mx, off, kWave);
+    mx = o > mx ? o : mx;
+  }
+  if ((threadIdx.x & (kWave - 1)) == 0) {
+    ss[threadIdx.x / kWave] = sum;
+    sm[threadIdx.x / kWave] = mx;
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  sum = 0;
+  for (int k = 0; k < W; ++k) {
+    sum += ss[k];
+    mx = sm[k] > mx ? sm[k] : mx;
+  }
+  stats[0] = sum;
+  stats[1] = (unsigned long long)mx;
+  dst[1] = sum;
+  dst[2] = (unsigned long long)mx;
+  for (int k = 2; k < words; ++k) dst[1 + k] = stats[k];
+  __threadfence_system();
+  dst[0] = seq;
 }
 
 // Copies n words of src, then n2 words of src2, behind the marker word, and writes the marker last.
@@ -515,12 +546,29 @@ void stream_wait(Ctx &c, const unsigned long long *src, int n, unsigned long lon
   stream_spin(c, seq, n + n2, out);
 }
 
-void count_stats(Ctx &c, const int32_t *cnt, int64_t n, unsigned long long *stats) {
-  if (n <= 0) return;
-  int nb = blocks_for(n, kStatThreads * 16);
-  nb = nb < 256 ? nb : 256;
-  hipLaunchKernelGGL(k_count_stats, dim3(nb), dim3(kStatThreads), 0, c.stream, n, cnt, stats);
+void count_stats(Ctx &c, const int32_t *cnt, int64_t n, unsigned long long *stats, const int32_t *cnt2, int64_t n2,
+                 unsigned long long *stats2) {
+  auto blocks = [](int64_t m) {
+    const int nb = blocks_for(m, kStatThreads * 16);
+    return nb < 256 ? nb : 256;
+  };
+  const int nb = blocks(n), nb2 = blocks(n2);
+  if (nb + nb2 == 0) return;
+  hipLaunchKernelGGL(k_count_stats, dim3(nb + nb2), dim3(kStatThreads), 0, c.stream, n, cnt, stats, (int32_t)nb, n2,
+                     cnt2, stats2);
   LJG_HIP(hipGetLastError());
+}
+
+unsigned long long count_stats_mark(Ctx &c, const int32_t *cnt, int64_t n, unsigned long long *stats, int words) {
+  if (n > kStatMarkMax) {
+    count_stats(c, cnt, n, stats);
+    return stream_mark(c, stats, words);
+  }
+  const unsigned long long seq = ++c.mark_seq;
+  hipLaunchKernelGGL(k_count_stats_mark, dim3(1), dim3(kStatMarkThreads), 0, c.stream, (int32_t)n, cnt, stats,
+                     (int32_t)words, c.pin_mark_dev, seq);
+  LJG_HIP(hipGetLastError());
+  return seq;
 }
 
 void reduce_launch(hipStream_t st, int64_t nitems, const double *pe, const double *pv, const int64_t *ph,

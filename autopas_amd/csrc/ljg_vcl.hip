@@ -530,30 +530,31 @@ __global__ __launch_bounds__(W *kWave) void k_tower_sort_parts(
   for (int64_t c = c0 + threadIdx.x; c < c1; c += W * kWave) cluster_tower[c] = (int32_t)t;
 }
 
-// One lane per slot, the M lanes of a cluster reduce with shuffles (M divides the wavefront, and the
-// cluster's slots are consecutive, so a cluster never straddles two wavefronts).  The members are sorted
-// by z, so the first and last real members' z are the minimum and maximum.
-// In an ensemble (cluster_box given) only the clusters of the boxes box_active marks (every box when it
-// is null) are written, and an empty cluster of a region's tail gets an empty row (lcount = 0).
-__global__ void k_cluster_bbox(int64_t nitems, Segs sg, int32_t M, const double *__restrict__ x,
-                               const double *__restrict__ y, const double *__restrict__ z,
-                               const int32_t *__restrict__ orig, double *__restrict__ bbox,
-                               double4 *__restrict__ c0, const int32_t *__restrict__ cluster_box,
-                               const int32_t *__restrict__ box_active, int32_t *__restrict__ lcount) {
-  // segments are whole clusters, so the M lanes of a cluster stay together in a wavefront
-  const int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const int64_t s = it < nitems ? seg_index(sg, it) : -1;
-  // a cluster's M slots are in one box: the test is uniform over the lanes that exchange values below
-  const bool mine = s >= 0 && (box_active == nullptr || box_active[cluster_box[s / M]] != 0);
-  const bool real = mine && orig[s] >= 0;
+// What a cluster layout derives from a slot's position: the cluster's bounding box and reference point
+// (the M lanes of a cluster are consecutive in a wavefront and reduce with shuffles) and, for the
+// cluster-entry kernels (pos32 given), the FP32 position relative to that reference point, particle type bits
+// in w, and the FP64 position.  Padding slots sit at the sentinel +3e30 in every coordinate: any distance to
+// them squares to +inf in FP32, which fails the cutoff test, while the difference itself stays finite (so
+// masked terms contribute exact zeros).  Both position buffers are written: the fused integrator of the FP32
+// cluster kernel writes the real slots of the second one each step, and the padding slots must hold the
+// sentinel in both.  Returns the largest |component| of the FP32 position (0 for padding).  In an ensemble
+// (lcount given) an empty cluster of a region's tail gets an empty row.  Every lane of the wavefront calls
+// this; mine: the lane holds a slot to write (uniform over a cluster).
+struct ClusterOut {
+  double *bbox;
+  double4 *c0;
+  int32_t *lcount;
+  float4 *pos32, *pos32_next;
+  double4 *posd, *posd_next;
+  unsigned long long *ext;
+};
+
+__device__ inline float cluster_derive(int64_t s, int32_t M, bool mine, bool real, double px, double py, double pz,
+                                       int32_t type, const ClusterOut &o) {
   const double inf = __builtin_inf();
-  double xl = inf, xh = -inf, yl = inf, yh = -inf, zl = inf, zh = -inf;
+  double xl = real ? px : inf, xh = real ? px : -inf, yl = real ? py : inf, yh = real ? py : -inf;
+  double zl = real ? pz : inf, zh = real ? pz : -inf;
   int nreal = real ? 1 : 0;
-  if (real) {
-    xl = xh = x[s];
-    yl = yh = y[s];
-    zl = zh = z[s];
-  }
   for (int off = M >> 1; off > 0; off >>= 1) {
     xl = fmin(xl, __shfl_xor(xl, off, kWave));
     xh = fmax(xh, __shfl_xor(xh, off, kWave));
@@ -563,13 +564,216 @@ __global__ void k_cluster_bbox(int64_t nitems, Segs sg, int32_t M, const double 
     zh = fmax(zh, __shfl_xor(zh, off, kWave));
     nreal += __shfl_xor(nreal, off, kWave);
   }
-  if (mine && s % M == 0) {
+  if (!mine) return 0.f;
+  const double cx = (xl + xh) * 0.5, cy = (yl + yh) * 0.5, cz = (zl + zh) * 0.5;
+  if (s % M == 0) {
     const int64_t c = s / M;
-    double *bb = bbox + 6 * c;
+    double *bb = o.bbox + 6 * c;
     bb[0] = xl; bb[1] = yl; bb[2] = zl; bb[3] = xh; bb[4] = yh; bb[5] = zh;
-    c0[c] = make_double4((xl + xh) * 0.5, (yl + yh) * 0.5, (zl + zh) * 0.5, (double)nreal);
-    if (lcount && nreal == 0) lcount[c] = 0;
+    o.c0[c] = make_double4(cx, cy, cz, (double)nreal);
+    if (o.lcount && nreal == 0) o.lcount[c] = 0;
   }
+  if (!o.pos32) return 0.f;
+  float4 p = make_float4(kPadPos32, kPadPos32, kPadPos32, __int_as_float(0));
+  double4 d = make_double4(kDummyPos, kDummyPos, kDummyPos, 0.);
+  float e = 0.f;
+  if (real) {
+    d = make_double4(px, py, pz, 0.);
+    p = make_float4((float)(px - cx), (float)(py - cy), (float)(pz - cz), __int_as_float(type));
+    e = fmaxf(fabsf(p.x), fmaxf(fabsf(p.y), fabsf(p.z)));
+  }
+  o.pos32[s] = p;
+  o.pos32_next[s] = p;
+  o.posd[s] = d;
+  o.posd_next[s] = d;
+  return e;
+}
+
+// The permutation of a whole build: new slot s takes the particle of old slot src[s]; src[s] < 0 makes a
+// padding slot.  The rebuild reference positions are set to the positions; when posfx is given the slots'
+// 32-bit fixed-point positions are written too (type -1 for padding).  Inside the step loop the force is
+// recomputed right after a rebuild, so it is not carried.  The cluster's box and FP32 positions come from the
+// values this pass holds anyway: passes of their own over the slots cost 21 and (cluster-entry builds) 40 us more at 2.0M slots, and two
+// launches.
+__global__ __launch_bounds__(256) void k_permute_clusters(int64_t nnew, int32_t M, const int32_t *__restrict__ src,
+                                                          StateView o, StateView n, int32_t carry_force,
+                                                          int4 *__restrict__ posfx, FixGeom f, ClusterOut out) {
+  const int64_t s = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool mine = s < nnew;
+  const int32_t k = mine ? src[s] : -1;
+  double x = kDummyPos, y = kDummyPos, z = kDummyPos;
+  int32_t t = 0;
+  if (k >= 0) {
+    x = o.x[k]; y = o.y[k]; z = o.z[k];
+    t = o.type[k];
+    n.vx[s] = o.vx[k]; n.vy[s] = o.vy[k]; n.vz[s] = o.vz[k];
+    if (carry_force) { n.fx[s] = o.fx[k]; n.fy[s] = o.fy[k]; n.fz[s] = o.fz[k]; }
+    n.ofx[s] = o.ofx[k]; n.ofy[s] = o.ofy[k]; n.ofz[s] = o.ofz[k];
+    n.orig[s] = o.orig[k]; n.id[s] = o.id[k];
+    if (posfx)
+      posfx[s] = make_int4((int32_t)(uint32_t)(uint64_t)__double2ll_rn((x - f.min[0]) * f.inv_scale[0]),
+                           (int32_t)(uint32_t)(uint64_t)__double2ll_rn((y - f.min[1]) * f.inv_scale[1]),
+                           (int32_t)(uint32_t)(uint64_t)__double2ll_rn((z - f.min[2]) * f.inv_scale[2]), t);
+  } else if (mine) {
+    n.vx[s] = 0.; n.vy[s] = 0.; n.vz[s] = 0.;
+    n.fx[s] = 0.; n.fy[s] = 0.; n.fz[s] = 0.;
+    n.ofx[s] = 0.; n.ofy[s] = 0.; n.ofz[s] = 0.;
+    n.orig[s] = -1; n.id[s] = -1;
+    if (posfx) posfx[s] = make_int4(0, 0, 0, -1);
+  }
+  if (mine) {
+    n.x[s] = x;  n.y[s] = y;  n.z[s] = z;
+    n.rx[s] = x; n.ry[s] = y; n.rz[s] = z;
+    n.type[s] = t;
+  }
+  const float e = cluster_derive(s, M, mine, k >= 0, x, y, z, t, out);
+  if (out.pos32) block_max_to_lines(e, out.ext);
+}
+
+// The second half of a partial ensemble build's permutation (k_permute_boxes gathered the marked boxes'
+// slots into the other buffer): the slots are copied back, with what the layout derives from them.
+__global__ __launch_bounds__(256) void k_copy_box_clusters(int64_t nitems, Segs sg, int32_t M, StateView from,
+                                                           StateView to, const unsigned long long *__restrict__ skip,
+                                                           ClusterOut out) {
+  if (skip && *skip) return;
+  const int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  const bool mine = it < nitems;  // the segments hold the marked boxes' whole clusters
+  const int64_t s = mine ? seg_index(sg, it) : 0;
+  double x = 0., y = 0., z = 0.;
+  int32_t t = 0, g = -1;
+  if (mine) {
+    x = from.x[s]; y = from.y[s]; z = from.z[s];
+    t = from.type[s]; g = from.orig[s];
+    to.x[s] = x; to.y[s] = y; to.z[s] = z;
+    to.vx[s] = from.vx[s]; to.vy[s] = from.vy[s]; to.vz[s] = from.vz[s];
+    to.fx[s] = from.fx[s]; to.fy[s] = from.fy[s]; to.fz[s] = from.fz[s];
+    to.ofx[s] = from.ofx[s]; to.ofy[s] = from.ofy[s]; to.ofz[s] = from.ofz[s];
+    to.rx[s] = x; to.ry[s] = y; to.rz[s] = z;  // a rebuild's reference is its positions
+    to.type[s] = t; to.orig[s] = g; to.id[s] = from.id[s];
+  }
+  const float e = cluster_derive(s, M, mine, g >= 0, x, y, z, t, out);
+  block_max_to_lines(e, out.ext);
+}
+
+// The first passes of a small build in one workgroup: wrap and towers of the particles, tower and cluster
+// offsets, and each particle's place among its tower's (z, then id) by counting those before it, with the
+// tower's z in LDS.  A build of a few hundred to a few thousand particles is bound by its launches (~5 us
+// each with the gap before it), and these were seven: clear, histogram, offsets, their marker, scatter, sort,
+// and a second clear.  The sizes go to the host's marker words as soon as they are known.  Towers longer than
+// kSmallTower are left to the sorts of the general path, which find the histogram's results in place.
+// A job of 700 particles with 150 steps and 15 builds: 2805 -> 2385 us with the other launches saved.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallSlots = 4096;   // old slots (padding included); also bounds the offsets below 2^16
+constexpr int kSmallTowers = kSmallThreads;
+constexpr int kSmallTower = 256;
+
+__global__ __launch_bounds__(kSmallThreads) void k_tower_small(
+    int32_t nslots, double *__restrict__ x, double *__restrict__ y, double *__restrict__ z,
+    const int32_t *__restrict__ orig, const int64_t *__restrict__ id, TowerGeom g, WrapArgs w, int32_t ntow, int32_t M,
+    int32_t *__restrict__ tower_of, int32_t *__restrict__ rank, int32_t *__restrict__ count,
+    int64_t *__restrict__ start, int32_t *__restrict__ ccount, int64_t *__restrict__ cstart, int32_t *__restrict__ src,
+    int32_t *__restrict__ cluster_tower, unsigned long long *__restrict__ tstats,
+    unsigned long long *__restrict__ stats, unsigned long long *__restrict__ ext, unsigned long long *__restrict__ mark,
+    unsigned long long seq) {
+  constexpr int PER = kSmallSlots / kSmallThreads, WAVES = kSmallThreads / kWave;
+  __shared__ double s_z[kSmallSlots];
+  __shared__ int32_t s_i[kSmallSlots];
+  __shared__ int32_t s_cnt[kSmallTowers], s_off[kSmallTowers];  // particles; particle | cluster << 16 offsets
+  __shared__ int32_t s_tot[WAVES], s_max[WAVES];
+  const int tid = threadIdx.x, lane = tid & (kWave - 1), wv = tid / kWave;
+  s_cnt[tid] = 0;
+  if (tid < 6) stats[tid] = 0ull;
+  if (ext && tid < kAccSlots * kAccStride) ext[tid] = 0ull;
+  __syncthreads();
+  double pz[PER];
+  int32_t t[PER], r[PER];
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const int i = tid + k * kSmallThreads;
+    t[k] = -1;
+    r[k] = 0;
+    pz[k] = 0.;
+    if (i < nslots) {
+      if (orig[i] >= 0) {
+        const double ox = x[i], oy = y[i], oz = z[i];
+        const double px = wrap_coord(ox, 0, w), py = wrap_coord(oy, 1, w);
+        pz[k] = wrap_coord(oz, 2, w);
+        if (px != ox) x[i] = px;
+        if (py != oy) y[i] = py;
+        if (pz[k] != oz) z[i] = pz[k];
+        t[k] = tower_index(g, px, py);
+        r[k] = atomicAdd(&s_cnt[t[k]], 1);
+      }
+      tower_of[i] = t[k];
+      rank[i] = r[k];
+    }
+  }
+  __syncthreads();
+  const int32_t n = tid < ntow ? s_cnt[tid] : 0, nc = (n + M - 1) / M;
+  int32_t inc = n | (nc << 16), mx = n;
+  for (int off = 1; off < kWave; off <<= 1) {
+    const int32_t a = __shfl_up(inc, off, kWave), m = __shfl_xor(mx, off, kWave);
+    if (lane >= off) inc += a;
+    mx = m > mx ? m : mx;
+  }
+  if (lane == kWave - 1) {
+    s_tot[wv] = inc;
+    s_max[wv] = mx;
+  }
+  __syncthreads();
+  int32_t before = 0, total = 0, longest = 0;
+#pragma unroll
+  for (int k = 0; k < WAVES; ++k) {
+    before += k < wv ? s_tot[k] : 0;
+    total += s_tot[k];
+    longest = s_max[k] > longest ? s_max[k] : longest;
+  }
+  const int32_t first = before + inc - (n | (nc << 16));
+  s_off[tid] = first;
+  const int32_t c0 = (int32_t)((uint32_t)first >> 16);
+  if (tid < ntow) {
+    count[tid] = n;
+    start[tid] = first & 0xffff;
+    ccount[tid] = nc;
+    cstart[tid] = c0;
+  }
+  if (tid == 0) {
+    const unsigned long long np = (unsigned long long)(total & 0xffff), ncl = (uint32_t)total >> 16;
+    start[ntow] = (int64_t)np;
+    cstart[ntow] = (int64_t)ncl;
+    tstats[0] = mark[1] = np;
+    tstats[1] = mark[2] = (unsigned long long)longest;
+    tstats[2] = mark[3] = ncl;
+    tstats[3] = mark[4] = 0ull;  // the shortest tower is not tracked
+    __threadfence_system();
+    mark[0] = seq;
+  }
+  if (longest > kSmallTower) return;
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    if (t[k] >= 0) {
+      const int p = (s_off[t[k]] & 0xffff) + r[k];
+      s_z[p] = pz[k];
+      s_i[p] = tid + k * kSmallThreads;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < PER; ++k)
+    if (t[k] >= 0) {
+      const int i = tid + k * kSmallThreads, b = s_off[t[k]] & 0xffff, e = b + s_cnt[t[k]];
+      int place = 0;
+#pragma unroll 4
+      for (int m = b; m < e; ++m) {
+        const double zm = s_z[m];
+        bool less = zm < pz[k];
+        if (zm == pz[k] && s_i[m] != i) less = id[s_i[m]] < id[i];
+        place += less ? 1 : 0;
+      }
+      src[(int)((uint32_t)s_off[t[k]] >> 16) * M + place] = i;
+    }
+  for (int q = n; q < nc * M; ++q) src[c0 * M + q] = -1;
+  for (int q = 0; q < nc; ++q) cluster_tower[c0 + q] = tid;
 }
 
 // Newton-3 lists keep only forward entries: a higher j-cluster, or the i-cluster itself at shift id 13 (its
@@ -1197,64 +1401,6 @@ __global__ void k_zero_u64(int64_t n, unsigned long long *__restrict__ p) {
   if (i < n) p[i] = 0ull;
 }
 
-// FP32 position relative to the cluster reference point, particle type bits in w.  Padding slots sit at
-// the sentinel +3e30 in every coordinate: any distance to them squares to +inf in FP32, which fails the
-// cutoff test, while the difference itself stays finite (so masked terms contribute exact zeros).
-// Written to both position buffers: the fused integrator of the FP32 cluster kernel writes the real
-// slots of the second one each step, and the padding slots must hold the sentinel in both.  The FP64
-// positions go to posd (both buffers too), and the largest |component| of the real slots' FP32 positions
-// into the lines of ext.
-__global__ void k_pos32(int64_t nslots, Segs sg, int32_t M, const double *__restrict__ x, const double *__restrict__ y,
-                        const double *__restrict__ z, const int32_t *__restrict__ type,
-                        const int32_t *__restrict__ orig, const double4 *__restrict__ c0, float4 *__restrict__ pos32,
-                        float4 *__restrict__ pos32_next, double4 *__restrict__ posd, double4 *__restrict__ posd_next,
-                        unsigned long long *__restrict__ ext, const int32_t *__restrict__ cluster_box,
-                        const int32_t *__restrict__ box_active) {
-  const int64_t it = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  float e = 0.f;
-  if (it < nslots) {
-    const int64_t s = seg_index(sg, it);
-    if (!box_active || box_active[cluster_box[s / M]] != 0) {
-      float4 p;
-      double4 d;
-      if (orig[s] < 0) {
-        p = make_float4(kPadPos32, kPadPos32, kPadPos32, __int_as_float(0));
-        d = make_double4(kDummyPos, kDummyPos, kDummyPos, 0.);
-      } else {
-        const double4 r = c0[s / M];
-        d = make_double4(x[s], y[s], z[s], 0.);
-        p = make_float4((float)(d.x - r.x), (float)(d.y - r.y), (float)(d.z - r.z), __int_as_float(type[s]));
-        e = fmaxf(fabsf(p.x), fmaxf(fabsf(p.y), fabsf(p.z)));
-      }
-      pos32[s] = p;
-      pos32_next[s] = p;
-      posd[s] = d;
-      posd_next[s] = d;
-    }
-  }
-  block_max_to_lines(e, ext);
-}
-
-void vcl_pos32(Ctx &c, const int32_t *active) {
-  c.pos32.ensure(c.nslots);
-  c.pos32_next.ensure(c.nslots);
-  c.posd.ensure(c.nslots);
-  c.posd_next.ensure(c.nslots);
-  c.pos32_ext.ensure(kAccSlots * kAccStride);
-  State &s = c.st[c.cur];
-  const int64_t ni = active ? c.seg_nslots : c.nslots;
-  const Segs sg = active ? c.seg_slots : Segs{nullptr, nullptr, 0};
-  // a whole build starts the bound again; a partial one only raises it (the other boxes keep theirs)
-  if (!active)
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(kAccSlots * kAccStride), 0, c.stream,
-                       (int64_t)(kAccSlots * kAccStride), c.pos32_ext.p);
-  if (ni == 0) return;
-  hipLaunchKernelGGL(k_pos32, dim3(blocks_for(ni, 256)), dim3(256), 0, c.stream, ni, sg, c.M, s.x.p, s.y.p, s.z.p,
-                     s.type.p, s.orig.p, c.c0.p, c.pos32.p, c.pos32_next.p, c.posd.p, c.posd_next.p, c.pos32_ext.p,
-                     c.cluster_box.p, active);
-  LJG_HIP(hipGetLastError());
-}
-
 // Member rows of the FP32 cluster kernel.  VCLClusterFunctor evaluates every member of every listed
 // j-cluster against every i-member (VCLClusterFunctor.h:38-89); a listed j-cluster (bounding boxes within
 // ilen) holds members farther than ilen from all i-members, which can never come within rc before the
@@ -1301,7 +1447,7 @@ __global__ __launch_bounds__(kXrowThreads) void k_cluster_xrows(int64_t nitems, 
     yi[q] = p.y;
     zi[q] = p.z;
   }
-  const int nj = live ? lcount[ic] * M : 0;
+  const int nj = live ? min(lcount[ic], row) * M : 0;
   int nmax = nj;  // the loop runs to the wave's longest stream so that the ballots stay uniform
 #pragma unroll
   for (int off = kWave / 2; off >= LG; off >>= 1) {
@@ -1421,6 +1567,20 @@ void vcl_member_rows(Ctx &c, bool partial, const int32_t *active) {
   c.xrows_valid = true;
 }
 
+// What a build starts from at zero, in one launch: the tower counts (n of them), the list statistics, and
+// where given the tower statistics and the lines of the FP32 positions' bound.
+constexpr int kExtWords = kAccSlots * kAccStride;
+static_assert(kExtWords <= 256, "one workgroup clears the lines");
+
+__global__ void k_clear_build(int64_t n, int32_t *__restrict__ count, unsigned long long *__restrict__ stats,
+                              unsigned long long *__restrict__ tstats, unsigned long long *__restrict__ ext) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) count[i] = 0;
+  if (i < 6) stats[i] = 0ull;
+  if (tstats && i < 4) tstats[i] = 0ull;
+  if (ext && i < kExtWords) ext[i] = 0ull;
+}
+
 __global__ void k_fill_i32(int64_t n, int32_t *__restrict__ p, int32_t v) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i] = v;
@@ -1504,21 +1664,44 @@ void vcl_build(Ctx &c) {
   c.ctow_count.ensure(ntow + 1);
   c.ctow_start.ensure(ntow + 1);
   c.flag.ensure(4);
-  fill_i32(c, c.tower_count.p, ntow + 1, 0);
   c.tstats.ensure(4);
+  // list_stats: [0], [1] total and longest row of the cluster-pair pass, [2] frame flag of the expansion
+  // pass, [3], [4] total and longest j-particle row, [5] sort tile exceeded; read back once at the end
+  c.list_stats.ensure(6);
+  c.pos32_ext.ensure(kExtWords);
+  const bool jrows = c.want_jrows;
+  // Small builds: the passes up to the sorts in one workgroup.  4096 slots at four per thread; a tower each.
+  const bool small = !ens && ns <= kSmallSlots && ntow <= kSmallTowers;
+  unsigned long long smark = 0;
+  if (small) {
+    const int64_t bound = c.n / M + ntow;  // clusters
+    c.perm.ensure(bound * M);
+    c.cluster_tower.ensure(bound);
+    smark = ++c.mark_seq;
+    hipLaunchKernelGGL(k_tower_small, dim3(1), dim3(kSmallThreads), 0, c.stream, (int32_t)ns, s.x.p, s.y.p, s.z.p,
+                       s.orig.p, s.id.p, g, wrap_args(c.prm), (int32_t)ntow, M, c.tower_of.p, c.rank.p,
+                       c.tower_count.p, c.tower_start.p, c.ctow_count.p, c.ctow_start.p, c.perm.p, c.cluster_tower.p,
+                       c.tstats.p, c.list_stats.p, jrows ? (unsigned long long *)nullptr : c.pos32_ext.p,
+                       c.pin_mark_dev, smark);
+    LJG_HIP(hipGetLastError());
+  }
+  // (a partial build only raises the bound of the FP32 positions: the other boxes keep theirs)
+  if (!small)
+    hipLaunchKernelGGL(k_clear_build, dim3(blocks_for(ntow + 1 > 256 ? ntow + 1 : 256, 256)), dim3(256), 0, c.stream,
+                     ntow + 1, c.tower_count.p, c.list_stats.p, ens ? c.tstats.p : (unsigned long long *)nullptr,
+                     jrows || partial ? (unsigned long long *)nullptr : c.pos32_ext.p);
+  LJG_HIP(hipGetLastError());
   if (ens) {
     // per-box layouts inside the fixed regions; only the longest tower is needed from the stats
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c.stream, (int64_t)4, c.tstats.p);
-    LJG_HIP(hipGetLastError());
     ensemble_tower_hist(c, active);
     ensemble_layout(c, active);
-  } else {
+  } else if (!small) {
     hipLaunchKernelGGL(k_tower_hist, dim3(blocks_for(ns, 256)), dim3(256), 0, c.stream, ns, s.x.p, s.y.p, s.z.p,
                        s.orig.p, g, wrap_args(c.prm), c.tower_of.p, c.rank.p, c.tower_count.p);
     LJG_HIP(hipGetLastError());
   }
   // tower offsets, clusters per tower and their offsets, and the sizes for the one synchronisation
-  if (ens) {
+  if (ens || small) {
   } else if (ntow <= kLayoutOneBlockMax) {
     hipLaunchKernelGGL(k_tower_layout, dim3(1), dim3(kLayoutThreads), 0, c.stream, ntow, c.tower_count.p, M,
                        c.tower_start.p, c.ctow_count.p, c.ctow_start.p, c.tstats.p);
@@ -1544,20 +1727,16 @@ void vcl_build(Ctx &c) {
   const Segs sg_clusters = partial ? c.seg_clusters : none;
   const int64_t n_slots = partial ? c.seg_nslots : ns, n_towers = partial ? c.seg_ntowers : ntow;
   const bool guess = partial && !c.partial_tower_sync;
-  // The sizes' marker goes before the scatter and the clearing of the list statistics, which need no
-  // size: they run while the host waits for it, and the first launch after the wait is a long one.
-  const unsigned long long tmark = guess ? 0ull : stream_mark(c, c.tstats.p, 4);
-  // list_stats: [0], [1] total and longest row of the cluster-pair pass, [2] frame flag of the expansion
-  // pass, [3], [4] total and longest j-particle row, [5] sort tile exceeded; read back once at the end
-  c.list_stats.ensure(6);
-  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c.stream, (int64_t)6, c.list_stats.p);
-  LJG_HIP(hipGetLastError());
-  if (n_slots > 0) {
+  // The sizes' marker goes before the scatter, which needs no size: it runs while the host waits.
+  const unsigned long long tmark = small ? smark : guess ? 0ull : stream_mark(c, c.tstats.p, 4);
+  auto scatter = [&]() {
+    if (n_slots == 0) return;
     hipLaunchKernelGGL(k_tower_scatter, dim3(blocks_for(n_slots, 256)), dim3(256), 0, c.stream, n_slots, sg_slots,
                        c.tower_of.p, c.rank.p, c.tower_start.p, s.z.p, s.id.p, c.tower_items.p, c.tower_z.p,
                        c.tower_id.p);
     LJG_HIP(hipGetLastError());
-  }
+  };
+  if (!small) scatter();
   // The sizes: the longest tower picks the sort instances (only those are launched: an instance with a
   // large LDS tile or many registers waits for room on a GPU busy with other work).  A partial build uses
   // the expected longest tower of the marked boxes instead of waiting for the readback, and launches the
@@ -1580,7 +1759,9 @@ void vcl_build(Ctx &c) {
   // Towers of up to 1024 particles sort in registers (an instance by length, launched only if some tower is
   // in its range), longer ones in LDS.  Every tower is sorted by exactly one instance; the longest tower
   // (ts[1]) and the shortest non-empty one (ts[3], 0 when not known) bound which ones can have work.
-  if (n_towers > 0) {
+  const bool sorted = small && ts[1] <= (unsigned long long)kSmallTower;
+  if (small && !sorted) scatter();
+  if (n_towers > 0 && !sorted) {
 #define LJG_SORT(KERNEL, BLOCKS, THREADS, OVER)                                                                  \
   {                                                                                                             \
     hipLaunchKernelGGL(KERNEL, dim3(BLOCKS), dim3(THREADS), 0, c.stream, n_towers, sg_towers, c.tower_start.p,  \
@@ -1609,31 +1790,47 @@ void vcl_build(Ctx &c) {
       LJG_HIP(hipGetLastError());
     }
   }
-  const bool jrows = c.want_jrows;
   if (jrows && ens) throw HipError{hipErrorInvalidValue, "j-particle rows on an ensemble of boxes", -2};
+  if (jrows && M > kMaxM) throw HipError{hipErrorInvalidValue, "cluster size above 8", -2};
+  c.bbox.ensure(6 * ncl);
+  c.c0.ensure(ncl);
+  c.list_count.ensure(ncl * kJclSplit + 1);
+  ClusterOut out{c.bbox.p, c.c0.p, ens ? c.list_count.p : nullptr, nullptr, nullptr, nullptr, nullptr, c.pos32_ext.p};
   if (jrows) {
     // fixed-point positions of every slot (padding: type -1), written by the permutation
     verlet_geometry(c);
     c.posfx.ensure(new_slots);
+    c.jcount.ensure(ncl + 1);
+  } else {
+    c.pos32.ensure(new_slots);
+    c.pos32_next.ensure(new_slots);
+    c.posd.ensure(new_slots);
+    c.posd_next.ensure(new_slots);
+    out.pos32 = c.pos32.p;
+    out.pos32_next = c.pos32_next.p;
+    out.posd = c.posd.p;
+    out.posd_next = c.posd_next.p;
   }
-  if (partial) permute_active(c, c.perm.p, active, guess ? c.list_stats.p + 5 : nullptr);
-  else permute_state(c, c.perm.p, new_slots, jrows ? c.posfx.p : nullptr);
+  const int other = 1 - c.cur;
+  c.st[other].ensure((size_t)(partial ? c.nslots : new_slots));
+  if (partial) {
+    // the marked boxes' slots, gathered into the other buffer and copied back; nothing moves on guessed
+    // sizes that were too small
+    const unsigned long long *skip = guess ? c.list_stats.p + 5 : nullptr;
+    permute_active(c, c.perm.p, active, skip);
+    if (n_slots > 0)
+      hipLaunchKernelGGL(k_copy_box_clusters, dim3(blocks_for(n_slots, 256)), dim3(256), 0, c.stream, n_slots,
+                         sg_slots, M, view(c.st[other]), view(c.st[c.cur]), skip, out);
+  } else {
+    hipLaunchKernelGGL(k_permute_clusters, dim3(blocks_for(new_slots, 256)), dim3(256), 0, c.stream, new_slots, M,
+                       c.perm.p, view(c.st[c.cur]), view(c.st[other]), (int32_t)c.carry_force,
+                       jrows ? c.posfx.p : (int4 *)nullptr, c.fg, out);
+    c.cur = other;
+    c.nslots = new_slots;
+  }
+  LJG_HIP(hipGetLastError());
   c.regions_valid = ens;
   c.M = M;
-  State &t = c.st[c.cur];
-  c.bbox.ensure(6 * ncl);
-  c.c0.ensure(ncl);
-  c.list_count.ensure(ncl * kJclSplit + 1);
-  const int64_t n_bbox = partial ? c.seg_nslots : new_slots;
-  if (n_bbox > 0) {
-    hipLaunchKernelGGL(k_cluster_bbox, dim3(blocks_for(n_bbox, 256)), dim3(256), 0, c.stream, n_bbox, sg_slots, M,
-                       t.x.p, t.y.p, t.z.p, t.orig.p, c.bbox.p, c.c0.p,
-                       ens ? c.cluster_box.p : (const int32_t *)nullptr, active,
-                       ens ? c.list_count.p : (int32_t *)nullptr);
-    LJG_HIP(hipGetLastError());
-  }
-  if (jrows && M > kMaxM) throw HipError{hipErrorInvalidValue, "cluster size above 8", -2};
-  if (jrows) c.jcount.ensure(ncl + 1);
   // Both passes are queued back to back and checked with one synchronisation; a row that overflowed
   // its capacity (the expansion pass reads at most ccap entries) makes both run again with larger rows.
   // cluster-entry lists: a lane per i-cluster when the towers hold few clusters, unless the caller chose
@@ -1647,16 +1844,17 @@ void vcl_build(Ctx &c) {
   int32_t cap = jrows ? (c.jccap > 0 ? c.jccap : kJclSplit * 24)
                       : partial ? c.list_row : (c.list_cap > 0 ? c.list_cap : 64);
   int32_t jcap = c.jcap > 0 ? c.jcap : 160;
-  bool pos32_queued = false;
-  for (;;) {
+  for (bool again = false;; again = true) {
     if (jrows) {
       c.jcl.ensure((size_t)ncl * cap + 1);
       c.jlist.ensure((size_t)ncl * jcap + 1);
     } else {
       c.list.ensure((size_t)ncl * cap + 1);
     }
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c.stream, (int64_t)5, c.list_stats.p);
-    LJG_HIP(hipGetLastError());
+    if (again) {
+      hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, c.stream, (int64_t)5, c.list_stats.p);
+      LJG_HIP(hipGetLastError());
+    }
     const TowerGeom *no_tg = nullptr;
     const int64_t *no_i64 = nullptr;
     const int32_t *no_i32 = nullptr;
@@ -1698,7 +1896,6 @@ void vcl_build(Ctx &c) {
                          ntow, none, g, no_tg, no_i64, no_i32, no_i32, c.ctow_start.p, c.ctow_count.p, c.bbox.p, c.c0.p,
                          cap, c.list_count.p, c.list.p, (int32_t *)nullptr, n3);
     LJG_HIP(hipGetLastError());
-    count_stats(c, c.list_count.p, jrows ? ncl * kJclSplit : ncl, c.list_stats.p);
     if (jrows) {
       // i-clusters per wavefront of the expansion pass (tuned on the 10^6-particle liquid: 4 for M >= 4)
       // (one i-cluster per wave below 2048 clusters: latency-bound small builds)
@@ -1734,12 +1931,24 @@ void vcl_build(Ctx &c) {
       throw HipError{hipErrorInvalidValue, "unsupported (cluster size, expansion groups) combination", -2};
     expanded:
       LJG_HIP(hipGetLastError());
-      count_stats(c, c.jcount.p, ncl, c.list_stats.p + 3);
+    }
+    // the lengths of the rows, with the marker the host waits for unless it waits later
+    const bool defer = jrows && c.defer_lists && !partial && !ens && c.jccap > 0 && c.jcap > 0;
+    unsigned long long lmark = 0;
+    if (jrows) {
+      count_stats(c, c.list_count.p, ncl * kJclSplit, c.list_stats.p, c.jcount.p, ncl, c.list_stats.p + 3);
+      if (!defer) lmark = stream_mark(c, c.list_stats.p, 6);
+    } else {
+      lmark = count_stats_mark(c, c.list_count.p, ncl, c.list_stats.p, 6);
+      // the member rows are queued behind the marker: they are made while the host waits (a row cut off at
+      // its capacity makes short member rows, and both again)
+      c.list_row = cap;
+      if (!partial && !n3 && !c.prm.whole_cluster_rows) vcl_member_rows(c, false, nullptr);
     }
     // A j-row build the step loop follows with its force at once: the lengths are read after that launch,
     // which exits on the device if a row overflowed (vcl_finish_lists).  The first build of a context
     // (capacities not yet measured) is checked here.
-    if (jrows && c.defer_lists && !partial && !ens && c.jccap > 0 && c.jcap > 0) {
+    if (defer) {
       c.lists_pending = true;
       c.pend_cap = cap;
       c.pend_jcap = jcap;
@@ -1751,15 +1960,8 @@ void vcl_build(Ctx &c) {
       c.xrows_valid = false;
       return;
     }
-    // the FP32 positions of the cluster kernels need no list: queued before the wait, they are made while
-    // the host waits (once, also when the lists are made again with larger rows; not in a partial build
-    // on guessed sizes, which may find that nothing was permuted and start again)
-    if (!jrows && !guess && !pos32_queued) {
-      vcl_pos32(c, active);
-      pos32_queued = true;
-    }
     unsigned long long st[6] = {0, 0, 0, 0, 0, 0};
-    stream_wait(c, c.list_stats.p, 6, st);
+    stream_spin(c, lmark, 6, st);
     if (st[5] && guess) {
       // a marked tower was longer than the register sorts take: nothing was permuted, so build again
       // with the longest tower read back first
@@ -1804,9 +2006,8 @@ void vcl_build(Ctx &c) {
   c.lists_n3 = c.want_n3 && !jrows;
   c.built_M = M;
   c.layout = Layout::Clusters;
-  if (!jrows && !pos32_queued) vcl_pos32(c, active);
-  if (!jrows && !c.lists_n3 && !c.prm.whole_cluster_rows) vcl_member_rows(c, partial, active);
-  else c.xrows_valid = false;
+  if (jrows || c.lists_n3 || c.prm.whole_cluster_rows) c.xrows_valid = false;
+  else if (partial) vcl_member_rows(c, true, active);
 }
 
 }  // namespace ljg

@@ -69,3 +69,29 @@ def test_tower_sorts_at_their_edges(oracle, longest):
     r = oracle.vcl_periodic(wx, wy, wz, ids, (0, 0, 0), box, RC + SKIN, 8)
     for k in ("slot_particle", "cluster_tower", "bbox"):
         assert np.array_equal(g[k], r[k]), k
+
+
+@pytest.mark.parametrize("M", [1, 4, 8])
+@pytest.mark.parametrize("n,box,column", [(5, (6.0, 6.0, 6.0), 0), (700, (10.0, 10.0, 10.0), 0), (1024, (40.0, 40.0, 4.0), 0),
+                                          (1025, (40.0, 40.0, 4.0), 0), (2000, (9.0, 9.0, 60.0), 256),
+                                          (2000, (9.0, 9.0, 60.0), 257), (4096, (17.0, 17.0, 18.0), 0),
+                                          (4097, (17.0, 17.0, 18.0), 0), (4096, (200.0, 200.0, 3.0), 0)])
+def test_small_builds(oracle, M, n, box, column):
+    # sizes around the limits of the one-workgroup passes: 4096 slots, 1024 towers, towers of 256; ties in z;
+    # positions outside the box (wrapped); then a second build from the padded cluster layout
+    announce(f"small build n={n} M={M} box {box} column {column}")
+    rng = np.random.default_rng(n + M + column)
+    x, y, z = (rng.uniform(-0.5 * b, 1.5 * b, n) for b in box)
+    z[1::3] = z[::3][:len(z[1::3])]
+    if column:
+        x[:column], y[:column] = 0.1, 0.1
+    ids = rng.permutation(n).astype(np.int64)
+    wx, wy, wz = oracle.wrap(x, y, z, (0, 0, 0), box)
+    r = oracle.vcl_periodic(wx, wy, wz, ids, (0, 0, 0), box, RC + SKIN, M)
+    with ap.Engine((0.0, 0.0, 0.0), box, RC, SKIN, cluster_size=M) as e:
+        e.upload(x, y, z, id=ids)
+        for _ in range(2):
+            e.build_pairs()
+            g = e.clusters()
+            for k in ("slot_particle", "cluster_tower", "list_offsets", "list_j", "list_shift", "bbox"):
+                assert np.array_equal(g[k], r[k]), k
