@@ -35,6 +35,7 @@ SOURCES = {
     "ljg_force.hip": [],
     "ljg_jrows.hip": [],
     "ljg_lc.hip": [],
+    "ljg_transfer.hip": [],
     "ljg_verlet.hip": ["-ffp-contract=off"],
     "ljg_ensemble.hip": ["-ffp-contract=off"],
     "ljg_generate.cpp": ["-ffp-contract=off"],

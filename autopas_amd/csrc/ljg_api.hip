@@ -38,16 +38,6 @@ static ljg_status fail(Ctx &c, ljg_status st, const std::string &msg) {
     return fail(c, LJG_ERR_HIP, "host allocation failed");                                          \
   }
 
-__global__ void k_init_upload(int64_t n, StateView s, const int64_t *__restrict__ id_in, int32_t have_id) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  s.fx[i] = 0.; s.fy[i] = 0.; s.fz[i] = 0.;
-  s.ofx[i] = 0.; s.ofy[i] = 0.; s.ofz[i] = 0.;
-  s.rx[i] = s.x[i]; s.ry[i] = s.y[i]; s.rz[i] = s.z[i];
-  s.orig[i] = (int32_t)i;
-  s.id[i] = have_id ? id_in[i] : i;
-}
-
 // Positions, velocities and forces of the particles with upload indices [first, first + count), array by
 // array (x, y, z, vx, vy, vz, fx, fy, fz), count values each.
 __global__ void k_gather_range(int64_t nslots, const int32_t *__restrict__ orig, int64_t first, int64_t count,
@@ -339,7 +329,7 @@ ljg_status ljg_destroy(ljg_ctx *h) {
   c.tower_items.release(); c.tower_z.release(); c.tower_id.release(); c.ctow_count.release(); c.ctow_start.release(); c.cluster_tower.release();
   c.bbox.release(); c.c0.release(); c.list_count.release(); c.list_stats.release(); c.list.release();
   c.pos32.release(); c.pos32_next.release(); c.posd.release(); c.posd_next.release(); c.pos32_ext.release(); c.posfx.release(); c.jcl.release(); c.jlist.release(); c.jcount.release(); c.xrow.release(); c.xcount.release(); c.xrow_tmp.release(); c.xcount_tmp.release(); c.tstats.release(); c.posfx_next.release(); c.hits_slots.release(); c.vcount.release(); c.vlist.release(); c.tab.release(); c.part_e.release(); c.part_v.release(); c.part_hits.release();
-  c.red_out.release(); c.red_hits.release(); c.flag.release(); c.scan_tmp.release();
+  c.flag.release(); c.scan_tmp.release();
   c.box_tg.release(); c.box_wrap.release(); c.box_of.release(); c.box_tbase.release(); c.tower_box.release();
   c.box_cbase.release(); c.box_pbase.release(); c.cluster_box.release();
   c.box_flag.release(); c.list_tmp.release(); c.seg_buf.release(); c.cell_sorted.release();
@@ -350,7 +340,7 @@ ljg_status ljg_destroy(ljg_ctx *h) {
   if (c.host_flag) (void)hipHostFree(c.host_flag);
   if (c.pin_mark) (void)hipHostFree(c.pin_mark);
   if (c.pin_seg) (void)hipHostFree(c.pin_seg);
-  if (c.pin_dl) (void)hipHostFree(c.pin_dl);
+  release_stage(c);
   if (c.pin_flags) (void)hipHostFree(c.pin_flags);
   for (auto e : c.event_pool) (void)hipEventDestroy(e);
   if (c.ev0) (void)hipEventDestroy(c.ev0);
@@ -443,7 +433,6 @@ static void mix_types(Ctx &c, int32_t ntypes, const double *eps, const double *s
 
 // The periodic box the kernels work in; the particles are dropped.
 static void reset_box(Ctx &c, const double box_min[3], const double box_max[3]) {
-  LJG_HIP(hipStreamSynchronize(c.stream));
   for (int d = 0; d < 3; ++d) {
     c.prm.box_min[d] = box_min[d];
     c.prm.box_max[d] = box_max[d];
@@ -490,20 +479,6 @@ ljg_status ljg_set_owned(ljg_ctx *h, int64_t n_owned) {
   c.box_glob_valid = false;
   return LJG_OK;
   LJG_API_END
-}
-
-// An open box takes particles in its halo region only (host arrays, checked before any copy).
-static const char *outside_open_region(const Ctx &c, int64_t n, const double *x, const double *y,
-                                       const double *z) {
-  if (!c.open) return nullptr;
-  const double ilen = c.prm.cutoff + c.prm.skin;
-  const double *p[3] = {x, y, z};
-  for (int d = 0; d < 3; ++d) {
-    const double lo = c.open_min[d] - ilen, hi = c.open_max[d] + ilen;
-    for (int64_t i = 0; i < n; ++i)
-      if (!(p[d][i] >= lo && p[d][i] <= hi)) return "particle outside the open box and its halo region";
-  }
-  return nullptr;
 }
 
 ljg_status ljg_set_box(ljg_ctx *h, const double box_min[3], const double box_max[3]) {
@@ -662,27 +637,16 @@ ljg_status ljg_edit_boxes(ljg_ctx *h, int32_t nkeep, const int32_t *keep, int32_
 }
 
 // Upload indices [first, first + count): one pass gathers the nine arrays (null outputs are skipped on the
-// host), one copy brings them back through pinned memory.
+// host), which come back through pinned memory.
 static void gather_range(Ctx &c, int64_t first, int64_t count, double *x, double *y, double *z, double *vx,
                          double *vy, double *vz, double *fx, double *fy, double *fz) {
   State &s = c.st[c.cur];
   double *outs[9] = {x, y, z, vx, vy, vz, fx, fy, fz};
-  const size_t bytes = 9 * (size_t)count * sizeof(double);
   c.part_v.ensure(9 * (size_t)count);
   hipLaunchKernelGGL(k_gather_range, dim3(blocks_for(c.nslots, 256)), dim3(256), 0, c.stream, c.nslots, s.orig.p,
                      first, count, view(s), c.part_v.p);
   LJG_HIP(hipGetLastError());
-  if (c.pin_dl_cap < bytes) {
-    if (c.pin_dl) LJG_HIP(hipHostFree(c.pin_dl));
-    c.pin_dl = nullptr;
-    c.pin_dl_cap = 0;
-    LJG_HIP(hipHostMalloc((void **)&c.pin_dl, bytes + bytes / 2, hipHostMallocDefault));
-    c.pin_dl_cap = bytes + bytes / 2;
-  }
-  LJG_HIP(hipMemcpyAsync(c.pin_dl, c.part_v.p, bytes, hipMemcpyDeviceToHost, c.stream));
-  stream_wait(c);
-  for (int k = 0; k < 9; ++k)
-    if (outs[k]) std::memcpy(outs[k], c.pin_dl + (size_t)k * count, (size_t)count * sizeof(double));
+  download_arrays(c, c.part_v.p, (size_t)count, outs);
 }
 
 ljg_status ljg_download_range(ljg_ctx *h, int64_t first, int64_t count, double *x, double *y, double *z, double *vx,
@@ -717,6 +681,8 @@ ljg_status ljg_get_box_globals(ljg_ctx *h, int32_t nboxes, double *potential_ene
   LJG_API_END
 }
 
+static const char *const kOutsideRegion = "particle outside the open box and its halo region";
+
 ljg_status ljg_upload(ljg_ctx *h, int64_t n, const double *x, const double *y, const double *z, const double *vx,
                       const double *vy, const double *vz, const int32_t *type, const int64_t *id) {
   if (!h || n <= 0 || n > (int64_t)INT32_MAX / 2 || !x || !y || !z) return LJG_ERR_ARG;
@@ -730,41 +696,13 @@ ljg_status ljg_upload(ljg_ctx *h, int64_t n, const double *x, const double *y, c
     for (int64_t k : c.box_count) total += k;
     if (n != total) return fail(c, LJG_ERR_ARG, "particle count differs from the ensemble's boxes");
   }
-  if (const char *why = outside_open_region(c, n, x, y, z)) return fail(c, LJG_ERR_ARG, why);
+  const double *const pos[3] = {x, y, z}, *const vel[3] = {vx, vy, vz};
+  if (!upload_state(c, n, pos, vel, type, id)) return fail(c, LJG_ERR_ARG, kOutsideRegion);
   c.box_glob_valid = false;
   c.n_owned = -1;
-  c.cur = 0;
-  c.st[0].ensure((size_t)n);
   c.n = n;
   c.nslots = n;
-  State &s = c.st[0];
-  const size_t bytes = (size_t)n * sizeof(double);
-  LJG_HIP(hipMemcpyAsync(s.x.p, x, bytes, hipMemcpyHostToDevice, c.stream));
-  LJG_HIP(hipMemcpyAsync(s.y.p, y, bytes, hipMemcpyHostToDevice, c.stream));
-  LJG_HIP(hipMemcpyAsync(s.z.p, z, bytes, hipMemcpyHostToDevice, c.stream));
-  if (vx && vy && vz) {
-    LJG_HIP(hipMemcpyAsync(s.vx.p, vx, bytes, hipMemcpyHostToDevice, c.stream));
-    LJG_HIP(hipMemcpyAsync(s.vy.p, vy, bytes, hipMemcpyHostToDevice, c.stream));
-    LJG_HIP(hipMemcpyAsync(s.vz.p, vz, bytes, hipMemcpyHostToDevice, c.stream));
-  } else {
-    LJG_HIP(hipMemsetAsync(s.vx.p, 0, bytes, c.stream));
-    LJG_HIP(hipMemsetAsync(s.vy.p, 0, bytes, c.stream));
-    LJG_HIP(hipMemsetAsync(s.vz.p, 0, bytes, c.stream));
-  }
-  if (type) LJG_HIP(hipMemcpyAsync(s.type.p, type, (size_t)n * sizeof(int32_t), hipMemcpyHostToDevice, c.stream));
-  else LJG_HIP(hipMemsetAsync(s.type.p, 0, (size_t)n * sizeof(int32_t), c.stream));
-  int64_t *did = nullptr;
-  if (id) {
-    c.scan_tmp.ensure((size_t)n);
-    did = c.scan_tmp.p;
-    LJG_HIP(hipMemcpyAsync(did, id, (size_t)n * sizeof(int64_t), hipMemcpyHostToDevice, c.stream));
-  }
-  hipLaunchKernelGGL(k_init_upload, dim3(blocks_for(n, 256)), dim3(256), 0, c.stream, n, view(s), did,
-                     (int32_t)(id != nullptr));
-  LJG_HIP(hipGetLastError());
   if (c.nboxes > 0) ensemble_wrap(c);
-  else wrap_positions(c);
-  stream_wait(c);  // the caller's arrays are free to change once this returns
   c.layout = Layout::Upload;
   c.regions_valid = false;
   c.have_forces = false;
@@ -797,20 +735,18 @@ ljg_status ljg_update_positions(ljg_ctx *h, const double *x, const double *y, co
   if (!h || !x || !y || !z) return LJG_ERR_ARG;
   LJG_API_BEGIN(h)
   if (c.n == 0) return fail(c, LJG_ERR_STATE, "no particles uploaded");
-  if (const char *why = outside_open_region(c, c.n, x, y, z)) return fail(c, LJG_ERR_ARG, why);
-  const bool vel = vx && vy && vz;
+  const double *const pos[3] = {x, y, z}, *const vel[3] = {vx, vy, vz};
+  const bool hv = vx && vy && vz;
   const size_t n = (size_t)c.n;
-  c.part_v.ensure((vel ? 6 : 3) * n);
-  double *buf = c.part_v.p;
-  const double *src[6] = {x, y, z, vx, vy, vz};
-  for (int k = 0; k < (vel ? 6 : 3); ++k)
-    LJG_HIP(hipMemcpyAsync(buf + k * n, src[k], n * sizeof(double), hipMemcpyHostToDevice, c.stream));
+  c.part_v.ensure((hv ? 6 : 3) * n);
+  const double *buf = stage_positions(c, pos, vel, c.part_v.p);
+  if (!buf) return fail(c, LJG_ERR_ARG, kOutsideRegion);
   hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, c.stream, (int64_t)1, c.flag.p + 2);
   LJG_HIP(hipGetLastError());
-  md_set_positions(c, buf, vel ? buf + 3 * n : nullptr);
-  int32_t mv = 0;
-  LJG_HIP(hipMemcpyAsync(&mv, c.flag.p + 2, sizeof mv, hipMemcpyDeviceToHost, c.stream));
-  LJG_HIP(hipStreamSynchronize(c.stream));
+  md_set_positions(c, buf, hv ? buf + 3 * n : nullptr);
+  unsigned long long word = 0;  // flag[2] and flag[3]
+  stream_wait(c, reinterpret_cast<const unsigned long long *>(c.flag.p + 2), 1, &word);
+  const int32_t mv = (int32_t)(uint32_t)word;
   c.have_forces = false;
   c.box_glob_valid = false;
   if (moved) *moved = mv != 0;

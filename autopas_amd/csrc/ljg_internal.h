@@ -384,8 +384,6 @@ struct Ctx {
   unsigned long long *hits_acc = nullptr;  // when set, force kernels add their pair counts here (kAccSlots lines)
   SkipIf skip{nullptr, 0};                 // force launches exit at once when skip_launch(skip)
   DevBuf<unsigned long long> hits_slots;   // the step loop's pair-count lines
-  DevBuf<double> red_out;         // [0]=e [1]=v
-  DevBuf<int64_t> red_hits;       // [0]
   DevBuf<int32_t> flag;           // [0] displacement, [1] capacity error
   int32_t *host_flag = nullptr;   // pinned, device-mapped: [0] the drift's displacement stamp
   int32_t *host_flag_dev = nullptr;  // device address of host_flag
@@ -450,8 +448,12 @@ struct Ctx {
   size_t pin_seg_cap = 0;
   int32_t *pin_flags = nullptr;
   size_t pin_flags_cap = 0;
-  double *pin_dl = nullptr;           // pinned staging of ljg_download_range
-  size_t pin_dl_cap = 0;
+  // Pinned, device-mapped staging of uploads and downloads (bytes pin_stage_cap), and a download's progress
+  // word.  stage_mark: kernels may read the staging buffer until a marker of at least this number was seen.
+  double *pin_stage = nullptr, *pin_stage_dev = nullptr;
+  size_t pin_stage_cap = 0;
+  unsigned long long *pin_progress = nullptr, *pin_progress_dev = nullptr;
+  unsigned long long progress_seq = 0, stage_mark = 0, mark_seen = 0;
   // second buffers an edit of the ensemble writes the moved layout into, then swaps in
   DevBuf<float4> pos32_alt, pos32n_alt;
   DevBuf<double4> posd_alt, posdn_alt;
@@ -536,6 +538,17 @@ void cluster_jrows_force(Ctx &c, bool globals, const IntegArgs *integ = nullptr)
 IntegArgs integ_args(Ctx &c, bool kick, bool drift, double dt, int32_t stamp);    // ljg_md.hip
 void md_kick_drift(Ctx &c, bool kick, bool drift, double dt, int32_t stamp, SkipIf skip = SkipIf{nullptr, 0});  // ljg_md.hip
 void wrap_positions(Ctx &c);               // ljg_md.hip
+// Whether all positions lie in the open box's halo region (always in other boxes), copied to dst where given.
+bool region_check(const Ctx &c, int64_t n, const double *const src[3], double *const dst[3]);  // ljg_transfer.hip
+// The caller's arrays into state buffer 0, made current (velocities if all three are given, type and id
+// optional); false, with nothing changed, when an open box's region does not hold a position.  ljg_transfer.hip
+bool upload_state(Ctx &c, int64_t n, const double *const pos[3], const double *const vel[3], const int32_t *type,
+                  const int64_t *id);
+// The caller's positions (and velocities) back to back in dev; null as above.  ljg_transfer.hip
+const double *stage_positions(Ctx &c, const double *const pos[3], const double *const vel[3], double *dev);
+// Nine arrays of `count` doubles, back to back on the device, to the caller's arrays (null: left out).
+void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs[9]);  // ljg_transfer.hip
+void release_stage(Ctx &c);  // ljg_transfer.hip
 // Rebuild permutation of the cell layout (also sets the rebuild reference positions).
 void permute_state(Ctx &c, const int32_t *src, int64_t new_slots);  // ljg_md.hip
 void reduce_partials(Ctx &c, int64_t nitems, ljg_globals *out, bool globals);  // ljg_md.hip

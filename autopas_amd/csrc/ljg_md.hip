@@ -1,8 +1,8 @@
 // ljg_md.hip -- device-wide scan, state permutation, velocity-Verlet integrator, periodic wrap and the
 // deterministic reductions of per-work-item partial sums.
-#include <cmath>
-
 #include <chrono>
+#include <cmath>
+#include <cstring>
 
 #include "ljg_internal.h"
 
@@ -379,10 +379,12 @@ void wrap_positions(Ctx &c) {
 // ---------------------------------------------------------------------------------------------------
 // Deterministic reduction of per-work-item partials: one workgroup, fixed assignment of items to
 // threads and a fixed tree, so the result does not depend on scheduling.
+// The results go to out and out_h, or (mark given) to the host behind its marker word.
 __global__ __launch_bounds__(1024) void k_reduce(int64_t n, const double *__restrict__ e,
                                                  const double *__restrict__ v, const int64_t *__restrict__ h,
                                                  double *__restrict__ out, int64_t *__restrict__ out_h,
-                                                 int32_t globals) {
+                                                 int32_t globals, unsigned long long *__restrict__ mark,
+                                                 unsigned long long seq) {
   __shared__ double se[1024], sv[1024];
   __shared__ int64_t sh[1024];
   double ae = 0., av = 0.;
@@ -406,7 +408,14 @@ __global__ __launch_bounds__(1024) void k_reduce(int64_t n, const double *__rest
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
+  if (threadIdx.x != 0) return;
+  if (mark) {
+    mark[1] = (unsigned long long)__double_as_longlong(se[0]);
+    mark[2] = (unsigned long long)__double_as_longlong(sv[0]);
+    mark[3] = (unsigned long long)sh[0];
+    __threadfence_system();
+    mark[0] = seq;
+  } else {
     out[0] = se[0];
     out[1] = sv[0];
     out_h[0] = sh[0];
@@ -534,6 +543,7 @@ void stream_spin(Ctx &c, unsigned long long seq, int n, unsigned long long *out)
     }
   }
   for (int i = 0; i < n; ++i) out[i] = m[1 + i];
+  c.mark_seen = seq;
 }
 
 unsigned long long stream_mark(Ctx &c, const unsigned long long *src, int n) {
@@ -573,21 +583,21 @@ unsigned long long count_stats_mark(Ctx &c, const int32_t *cnt, int64_t n, unsig
 
 void reduce_launch(hipStream_t st, int64_t nitems, const double *pe, const double *pv, const int64_t *ph,
                    double *out, int64_t *out_h, bool globals) {
-  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, st, nitems, pe, pv, ph, out, out_h, (int32_t)globals);
+  hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, st, nitems, pe, pv, ph, out, out_h, (int32_t)globals,
+                     (unsigned long long *)nullptr, 0ull);
   LJG_HIP(hipGetLastError());
 }
 
 void reduce_partials(Ctx &c, int64_t nitems, ljg_globals *out, bool globals) {
-  c.red_out.ensure(2);
-  c.red_hits.ensure(1);
+  const unsigned long long seq = ++c.mark_seq;
   hipLaunchKernelGGL(k_reduce, dim3(1), dim3(1024), 0, c.stream, nitems, c.part_e.p, c.part_v.p, c.part_hits.p,
-                     c.red_out.p, c.red_hits.p, (int32_t)globals);
+                     (double *)nullptr, (int64_t *)nullptr, (int32_t)globals, c.pin_mark_dev, seq);
   LJG_HIP(hipGetLastError());
-  double hv[2] = {0., 0.};
-  int64_t hh = 0;
-  LJG_HIP(hipMemcpyAsync(hv, c.red_out.p, 2 * sizeof(double), hipMemcpyDeviceToHost, c.stream));
-  LJG_HIP(hipMemcpyAsync(&hh, c.red_hits.p, sizeof(int64_t), hipMemcpyDeviceToHost, c.stream));
-  LJG_HIP(hipStreamSynchronize(c.stream));
+  unsigned long long words[3] = {0, 0, 0};
+  stream_spin(c, seq, 3, words);
+  double hv[2];
+  std::memcpy(hv, words, sizeof hv);
+  const int64_t hh = (int64_t)words[2];
   // Full lists visit each unique pair from both sides: LJFunctor::endTraversal halves the sums and
   // divides the energy by 6 (LJFunctor.h:661-685).
   out->potential_energy = hv[0] * 0.5 / 6.;
