@@ -328,7 +328,7 @@ ljg_status ljg_destroy(ljg_ctx *h) {
   c.cell_of_particle.release(); c.tower_of.release(); c.tower_count.release(); c.tower_start.release();
   c.tower_items.release(); c.tower_z.release(); c.tower_id.release(); c.ctow_count.release(); c.ctow_start.release(); c.cluster_tower.release();
   c.bbox.release(); c.c0.release(); c.list_count.release(); c.list_stats.release(); c.list.release();
-  c.pos32.release(); c.pos32_next.release(); c.posd.release(); c.posd_next.release(); c.pos32_ext.release(); c.posfx.release(); c.jcl.release(); c.jlist.release(); c.jcount.release(); c.xrow.release(); c.xcount.release(); c.xrow_tmp.release(); c.xcount_tmp.release(); c.tstats.release(); c.posfx_next.release(); c.hits_slots.release(); c.vcount.release(); c.vlist.release(); c.tab.release(); c.part_e.release(); c.part_v.release(); c.part_hits.release();
+  c.pos32.release(); c.pos32_next.release(); c.posd.release(); c.posd_next.release(); c.pos32_ext.release(); c.posfx.release(); c.boxf.release(); c.jcl.release(); c.jlist.release(); c.jcount.release(); c.xrow.release(); c.xcount.release(); c.xrow_tmp.release(); c.xcount_tmp.release(); c.tstats.release(); c.posfx_next.release(); c.hits_slots.release(); c.vcount.release(); c.vlist.release(); c.tab.release(); c.part_e.release(); c.part_v.release(); c.part_hits.release();
   c.flag.release(); c.scan_tmp.release();
   c.box_tg.release(); c.box_wrap.release(); c.box_of.release(); c.box_tbase.release(); c.tower_box.release();
   c.box_cbase.release(); c.box_pbase.release(); c.cluster_box.release();

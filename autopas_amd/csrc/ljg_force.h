@@ -13,15 +13,6 @@ struct ForceArgs {
   double eps24, sig2, shift6;  // single-type constants
 };
 
-// Workgroups are dealt to the 8 XCDs in turn.  The work of workgroup `block` of a grid of xcd_grid(n) for n
-// workgroups' worth of work: XCD k takes the k-th eighth, so that what neighbouring work shares (positions of
-// clusters side by side) meets in one L2; n or more: none.
-inline unsigned xcd_grid(int n) { return (unsigned)((n + 7) / 8 * 8); }
-__device__ inline int xcd_block(int n, unsigned block, unsigned grid) {
-  const int each = (int)(grid >> 3), k = (int)(block & 7u) * each + (int)(block >> 3);
-  return k < n ? k : n;
-}
-
 constexpr int kFThreads = 256;
 constexpr int kWavesPerBlock = kFThreads / kWave;
 

@@ -354,6 +354,7 @@ struct Ctx {
   FixGeom fg{};
   DevBuf<int4> posfx;            // per slot: fixed-point x, y, z and the type
   DevBuf<int4> posfx_next;       // the fused integrator writes the next step's fixed-point positions here
+  DevBuf<float> boxf;            // j-row builds: FP32 cluster boxes, six arrays
   DevBuf<int32_t> jcl;           // j-row build, first pass: per i-cluster row of j-cluster indices
   int32_t jccap = 0;
   DevBuf<int32_t> jlist;         // cluster layout: per i-cluster row of j slots (union of members' lists)
@@ -627,6 +628,15 @@ __host__ __device__ inline int shift_component(int sid, int d) {
 }
 
 inline int blocks_for(int64_t n, int threads) { return (int)((n + threads - 1) / threads); }
+
+// Workgroups are dealt to the 8 XCDs in turn.  The work of workgroup `block` of a grid of xcd_grid(n) for n
+// workgroups' worth of work: XCD k takes the k-th eighth, so that what neighbouring work shares (positions of
+// clusters side by side) meets in one L2; n or more: none.
+inline unsigned xcd_grid(int n) { return (unsigned)((n + 7) / 8 * 8); }
+__device__ inline int xcd_block(int n, unsigned block, unsigned grid) {
+  const int each = (int)(grid >> 3), k = (int)(block & 7u) * each + (int)(block >> 3);
+  return k < n ? k : n;
+}
 
 // The FP32 cluster kernel's two position buffers change roles (its fused integrator wrote the next step's
 // positions into the second): the FP32 and the FP64 copies always together.

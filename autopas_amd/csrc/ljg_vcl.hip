@@ -541,6 +541,9 @@ __global__ __launch_bounds__(W *kWave) void k_tower_sort_parts(
 // (lcount given) an empty cluster of a region's tail gets an empty row.  Every lane of the wavefront calls
 // this; mine: the lane holds a slot to write (uniform over a cluster).
 struct ClusterOut {
+  float *boxf;        // j-row builds: FP32 boxes from the box's corner in units of 1 / per_ilen, six arrays of ncl
+  int64_t ncl;
+  double corner[3], per_ilen;
   double *bbox;
   double4 *c0;
   int32_t *lcount;
@@ -572,6 +575,11 @@ __device__ inline float cluster_derive(int64_t s, int32_t M, bool mine, bool rea
     bb[0] = xl; bb[1] = yl; bb[2] = zl; bb[3] = xh; bb[4] = yh; bb[5] = zh;
     o.c0[c] = make_double4(cx, cy, cz, (double)nreal);
     if (o.lcount && nreal == 0) o.lcount[c] = 0;
+    if (o.boxf) {
+      const double b[6] = {xl, yl, zl, xh, yh, zh};
+#pragma unroll
+      for (int k = 0; k < 6; ++k) o.boxf[k * o.ncl + c] = (float)((b[k] - o.corner[k % 3]) * o.per_ilen);
+    }
   }
   if (!o.pos32) return 0.f;
   float4 p = make_float4(kPadPos32, kPadPos32, kPadPos32, __int_as_float(0));
@@ -806,38 +814,9 @@ __device__ inline double box_dist2(const double *a, const double *b, double shx,
 constexpr int kListThreads = 64;
 constexpr int kListLds = 128;  // j-clusters staged per chunk
 
-// JCL = true (the j-particle row build, first pass): entries are the j-cluster index only (int32), and a
-// j-cluster that passes the box test under several images (small boxes, long clusters) is listed only at
-// the first of them in traversal order, since the expansion pass tests minimum-image separations.
 constexpr int kMaxM = 8;
 
 __device__ inline int floor_div(int a, int b) { return a >= 0 ? a / b : -((-a + b - 1) / b); }
-
-// Whether the j-cluster with box bj passed the box test at a visit before (oy, ox, sz) in the traversal
-// order of k_cluster_lists_tower.  xy_repeats: the +-R tower window covers some tower twice.
-__device__ inline bool passed_earlier(const double *bi, const double *bj, const TowerGeom &g, int tx, int ty,
-                                      int oy, int ox, int sz, bool xy_repeats, double il2) {
-  const double shx = floor_div(tx + ox, g.nt[0]) * g.L[0], shy = floor_div(ty + oy, g.nt[1]) * g.L[1];
-  for (int s2 = -1; s2 < sz; ++s2)
-    if (box_dist2(bi, bj, shx, shy, s2 * g.L[2]) <= il2) return true;
-  if (!xy_repeats) return false;
-  for (int oy2 = -g.R; oy2 <= oy; ++oy2) {
-    if ((oy2 - oy) % g.nt[1] != 0) continue;
-    const int aoy = oy2 < 0 ? -oy2 : oy2;
-    const double dty = (double)(aoy - 1 > 0 ? aoy - 1 : 0) * g.side[1];
-    for (int ox2 = -g.R; ox2 <= g.R; ++ox2) {
-      if (oy2 == oy && ox2 >= ox) break;
-      if ((ox2 - ox) % g.nt[0] != 0) continue;
-      const int aox = ox2 < 0 ? -ox2 : ox2;
-      const double dtx = (double)(aox - 1 > 0 ? aox - 1 : 0) * g.side[0];
-      if (dtx * dtx + dty * dty > il2) continue;
-      const double sx2 = floor_div(tx + ox2, g.nt[0]) * g.L[0], sy2 = floor_div(ty + oy2, g.nt[1]) * g.L[1];
-      for (int s2 = -1; s2 <= 1; ++s2)
-        if (box_dist2(bi, bj, sx2, sy2, s2 * g.L[2]) <= il2) return true;
-    }
-  }
-  return false;
-}
 
 // LDS exchange among the lanes of one wavefront (the waves of a workgroup stage different towers).
 __device__ inline void wave_sync() {
@@ -846,26 +825,17 @@ __device__ inline void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// NS wavefronts per tower split the neighbour-tower visits (oy, ox) of the traversal into NS consecutive
-// ranges; wave w writes its entries for i-cluster ci into sub-row w, [ci*cap + w*cap/NS, ...), with its
-// length in count[ci*NS + w], so the sub-rows read in order give the single-wave traversal order.
-// The cluster-entry lists (JCL = false, compared entry by entry with the oracle) use NS = 1.
 // MB (an ensemble of boxes): tower t belongs to box tbox[t], whose grid is tgs[box] and whose towers
 // start at tbase[box]; the traversal inside the box is the single-box one.
-template <bool JCL, int NS, bool MB>
-__global__ __launch_bounds__(kListThreads * NS, JCL ? 4 : 1) void k_cluster_lists_tower(
+template <bool MB>
+__global__ __launch_bounds__(kListThreads) void k_cluster_lists_tower(
     int64_t ntowers, Segs sg, TowerGeom g1, const TowerGeom *__restrict__ tgs, const int64_t *__restrict__ tbase,
     const int32_t *__restrict__ tbox, const int32_t *__restrict__ box_active, const int64_t *__restrict__ cstart,
     const int32_t *__restrict__ ccount, const double *__restrict__ bbox, const double4 *__restrict__ c0,
-    int32_t cap, int32_t *__restrict__ count, int4 *__restrict__ list, int32_t *__restrict__ jcl, int32_t n3) {
-  // the j-cluster index pass (JCL) needs neither the reference points nor as deep a chunk, and the smaller
-  // LDS footprint lets more workgroups share a CU
-  constexpr int LDSN = JCL ? kListLds / 2 : kListLds;
-  __shared__ double sbw[NS][LDSN * 6];
-  __shared__ double4 scw[NS][JCL ? 1 : LDSN];
-  const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-  double *sb = sbw[wv];
-  double4 *sc = scw[wv];
+    int32_t cap, int32_t *__restrict__ count, int4 *__restrict__ list, int32_t n3) {
+  __shared__ double sb[kListLds * 6];
+  __shared__ double4 sc[kListLds];
+  const int lane = threadIdx.x;
   if ((int64_t)blockIdx.x >= ntowers) return;
   const int64_t t = seg_index(sg, blockIdx.x);
   TowerGeom g = g1;
@@ -881,14 +851,6 @@ __global__ __launch_bounds__(kListThreads * NS, JCL ? 4 : 1) void k_cluster_list
   const int64_t ib = cstart[t], ie = ib + ccount[t];
   const double il2 = g.ilen * g.ilen;
   const double zwin = g.ilen * (1.0 + 1e-9) + 1e-9;
-  const bool xy_repeats = g.nt[0] < 2 * g.R + 1 || g.nt[1] < 2 * g.R + 1;
-  // Two z images of a j-cluster can both pass the box test only if 2 ilen and the two clusters' z-extents
-  // together reach the box length: below one_image_z no earlier image needs a look (all but the longest
-  // clusters; 184 -> 151 us per pass on the 10^6-particle liquid).
-  const double one_image_z = xy_repeats ? -1. : g.L[2] - 2. * zwin - 1e-9 * g.L[2];
-  const int side = 2 * g.R + 1, nvis = side * side;
-  const int vbeg = (int)((int64_t)nvis * wv / NS), vend = (int)((int64_t)nvis * (wv + 1) / NS);
-  const int32_t subcap = cap / NS;
   for (int64_t base = ib; base < ie; base += kListThreads) {
     const int64_t ci = base + lane;
     const bool act = ci < ie;
@@ -899,102 +861,54 @@ __global__ __launch_bounds__(kListThreads * NS, JCL ? 4 : 1) void k_cluster_list
       for (int k = 0; k < 6; ++k) bi[k] = bbox[6 * ci + k];
       ai = c0[ci];
     }
-    const int64_t w0 = ci * (int64_t)cap + (int64_t)wv * subcap;
+    const int64_t w0 = ci * (int64_t)cap;
     int32_t cnt = 0;
-    // The visits with work, in order: the neighbour tower of visit v within reach and not empty.
-    auto next_visit = [&](int v0, int &vo, int &sxo, int &syo, int64_t &cbo, int64_t &ceo) {
-      for (int v = v0; v < vend; ++v) {
-        const int oy = v / side - g.R, ox = v % side - g.R;
-        const int aoy = oy < 0 ? -oy : oy;
-        const double dty = (double)(aoy - 1 > 0 ? aoy - 1 : 0) * g.side[1];
+    for (int oy = -g.R; oy <= g.R; ++oy) {
+      const int aoy = oy < 0 ? -oy : oy;
+      const double dty = (double)(aoy - 1 > 0 ? aoy - 1 : 0) * g.side[1];
+      int jy = ty + oy, sy = 0;
+      while (jy < 0) { jy += g.nt[1]; --sy; }
+      while (jy >= g.nt[1]) { jy -= g.nt[1]; ++sy; }
+      for (int ox = -g.R; ox <= g.R; ++ox) {
         const int aox = ox < 0 ? -ox : ox;
         const double dtx = (double)(aox - 1 > 0 ? aox - 1 : 0) * g.side[0];
         if (dtx * dtx + dty * dty > il2) continue;
-        int jx = tx + ox, jy = ty + oy, sx = 0, sy = 0;
+        int jx = tx + ox, sx = 0;
         while (jx < 0) { jx += g.nt[0]; --sx; }
         while (jx >= g.nt[0]) { jx -= g.nt[0]; ++sx; }
-        while (jy < 0) { jy += g.nt[1]; --sy; }
-        while (jy >= g.nt[1]) { jy -= g.nt[1]; ++sy; }
         const int64_t tj = tb + jx + (int64_t)jy * g.nt[0];
         const int64_t cb = cstart[tj], ce = cb + ccount[tj];
         if (cb == ce) continue;
-        vo = v; sxo = sx; syo = sy; cbo = cb; ceo = ce;
-        return true;
-      }
-      vo = vend;
-      return false;
-    };
-    // JCL: the boxes of the next visit's tower (one chunk) are loaded into registers while this visit runs
-    // from LDS, and stored to LDS when the next visit starts, so no visit waits for its tower's boxes
-    constexpr int kPf = JCL ? 6 * LDSN / kWave : 1;
-    double pf[kPf];
-    auto prefetch = [&](int64_t pcb, int64_t pce) {
-      const int pn = 6 * (int)(pce - pcb);
-#pragma unroll
-      for (int i = 0; i < kPf; ++i) {
-        const int k = lane + i * kWave;
-        pf[i] = k < pn ? bbox[6 * pcb + k] : 0.;
-      }
-    };
-    int v = vbeg, sx = 0, sy = 0;
-    int64_t cb = 0, ce = 0;
-    bool have = next_visit(vbeg, v, sx, sy, cb, ce);
-    if (JCL && have && ce - cb <= LDSN) prefetch(cb, ce);
-    while (have) {
-      int v2 = vend, sx2 = 0, sy2 = 0;
-      int64_t cb2 = 0, ce2 = 0;
-      const bool have2 = next_visit(v + 1, v2, sx2, sy2, cb2, ce2);
-      const bool single = ce - cb <= LDSN;
-      if (JCL && single) {
-        const int pn = 6 * (int)(ce - cb);
-        wave_sync();
-#pragma unroll
-        for (int i = 0; i < kPf; ++i) {
-          const int k = lane + i * kWave;
-          if (k < pn) sb[k] = pf[i];
-        }
-        wave_sync();
-      }
-      // (after this visit's boxes left the registers; a visit of several chunks stages its own)
-      if (JCL && have2 && ce2 - cb2 <= LDSN) prefetch(cb2, ce2);
-      const int oy = v / side - g.R, ox = v % side - g.R;
-      for (int sz = -1; sz <= 1; ++sz) {
-        const double shx = sx * g.L[0], shy = sy * g.L[1], shz = sz * g.L[2];
-        const double zmin = bi[2] - zwin - shz;  // window in the j tower's own frame
-        const double zmax = bi[5] + zwin - shz;
-        for (int64_t jb = cb; jb < ce; jb += LDSN) {
-          const int nj = (int)(ce - jb < LDSN ? ce - jb : LDSN);
-          if (!single || (!JCL && sz == -1 && jb == cb)) {
-            wave_sync();
-            for (int k = lane; k < 6 * nj; k += kWave) sb[k] = bbox[6 * jb + k];
-            if constexpr (!JCL)
+        const bool single = ce - cb <= kListLds;
+        for (int sz = -1; sz <= 1; ++sz) {
+          const double shx = sx * g.L[0], shy = sy * g.L[1], shz = sz * g.L[2];
+          const double zmin = bi[2] - zwin - shz;  // window in the j tower's own frame
+          const double zmax = bi[5] + zwin - shz;
+          for (int64_t jb = cb; jb < ce; jb += kListLds) {
+            const int nj = (int)(ce - jb < kListLds ? ce - jb : kListLds);
+            if (!single || sz == -1) {
+              wave_sync();
+              for (int k = lane; k < 6 * nj; k += kWave) sb[k] = bbox[6 * jb + k];
               for (int k = lane; k < nj; k += kWave) sc[k] = c0[jb + k];
-            wave_sync();
-          }
-          if (!act) continue;
-          // every cluster's z-range lies in [box_min, box_min + L): a window outside it finds nothing
-          if (zmax < g.box_min[2] || zmin > g.box_min[2] + g.L[2]) continue;
-          // lower bound of zhi >= zmin in the chunk
-          int lo = 0, hi = nj;
-          while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            if (sb[6 * mid + 5] < zmin) lo = mid + 1;
-            else hi = mid;
-          }
-          for (int k = lo; k < nj; ++k) {
-            const double *bj = sb + 6 * k;
-            if (bj[2] > zmax) break;
-            if (box_dist2(bi, bj, shx, shy, shz) <= il2) {
-              if constexpr (JCL) {
-                if ((bi[5] - bi[2]) + (bj[5] - bj[2]) < one_image_z ||
-                    !passed_earlier(bi, bj, g, tx, ty, oy, ox, sz, xy_repeats, il2)) {
-                  if (cnt < subcap) jcl[w0 + cnt] = (int32_t)(jb + k);
-                  ++cnt;
-                }
-              } else {
+              wave_sync();
+            }
+            if (!act) continue;
+            // every cluster's z-range lies in [box_min, box_min + L): a window outside it finds nothing
+            if (zmax < g.box_min[2] || zmin > g.box_min[2] + g.L[2]) continue;
+            // lower bound of zhi >= zmin in the chunk
+            int lo = 0, hi = nj;
+            while (lo < hi) {
+              const int mid = (lo + hi) >> 1;
+              if (sb[6 * mid + 5] < zmin) lo = mid + 1;
+              else hi = mid;
+            }
+            for (int k = lo; k < nj; ++k) {
+              const double *bj = sb + 6 * k;
+              if (bj[2] > zmax) break;
+              if (box_dist2(bi, bj, shx, shy, shz) <= il2) {
                 const int sid = (sx + 1) + 3 * (sy + 1) + 9 * (sz + 1);
                 if (n3 && !forward_entry(ci, jb + k, sid)) continue;
-                if (cnt < subcap) {
+                if (cnt < cap) {
                   const double4 b = sc[k];
                   const float dx = (float)((b.x + shx) - ai.x);
                   const float dy = (float)((b.y + shy) - ai.y);
@@ -1008,10 +922,191 @@ __global__ __launch_bounds__(kListThreads * NS, JCL ? 4 : 1) void k_cluster_list
           }
         }
       }
-      v = v2; sx = sx2; sy = sy2; cb = cb2; ce = ce2; have = have2;
+    }
+    if (act) count[ci] = cnt;
+  }
+}
+
+// First pass of the j-particle row build: the j-clusters whose bounding box comes within reach of the
+// i-cluster's, as indices, each once (at the first of its images in the traversal order oy, ox, sz, j that passes:
+// the expansion pass tests minimum-image separations).  That pass decides every particle exactly, so this
+// one may list a cluster too many: boxes are FP32, from the box's corner in units of ilen (boxf, six arrays of
+// ncl), and the reach is ilen and a margin above their rounding (jcl_geom).  Every test of a pair of boxes in one image
+// computes the same value wherever it is asked.
+// kJclSplit wavefronts per tower split the neighbour-tower visits (oy, ox) into consecutive ranges, a lane per
+// i-cluster; wavefront w writes its entries for i-cluster ci into sub-row w, [ci*cap + w*cap/NS, ...), with its
+// length in count[ci*NS + w], so the sub-rows read in order give the whole traversal's order.  Rows have a
+// fixed capacity; the length is the full one even when it exceeds it, so the host can grow it and build
+// again.  The next visit's boxes are loaded into registers while this one runs from LDS.
+// The pass is bound by LDS: with FP64 boxes in LDS as records of 48 bytes the lanes, each at its own place
+// in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 106 us, the 2.0M
+// particle slab 308 -> 170.  Workgroups are dealt so that an XCD takes neighbouring towers.
+constexpr int kJclChunk = kWave;
+
+struct JclGeom {
+  int32_t nt[2], R, xy_repeats;
+  float side[2], L[3], reach, wide, one_image_z;
+};
+
+__device__ inline float boxf_dist2(const float (&a)[6], float xl, float yl, float zl, float xh, float yh, float zh,
+                                   float shx, float shy, float shz) {
+  const float dx = fmaxf(fmaxf((a[0] - shx) - xh, xl - (a[3] - shx)), 0.f);
+  const float dy = fmaxf(fmaxf((a[1] - shy) - yh, yl - (a[4] - shy)), 0.f);
+  const float dz = fmaxf(fmaxf((a[2] - shz) - zh, zl - (a[5] - shz)), 0.f);
+  return dx * dx + dy * dy + dz * dz;
+}
+
+// Whether the j-cluster passed the box test at a visit before (oy, ox, sz) in the traversal order.
+__device__ inline bool passed_earlier(const float (&bi)[6], const float (&bj)[6], const JclGeom &g, int tx, int ty,
+                                      int oy, int ox, int sz, float r2) {
+  const float shx = (float)floor_div(tx + ox, g.nt[0]) * g.L[0], shy = (float)floor_div(ty + oy, g.nt[1]) * g.L[1];
+  for (int s2 = -1; s2 < sz; ++s2)
+    if (boxf_dist2(bi, bj[0], bj[1], bj[2], bj[3], bj[4], bj[5], shx, shy, (float)s2 * g.L[2]) <= r2) return true;
+  if (!g.xy_repeats) return false;
+  for (int oy2 = -g.R; oy2 <= oy; ++oy2) {
+    if ((oy2 - oy) % g.nt[1] != 0) continue;
+    for (int ox2 = -g.R; ox2 <= g.R; ++ox2) {
+      if (oy2 == oy && ox2 >= ox) break;
+      if ((ox2 - ox) % g.nt[0] != 0) continue;
+      const float sx2 = (float)floor_div(tx + ox2, g.nt[0]) * g.L[0];
+      const float sy2 = (float)floor_div(ty + oy2, g.nt[1]) * g.L[1];
+      for (int s2 = -1; s2 <= 1; ++s2)
+        if (boxf_dist2(bi, bj[0], bj[1], bj[2], bj[3], bj[4], bj[5], sx2, sy2, (float)s2 * g.L[2]) <= r2) return true;
+    }
+  }
+  return false;
+}
+
+__global__ __launch_bounds__(kWave *kJclSplit) void k_jcl_lists(int32_t ntowers, JclGeom g,
+                                                                const int64_t *__restrict__ cstart,
+                                                                const int32_t *__restrict__ ccount, int64_t ncl,
+                                                                const float *__restrict__ boxf, int32_t cap,
+                                                                int32_t *__restrict__ count,
+                                                                int32_t *__restrict__ jcl) {
+  constexpr int NS = kJclSplit;
+  __shared__ float s_box[NS][6][kJclChunk];
+  const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+  float(&sb)[6][kJclChunk] = s_box[wv];
+  const int t = xcd_block(ntowers, blockIdx.x, gridDim.x);
+  if (t >= ntowers) return;
+  const int tx = t % g.nt[0], ty = t / g.nt[0];
+  const int ib = (int)cstart[t], ie = ib + ccount[t];
+  const float r2 = g.reach * g.reach, w2 = g.wide * g.wide;
+  const int side = 2 * g.R + 1, nvis = side * side;
+  const int vbeg = nvis * wv / NS, vend = nvis * (wv + 1) / NS;
+  const int32_t subcap = cap / NS;
+  for (int base = ib; base < ie; base += kWave) {
+    const int ci = base + lane;
+    const bool act = ci < ie;
+    float bi[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) bi[k] = act ? boxf[k * ncl + ci] : 0.f;
+    int32_t *row = jcl + (int64_t)ci * cap + (int64_t)wv * subcap;
+    int32_t cnt = 0;
+    // the visits with work, in order: the neighbour tower of visit v within reach and not empty
+    auto next_visit = [&](int v, int &vo, int &oxo, int &oyo, int &sxo, int &syo, int &cbo, int &ceo) {
+      int oy = v / side - g.R, ox = v % side - g.R;
+      for (; v < vend; ++v, ++ox) {
+        if (ox > g.R) {
+          ox = -g.R;
+          ++oy;
+        }
+        const int aoy = oy < 0 ? -oy : oy, aox = ox < 0 ? -ox : ox;
+        const float dty = (float)(aoy > 1 ? aoy - 1 : 0) * g.side[1], dtx = (float)(aox > 1 ? aox - 1 : 0) * g.side[0];
+        if (dtx * dtx + dty * dty > w2) continue;
+        int jx = tx + ox, jy = ty + oy, sx = 0, sy = 0;
+        while (jx < 0) { jx += g.nt[0]; --sx; }
+        while (jx >= g.nt[0]) { jx -= g.nt[0]; ++sx; }
+        while (jy < 0) { jy += g.nt[1]; --sy; }
+        while (jy >= g.nt[1]) { jy -= g.nt[1]; ++sy; }
+        const int tj = jx + jy * g.nt[0];
+        const int n = ccount[tj];
+        if (n == 0) continue;
+        vo = v; oxo = ox; oyo = oy; sxo = sx; syo = sy;
+        cbo = (int)cstart[tj];
+        ceo = cbo + n;
+        return true;
+      }
+      return false;
+    };
+    float pf[6];
+    auto load_boxes = [&](int jb, int nj) {
+#pragma unroll
+      for (int k = 0; k < 6; ++k) pf[k] = lane < nj ? boxf[k * ncl + jb + lane] : 0.f;
+    };
+    auto store_boxes = [&]() {
+      wave_sync();
+#pragma unroll
+      for (int k = 0; k < 6; ++k) sb[k][lane] = pf[k];
+      wave_sync();
+    };
+    int v = vbeg, ox = 0, oy = 0, sx = 0, sy = 0, cb = 0, ce = 0;
+    bool have = next_visit(vbeg, v, ox, oy, sx, sy, cb, ce);
+    if (have) load_boxes(cb, min(ce - cb, kJclChunk));
+    while (have) {
+      int v2 = 0, ox2 = 0, oy2 = 0, sx2 = 0, sy2 = 0, cb2 = 0, ce2 = 0;
+      const bool have2 = next_visit(v + 1, v2, ox2, oy2, sx2, sy2, cb2, ce2);
+      const bool single = ce - cb <= kJclChunk;
+      store_boxes();
+      if (have2 && single) load_boxes(cb2, min(ce2 - cb2, kJclChunk));
+      const float shx = (float)sx * g.L[0], shy = (float)sy * g.L[1];
+      for (int jb = cb; jb < ce; jb += kJclChunk) {
+        const int nj = min(ce - jb, kJclChunk);
+        if (jb != cb) {  // a tower of several chunks
+          load_boxes(jb, nj);
+          store_boxes();
+        }
+        for (int sz = -1; sz <= 1; ++sz) {
+          const float shz = (float)sz * g.L[2];
+          const float zmin = (bi[2] - shz) - g.wide, zmax = (bi[5] - shz) + g.wide;  // in the j tower's own frame
+          if (!act || zmax < 0.f || zmin > g.L[2]) continue;
+          int lo = 0, hi = nj;  // the first with zhi >= zmin
+          while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (sb[5][mid] < zmin) lo = mid + 1;
+            else hi = mid;
+          }
+          for (int k = lo; k < nj; ++k) {
+            const float zl = sb[2][k], zh = sb[5][k];
+            if (zl > zmax) break;
+            const float xl = sb[0][k], yl = sb[1][k], xh = sb[3][k], yh = sb[4][k];
+            if (boxf_dist2(bi, xl, yl, zl, xh, yh, zh, shx, shy, shz) > r2) continue;
+            // Two z images of a j-cluster can both pass only if twice the reach and the two clusters' z-extents
+            // together come to the box length: below one_image_z no earlier image needs a look.
+            const float bj[6] = {xl, yl, zl, xh, yh, zh};
+            if ((bi[5] - bi[2]) + (zh - zl) >= g.one_image_z && passed_earlier(bi, bj, g, tx, ty, oy, ox, sz, r2))
+              continue;
+            if (cnt < subcap) row[cnt] = jb + k;
+            ++cnt;
+          }
+        }
+      }
+      if (have2 && !single) load_boxes(cb2, min(ce2 - cb2, kJclChunk));
+      v = v2; ox = ox2; oy = oy2; sx = sx2; sy = sy2; cb = cb2; ce = ce2; have = have2;
     }
     if (act) count[ci * NS + wv] = cnt;
   }
+}
+
+// The FP32 boxes' geometry.  Coordinates relative to the corner and shifts round at 2^-24 of at most twice the box
+// length, each a few times: a margin of 2^-19 of it covers them.  The tests
+// of whole towers and of the z window reach another margin farther, so that neither leaves out what the box test of
+// that image passes (passed_earlier asks the box test alone).
+static JclGeom jcl_geom(const TowerGeom &g) {
+  JclGeom j{};
+  const double per = 1.0 / g.ilen, L = std::fmax(g.L[0], std::fmax(g.L[1], g.L[2])) * per;
+  const double margin = std::ldexp(L, -19);
+  for (int d = 0; d < 2; ++d) {
+    j.nt[d] = g.nt[d];
+    j.side[d] = (float)(g.side[d] * per);
+  }
+  for (int d = 0; d < 3; ++d) j.L[d] = (float)(g.L[d] * per);
+  j.R = g.R;
+  j.xy_repeats = g.nt[0] < 2 * g.R + 1 || g.nt[1] < 2 * g.R + 1;
+  j.reach = (float)(1.0 + std::ldexp(1.0, -20) + margin);
+  j.wide = (float)((double)j.reach + margin);
+  j.one_image_z = j.xy_repeats ? -1.f : (float)(g.L[2] * per - 2.0 * (double)j.reach - margin);
+  return j;
 }
 
 // One neighbour-tower visit v of an i-cluster's traversal (k_cluster_lists_tower's order: oy, ox, then sz,
@@ -1243,14 +1338,16 @@ __device__ inline uint32_t abs_u32(int32_t a) { return a < 0 ? 0u - (uint32_t)a 
 
 template <int M, int NS, int G, bool STAGED>
 __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
-    int64_t nclusters, const int4 *__restrict__ posfx, const double4 *__restrict__ c0, int32_t ccap,
+    int64_t nclusters, int32_t nblocks, const int4 *__restrict__ posfx, const double4 *__restrict__ c0, int32_t ccap,
     const int32_t *__restrict__ ccount, const int32_t *__restrict__ jcl, FixGeom f, ExpandLimits lim, double ilen,
     uint32_t cut_lo, uint32_t cut_hi, int32_t cap, int32_t *__restrict__ count, int32_t *__restrict__ jrows,
     unsigned long long *__restrict__ stats) {
   constexpr int LG = kWave / G;  // lanes per i-cluster
   const int lane = threadIdx.x & (kWave - 1);
   const int grp = lane / LG, l = lane % LG;
-  int64_t ic = (int64_t)(blockIdx.x * (kExpandThreads / kWave) + threadIdx.x / kWave) * G + grp;
+  const int bid = xcd_block(nblocks, blockIdx.x, gridDim.x);
+  if (bid >= nblocks) return;
+  int64_t ic = (int64_t)(bid * (kExpandThreads / kWave) + (int)threadIdx.x / kWave) * G + grp;
   if constexpr (G == 1) ic = __builtin_amdgcn_readfirstlane((int)ic);
   const bool live = ic < nclusters;
   const int64_t icl = live ? ic : nclusters - 1;
@@ -1795,12 +1892,21 @@ void vcl_build(Ctx &c) {
   c.bbox.ensure(6 * ncl);
   c.c0.ensure(ncl);
   c.list_count.ensure(ncl * kJclSplit + 1);
-  ClusterOut out{c.bbox.p, c.c0.p, ens ? c.list_count.p : nullptr, nullptr, nullptr, nullptr, nullptr, c.pos32_ext.p};
+  ClusterOut out{};
+  out.bbox = c.bbox.p;
+  out.c0 = c.c0.p;
+  out.lcount = ens ? c.list_count.p : nullptr;
+  out.ext = c.pos32_ext.p;
   if (jrows) {
     // fixed-point positions of every slot (padding: type -1), written by the permutation
     verlet_geometry(c);
     c.posfx.ensure(new_slots);
     c.jcount.ensure(ncl + 1);
+    c.boxf.ensure(6 * ncl);
+    out.boxf = c.boxf.p;
+    out.ncl = ncl;
+    for (int d = 0; d < 3; ++d) out.corner[d] = g.box_min[d];
+    out.per_ilen = 1.0 / ilen;
   } else {
     c.pos32.ensure(new_slots);
     c.pos32_next.ensure(new_slots);
@@ -1863,10 +1969,8 @@ void vcl_build(Ctx &c) {
     if (n_towers == 0 || n_lane == 0)
       ;  // no box marked
     else if (jrows)
-      hipLaunchKernelGGL((k_cluster_lists_tower<true, kJclSplit, false>), dim3((unsigned)ntow),
-                         dim3(kListThreads * kJclSplit), 0, c.stream, ntow, none, g, no_tg, no_i64, no_i32, no_i32,
-                         c.ctow_start.p, c.ctow_count.p, c.bbox.p, c.c0.p, cap, c.list_count.p, (int4 *)nullptr,
-                         c.jcl.p, (int32_t)0);
+      hipLaunchKernelGGL(k_jcl_lists, dim3(xcd_grid((int)ntow)), dim3(kWave * kJclSplit), 0, c.stream, (int32_t)ntow,
+                         jcl_geom(g), c.ctow_start.p, c.ctow_count.p, ncl, c.boxf.p, cap, c.list_count.p, c.jcl.p);
     else if (split_lists && ens)
       hipLaunchKernelGGL((k_cluster_lists_split<true>), dim3(blocks_for(n_lane * kSplitLanes, kListSplitThreads)),
                          dim3(kListSplitThreads), 0, c.stream, n_lane, sg_clusters, g, c.box_tg.p, c.box_tbase.p,
@@ -1888,13 +1992,13 @@ void vcl_build(Ctx &c) {
                          c.cluster_tower.p, c.ctow_start.p, c.ctow_count.p, c.bbox.p, c.c0.p, cap, c.list_count.p,
                          c.list.p, n3);
     else if (ens)
-      hipLaunchKernelGGL((k_cluster_lists_tower<false, 1, true>), dim3((unsigned)n_towers), dim3(kListThreads), 0,
+      hipLaunchKernelGGL((k_cluster_lists_tower<true>), dim3((unsigned)n_towers), dim3(kListThreads), 0,
                          c.stream, n_towers, sg_towers, g, c.box_tg.p, c.box_tbase.p, c.tower_box.p, active, c.ctow_start.p, c.ctow_count.p,
-                         c.bbox.p, c.c0.p, cap, c.list_count.p, c.list.p, (int32_t *)nullptr, n3);
+                         c.bbox.p, c.c0.p, cap, c.list_count.p, c.list.p, n3);
     else
-      hipLaunchKernelGGL((k_cluster_lists_tower<false, 1, false>), dim3((unsigned)ntow), dim3(kListThreads), 0, c.stream,
+      hipLaunchKernelGGL((k_cluster_lists_tower<false>), dim3((unsigned)ntow), dim3(kListThreads), 0, c.stream,
                          ntow, none, g, no_tg, no_i64, no_i32, no_i32, c.ctow_start.p, c.ctow_count.p, c.bbox.p, c.c0.p,
-                         cap, c.list_count.p, c.list.p, (int32_t *)nullptr, n3);
+                         cap, c.list_count.p, c.list.p, n3);
     LJG_HIP(hipGetLastError());
     if (jrows) {
       // i-clusters per wavefront of the expansion pass (tuned on the 10^6-particle liquid: 4 for M >= 4)
@@ -1910,12 +2014,12 @@ void vcl_build(Ctx &c) {
   {                                                                                                               \
     const size_t lds = (size_t)(kExpandThreads / (kWave / GV)) * (size_t)cap * sizeof(int32_t);                   \
     if (lds <= 65536)                                                                                             \
-      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, true>), dim3(nb), dim3(kExpandThreads),         \
-                         (unsigned)lds, c.stream, ncl, c.posfx.p, c.c0.p, cap, c.list_count.p, c.jcl.p, c.fg,     \
+      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, true>), dim3(xcd_grid(nb)), dim3(kExpandThreads), \
+                         (unsigned)lds, c.stream, ncl, (int32_t)nb, c.posfx.p, c.c0.p, cap, c.list_count.p, c.jcl.p, c.fg,     \
                          lim, ilen, cut_lo, cut_hi, jcap, c.jcount.p, c.jlist.p, c.list_stats.p);                      \
     else                                                                                                          \
-      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, false>), dim3(nb), dim3(kExpandThreads), 0,     \
-                         c.stream, ncl, c.posfx.p, c.c0.p, cap, c.list_count.p, c.jcl.p, c.fg, lim, ilen, cut_lo,      \
+      hipLaunchKernelGGL((k_jrows_expand<MV, kJclSplit, GV, false>), dim3(xcd_grid(nb)), dim3(kExpandThreads), 0, \
+                         c.stream, ncl, (int32_t)nb, c.posfx.p, c.c0.p, cap, c.list_count.p, c.jcl.p, c.fg, lim, ilen, cut_lo,      \
                          cut_hi, jcap, c.jcount.p, c.jlist.p, c.list_stats.p);                                    \
   }
 #define LJG_EXPAND(MV, GV)                                                                                        \
