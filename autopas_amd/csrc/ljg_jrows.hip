@@ -30,26 +30,23 @@ namespace ljg {
 //    differs from the FP64 one leaves the force at rc (~0.04 epsilon/sigma) on a particle, and the two
 //    rows of a pair round r^2 differently in the FAST frame: at 10^6 particles a dozen such pairs would
 //    dominate the force error.  The band holds ~3e-5 of the candidate pairs (~1% of wave iterations).
-// The pair term's constants.  FAST: fixed-point units, the force over the distance as
-// (lj6 / r^2) (2 eps24 lj6 - eps24) with lj6 = (sigma^2 / r^2)^3.  Exact variant: r^2 is formed in a unit near
-// sigma (w2 weights the squares of the fixed-point separations), and with u = 1/r^6 the term is
-// (u / r^2) (A u - B), A = 2 eps24 sigma^12, B = eps24 sigma^6: a multiplication less, and fewer roundings.
+// The pair term's constants: fixed-point units for FAST, the caller's otherwise.  With lj6 = (sigma^2 / r^2)^3 the force
+// over the distance is (lj6 / r^2) (2 eps24 lj6 - eps24).
 struct JrowsPair {
-  float w2[3];               // exact variant: r^2 = sum of w2 d^2 over fixed-point separations d
-  float p, q, shift6;        // one type: FAST eps24 and sigma^2, otherwise A and B; the energy shift
-  uint32_t cut_lo, cut_hi;   // band around rc^2 (bits of r^2)
-  double rc2d;               // rc^2 (FP64)
-  double sig2_scale, eps_scale;  // several types: the table's sigma^2 and epsilon in the pair term's units
-  double fs[3], es;          // force and energy sums back to the caller's units
+  float eps24, sig2, shift6;  // one type
+  float sig2_scale;           // several types: the table's sigma^2 in the unit of r^2
+  uint32_t cut_lo, cut_hi;    // band around rc^2 (bits of r^2)
+  double rc2d;                // rc^2 (FP64)
+  double fs;                  // force sums back to the caller's units
 };
 
 // The FAST loop is bound by its ~170 VALU instructions per step of eight members: without any load it takes 0.9
 // of its time.  The row's slots are read two steps ahead: read with their positions they cost 7 us of waiting
 // per launch at 10^6 particles, M8 G8.
-// The exact variant rounds less (force RMS error of the four-type slab 1.6e-6 -> 1.2e-6) and is held to four
-// waves per SIMD: 2.0M
-// particles, four types, rc 3: 513 -> 447 us.  Below four i-clusters per wavefront (few clusters, bound by
-// latency) registers are not limited.
+// The exact variant is held to four waves per SIMD: 2.0M particles, four types, rc 3: 513 -> 472 us.  (A u - B) u / r^2
+// with u = 1/r^6 and constants of a unit near sigma takes two instructions less per pair, 441 us, but rounds otherwise:
+// pairs that cross rc a step earlier or later then tell two long runs apart.  Below four i-clusters per wavefront (few
+// clusters, bound by latency) registers are not limited.
 template <int M, int G, bool FAST, bool MIX, bool GLOB, bool INTEG>
 __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4) void k_force_cluster_jrows(
     int64_t nclusters, int32_t nblocks, const int4 *__restrict__ posfx, const double4 *__restrict__ c0, int32_t row,
@@ -65,10 +62,8 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
   __shared__ float s_sh[MIX && GLOB ? kMaxTypes * kMaxTypes : 1];
   if constexpr (MIX) {
     for (int k = threadIdx.x; k < ntypes * ntypes; k += kFThreads) {
-      const double e24 = tab64[3 * k] * pp.eps_scale, s2 = tab64[3 * k + 1] * pp.sig2_scale, s6 = s2 * s2 * s2;
-      if constexpr (FAST) s_ab[k] = make_float2((float)tab64[3 * k], (float)tab64[3 * k + 1] * (float)pp.sig2_scale);
-      else s_ab[k] = make_float2((float)(2.0 * e24 * s6 * s6), (float)(e24 * s6));
-      if constexpr (GLOB) s_sh[k] = (float)(tab64[3 * k + 2] * pp.eps_scale);
+      s_ab[k] = make_float2((float)tab64[3 * k], (float)tab64[3 * k + 1] * pp.sig2_scale);
+      if constexpr (GLOB) s_sh[k] = (float)tab64[3 * k + 2];
     }
     __syncthreads();
   }
@@ -83,10 +78,10 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
   const int nreal = (int)c0[icl].w;
   const int4 ref = posfx[icl * M];  // the first member is always real
   // (in vector registers: these instructions issue at half the rate with a scalar operand)
-  float w2x = pp.w2[0], w2y = pp.w2[1], w2z = pp.w2[2];
+  float scx = f.scale32[0], scy = f.scale32[1], scz = f.scale32[2];
   uint32_t cut1 = pp.cut_lo + 1u;
   asm volatile("" : "+v"(cut1));
-  if constexpr (!FAST) asm volatile("" : "+v"(w2x), "+v"(w2y), "+v"(w2z));
+  if constexpr (!FAST) asm volatile("" : "+v"(scx), "+v"(scy), "+v"(scz));
   const uint32_t in_from = 0u - pp.cut_lo, band = pp.cut_hi - pp.cut_lo;
   float xi[M], yi[M], zi[M];     // FAST: FP32 offsets from the first member
   uint32_t ux[M], uy[M], uz[M];  // exact variant: fixed-point positions
@@ -140,19 +135,18 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
         dy = yi[q] - jy;
         dz = zi[q] - jz;
       } else {
-        dx = (float)(int32_t)(ux[q] - (uint32_t)pf.x);
-        dy = (float)(int32_t)(uy[q] - (uint32_t)pf.y);
-        dz = (float)(int32_t)(uz[q] - (uint32_t)pf.z);
+        dx = (float)(int32_t)(ux[q] - (uint32_t)pf.x) * scx;
+        dy = (float)(int32_t)(uy[q] - (uint32_t)pf.y) * scy;
+        dz = (float)(int32_t)(uz[q] - (uint32_t)pf.z) * scz;
       }
     };
     auto square = [&](float dx, float dy, float dz, float far) {
       if constexpr (FAST) return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-      else
-        return __builtin_fmaf(dx * w2x, dx, __builtin_fmaf(dy * w2y, dy, __builtin_fmaf(dz * w2z, dz, far)));
+      else return __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, __builtin_fmaf(dz, dz, far)));
     };
     auto pair_term = [&](int q, float dx, float dy, float dz, float r2, bool m) {
       if constexpr (!FAST) m = m && q < nreal;
-      float p = pp.p, s = pp.q, shift6 = pp.shift6;
+      float p = pp.eps24, s = pp.sig2, shift6 = pp.shift6;
       if constexpr (MIX) {
         const float2 ps = *reinterpret_cast<const float2 *>(reinterpret_cast<const char *>(s_ab) + (ti[q] + tj));
         p = ps.x;
@@ -160,24 +154,16 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
         if constexpr (GLOB) shift6 = s_sh[(ti[q] + tj) / (int)sizeof(float2)];
       }
       const float inv = __builtin_amdgcn_rcpf(r2);
-      float fv, ev;  // force over distance, 6 x energy
-      if constexpr (FAST) {
-        const float lj2 = s * inv;
-        const float lj6 = lj2 * lj2 * lj2;
-        fv = (lj6 * inv) * __builtin_fmaf(p + p, lj6, -p);
-        ev = __builtin_fmaf(p, lj6 * lj6 - lj6, shift6);
-      } else {
-        const float u = inv * inv * inv;
-        fv = (u * inv) * __builtin_fmaf(p, u, -s);
-        ev = __builtin_fmaf(__builtin_fmaf(0.5f * p, u, -s), u, shift6);
-      }
+      const float lj2 = s * inv;
+      const float lj6 = lj2 * lj2 * lj2;
+      const float fv = (lj6 * inv) * __builtin_fmaf(p + p, lj6, -p);  // force over distance
       const float fac = m ? fv : 0.f;
       ax[q] = __builtin_fmaf(dx, fac, ax[q]);
       ay[q] = __builtin_fmaf(dy, fac, ay[q]);
       az[q] = __builtin_fmaf(dz, fac, az[q]);
       hits += (uint32_t)__popcll(__ballot(m));
       if constexpr (GLOB) {
-        ae[q] += m ? ev : 0.f;
+        ae[q] += m ? __builtin_fmaf(p, lj6 * lj6 - lj6, shift6) : 0.f;
         av[q] = __builtin_fmaf(m ? r2 : 0.f, fac, av[q]);
       }
     };
@@ -280,7 +266,7 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
   constexpr int KL = ilog2(LG), KV = ilog2(NV), K = KL < KV ? KL : KV;
   constexpr int R = NV >> K;
   const int q0 = group_value_slot<NV, LG>(l) * R;
-  const double *fs = pp.fs;
+  const double fs = FAST ? pp.fs : 1.0;
   double e_out = 0., v_out = 0.;
   if (live && (l & ((1 << (KL - K)) - 1)) == 0) {
     const int64_t s0 = icl * M;
@@ -289,15 +275,15 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
       const int q = q0 + r;
       const double val = v[r];
       if (q < M) {
-        if (!INTEG && q < nreal) fx[s0 + q] = val * fs[0];
+        if (!INTEG && q < nreal) fx[s0 + q] = val * fs;
       } else if (q < 2 * M) {
-        if (!INTEG && q - M < nreal) fy[s0 + q - M] = val * fs[1];
+        if (!INTEG && q - M < nreal) fy[s0 + q - M] = val * fs;
       } else if (q < 3 * M) {
-        if (!INTEG && q - 2 * M < nreal) fz[s0 + q - 2 * M] = val * fs[2];
+        if (!INTEG && q - 2 * M < nreal) fz[s0 + q - 2 * M] = val * fs;
       } else if (GLOB && q == 3 * M) {
-        e_out = val * pp.es;
+        e_out = val;
       } else if (GLOB && q == 3 * M + 1) {
-        v_out = val * pp.es;
+        v_out = val;
       }
     }
   }
@@ -320,7 +306,7 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
       for (int m = l; m < nreal; m += LG) {
 #pragma clang fp contract(off)
         const int64_t i = icl * M + m;
-        const double Fx = fsh[m] * fs[0], Fy = fsh[M + m] * fs[1], Fz = fsh[2 * M + m] * fs[2];
+        const double Fx = fsh[m] * fs, Fy = fsh[M + m] * fs, Fz = fsh[2 * M + m] * fs;
         const int4 pf = posfx[i];
         const int t = pf.w;
         fx[i] = Fx;
@@ -369,40 +355,13 @@ static void launch_jrows(Ctx &c, bool mix, bool glob, const ForceArgs &a, const 
   const bool fast = f.cubic && c.jrows_frame_ok;
   JrowsPair pp{};
   pp.rc2d = a.rc2;
-  if (fast) {
-    const double u2 = f.inv_scale[0] * f.inv_scale[0];  // (2^32/L)^2
-    pp.sig2_scale = u2;
-    pp.eps_scale = pp.es = 1.0;
-    pp.p = (float)a.eps24;
-    pp.q = (float)(a.sig2 * u2);
-    for (double &s : pp.fs) s = f.inv_scale[0];  // F = sum(d_u * fac_u) * (2^32 / L)
-  } else {
-    // The unit: the power of two times the first dimension's fixed-point unit nearest the geometric mean of the
-    // smallest and the largest sigma, so that A and B stay far from the ends of FP32's range.  The force sums
-    // carry fixed-point separations, so epsilon is taken down by as much.
-    double lo = c.lj.sig2[0], hi = c.lj.sig2[0];
-    for (int k = 1; k < c.lj.ntypes * c.lj.ntypes; ++k) {
-      lo = std::min(lo, c.lj.sig2[k]);
-      hi = std::max(hi, c.lj.sig2[k]);
-    }
-    const double sigma = std::sqrt(std::sqrt(lo) * std::sqrt(hi));
-    const int up = sigma > 0. && std::isfinite(sigma)
-                       ? std::min(60, std::max(0, (int)std::lround(std::log2(sigma * f.inv_scale[0]))))
-                       : 24;
-    const double unit = std::ldexp(f.scale[0], up);
-    pp.eps_scale = std::ldexp(1.0, -up);
-    pp.es = std::ldexp(1.0, up);
-    pp.sig2_scale = 1.0 / (unit * unit);
-    for (int d = 0; d < 3; ++d) {
-      pp.w2[d] = (float)((f.scale[d] / unit) * (f.scale[d] / unit));
-      pp.fs[d] = f.scale[d] / (unit * unit) * pp.es;
-    }
-    const double s2 = a.sig2 * pp.sig2_scale, s6 = s2 * s2 * s2;
-    pp.p = (float)(2.0 * a.eps24 * pp.eps_scale * s6 * s6);
-    pp.q = (float)(a.eps24 * pp.eps_scale * s6);
-  }
-  pp.shift6 = (float)(a.shift6 * pp.eps_scale);
-  const float rc2 = (float)(a.rc2 * pp.sig2_scale);
+  const double u2 = fast ? f.inv_scale[0] * f.inv_scale[0] : 1.0;  // (2^32/L)^2 in the fast variant
+  pp.sig2_scale = (float)u2;
+  pp.fs = fast ? f.inv_scale[0] : 1.0;  // F = sum(d_u * fac_u) * (2^32 / L)
+  pp.eps24 = (float)a.eps24;
+  pp.sig2 = (float)(a.sig2 * u2);
+  pp.shift6 = (float)a.shift6;
+  const float rc2 = (float)(a.rc2 * u2);
   // band around rc^2 decided in FP64, four times the FP32 error of r^2 and at least 2^-18 relative.  The
   // exact variant's r^2 is off by ~9 roundings (conversion, weight, three squares and sums: ~5e-7).
   // FAST offsets (up to 2^31 units from the first member) round by at most 64 units each, the

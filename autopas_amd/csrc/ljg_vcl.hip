@@ -939,9 +939,9 @@ __global__ __launch_bounds__(kListThreads) void k_cluster_lists_tower(
 // fixed capacity; the length is the full one even when it exceeds it, so the host can grow it and build
 // again.  The next visit's boxes are loaded into registers while this one runs from LDS.
 // The pass is bound by LDS: with FP64 boxes in LDS as records of 48 bytes the lanes, each at its own place
-// in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 106 us, the 2.0M
-// particle slab 308 -> 170.  Workgroups are dealt so that an XCD takes neighbouring towers.
-constexpr int kJclChunk = kWave;
+// in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 117 us, the 2.0M
+// particle slab 308 -> 150.  Workgroups are dealt so that an XCD takes neighbouring towers.
+constexpr int kJclChunk = 2 * kWave;
 
 struct JclGeom {
   int32_t nt[2], R, xy_repeats;
@@ -1029,15 +1029,20 @@ __global__ __launch_bounds__(kWave *kJclSplit) void k_jcl_lists(int32_t ntowers,
       }
       return false;
     };
-    float pf[6];
+    constexpr int PER = kJclChunk / kWave;
+    float pf[PER][6];
     auto load_boxes = [&](int jb, int nj) {
 #pragma unroll
-      for (int k = 0; k < 6; ++k) pf[k] = lane < nj ? boxf[k * ncl + jb + lane] : 0.f;
+      for (int h = 0; h < PER; ++h)
+#pragma unroll
+        for (int k = 0; k < 6; ++k) pf[h][k] = h * kWave + lane < nj ? boxf[k * ncl + jb + h * kWave + lane] : 0.f;
     };
     auto store_boxes = [&]() {
       wave_sync();
 #pragma unroll
-      for (int k = 0; k < 6; ++k) sb[k][lane] = pf[k];
+      for (int h = 0; h < PER; ++h)
+#pragma unroll
+        for (int k = 0; k < 6; ++k) sb[k][h * kWave + lane] = pf[h][k];
       wave_sync();
     };
     int v = vbeg, ox = 0, oy = 0, sx = 0, sy = 0, cb = 0, ce = 0;
@@ -1050,15 +1055,15 @@ __global__ __launch_bounds__(kWave *kJclSplit) void k_jcl_lists(int32_t ntowers,
       store_boxes();
       if (have2 && single) load_boxes(cb2, min(ce2 - cb2, kJclChunk));
       const float shx = (float)sx * g.L[0], shy = (float)sy * g.L[1];
-      for (int jb = cb; jb < ce; jb += kJclChunk) {
-        const int nj = min(ce - jb, kJclChunk);
-        if (jb != cb) {  // a tower of several chunks
-          load_boxes(jb, nj);
-          store_boxes();
-        }
-        for (int sz = -1; sz <= 1; ++sz) {
-          const float shz = (float)sz * g.L[2];
-          const float zmin = (bi[2] - shz) - g.wide, zmax = (bi[5] - shz) + g.wide;  // in the j tower's own frame
+      for (int sz = -1; sz <= 1; ++sz) {
+        const float shz = (float)sz * g.L[2];
+        const float zmin = (bi[2] - shz) - g.wide, zmax = (bi[5] - shz) + g.wide;  // in the j tower's own frame
+        for (int jb = cb; jb < ce; jb += kJclChunk) {
+          const int nj = min(ce - jb, kJclChunk);
+          if (!single && (jb != cb || sz != -1)) {  // a tower of several chunks (the first is in place)
+            load_boxes(jb, nj);
+            store_boxes();
+          }
           if (!act || zmax < 0.f || zmin > g.L[2]) continue;
           int lo = 0, hi = nj;  // the first with zhi >= zmin
           while (lo < hi) {
@@ -1303,19 +1308,20 @@ __global__ __launch_bounds__(kListSplitThreads) void k_cluster_lists_split(
 // frame; otherwise it uses exact per-pair differences.
 constexpr int kExpandThreads = 256;
 
-// The member test runs in FP32 in the frame of the cluster's first member: members and j enter as their
-// minimum-image fixed-point offsets from it, scaled to units of ilen once per particle, so a test is three
-// subtractions, a square and a minimum over the members.  With qmax the largest member offset, the j of a
-// pair within ilen lies within qmax + ilen, and 2 qmax + ilen < L/2 leaves such a pair no wrap-around; a
-// difference of two offsets is some image of the pair, so none is taken for near that is not.  A cluster
-// that fails that, or is longer than kExpandSpan ilen, takes the FP64 test for every pair.  Of a pair near
-// ilen each offset is rounded twice, the member's below kExpandSpan ilen and j's below (kExpandSpan + 1) ilen;
-// the difference and the scale round once: d^2 is off by at most
-// 2 sqrt(3) (2 (2 kExpandSpan + 1) + 2) 2^-24 + 3 2^-24 = 38 2^-24 relative.  Tests within 2^-17 of ilen^2
-// (cut_lo, cut_hi on the bit pattern) are decided again by the FP64 test, so the rows are its rows.
-// The pass is bound by VALU instructions; it tested every member of a non-cubic box in FP64 (2.0M
-// particles, M 8: 954 us a pass) and formed the exact integer difference per pair in cubic ones (10^6
-// particles: 237 us).  Now 610 and 188 us.
+// The member test runs in FP32 in the frame of the cluster's first member: members q and j enter as their
+// minimum-image fixed-point offsets from it, scaled to units of ilen once per particle, and
+// d^2 = |j|^2 + min over q of (|q|^2 - 2 q j): three fused multiply-adds and half a minimum per member.  With
+// qmax the largest member offset, the j of a pair within ilen lies within qmax + ilen, and 2 qmax + ilen < L/2
+// leaves such a pair no wrap-around; a difference of two offsets is some image of the pair, so none is taken for
+// near that is not.  A cluster that fails that, or is longer than kExpandSpan ilen, takes the FP64 test for every
+// pair.  Of a pair near ilen |q| is at most sqrt(3) kExpandSpan = 2.6 and |j| 3.6 (units of ilen): the offsets
+// round twice each (8 2^-24 of a component, 28 2^-24 of d^2), |q|^2 and |j|^2 three times (60 2^-24), the four sums
+// stay below 39 (156 2^-24): d^2 is off by less than 250 2^-24.  Tests within 2^-14 = 1024 2^-24 of ilen^2 (cut_lo,
+// cut_hi; one wave iteration in ~300) are decided again by the FP64 test, so the rows are its rows.
+// The pass is bound by VALU instructions (90 % of the issue slots; ~1000 candidates of a cluster, one in four
+// kept).  Every member of a non-cubic box tested in FP64: 954 us a pass for 2.0M particles, M 8; the exact integer
+// difference per pair, in cubic ones: 237 us for 10^6; three FP32 subtractions and a square per pair: 591 and 181;
+// now 613 and 178 us.  The same sums by v_mfma_f32_4x4x1, a lane's j against four members: 669 and 205.
 constexpr double kExpandSpan = 1.5;
 
 // Limits in fixed-point units, per dimension: j: L/2 - ilen; q: the largest member offset that the FP32 test
@@ -1340,7 +1346,7 @@ template <int M, int NS, int G, bool STAGED>
 __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
     int64_t nclusters, int32_t nblocks, const int4 *__restrict__ posfx, const double4 *__restrict__ c0, int32_t ccap,
     const int32_t *__restrict__ ccount, const int32_t *__restrict__ jcl, FixGeom f, ExpandLimits lim, double ilen,
-    uint32_t cut_lo, uint32_t cut_hi, int32_t cap, int32_t *__restrict__ count, int32_t *__restrict__ jrows,
+    float cut_lo, float cut_hi, int32_t cap, int32_t *__restrict__ count, int32_t *__restrict__ jrows,
     unsigned long long *__restrict__ stats) {
   constexpr int LG = kWave / G;  // lanes per i-cluster
   const int lane = threadIdx.x & (kWave - 1);
@@ -1359,7 +1365,7 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
   // frame limits for the row entries: L/2 - ilen minus the largest member offset; the FP32 test's condition
   uint32_t jlim[3];
   bool frame_bad = false, exact = false;
-  float fxi[M], fyi[M], fzi[M];  // offsets from the first member (padding: far from every j)
+  float fxi[M], fyi[M], fzi[M], sqi[M];  // -2 x offset from the first member, its square (padding: far from all)
   const float scx = (float)(f.scale[0] / ilen), scy = (float)(f.scale[1] / ilen), scz = (float)(f.scale[2] / ilen);
   {
     uint32_t qmax[3] = {0, 0, 0};
@@ -1373,9 +1379,11 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
         qmax[1] = max(qmax[1], abs_u32(oy));
         qmax[2] = max(qmax[2], abs_u32(oz));
       }
-      fxi[q] = q < nri ? (float)ox * scx : kPadPos32;
-      fyi[q] = q < nri ? (float)oy * scy : kPadPos32;
-      fzi[q] = q < nri ? (float)oz * scz : kPadPos32;
+      const float x = (float)ox * scx, y = (float)oy * scy, z = (float)oz * scz;
+      fxi[q] = -2.f * x;
+      fyi[q] = -2.f * y;
+      fzi[q] = -2.f * z;
+      sqi[q] = q < nri ? __builtin_fmaf(x, x, __builtin_fmaf(y, y, z * z)) : kPadPos32;
     }
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -1472,12 +1480,11 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
       const float jx = (float)ox * scx, jy = (float)oy * scy, jz = (float)oz * scz;
       float dmin = __builtin_inff();
 #pragma unroll
-      for (int q = 0; q < M; ++q) {
-        const float dx = fxi[q] - jx, dy = fyi[q] - jy, dz = fzi[q] - jz;
-        dmin = fminf(dmin, __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)));
-      }
-      near = __float_as_uint(dmin) < cut_lo;
-      if (exact || (!near && __float_as_uint(dmin) < cut_hi)) {
+      for (int q = 0; q < M; ++q)
+        dmin = fminf(dmin, __builtin_fmaf(fxi[q], jx, __builtin_fmaf(fyi[q], jy, __builtin_fmaf(fzi[q], jz, sqi[q]))));
+      const float d2 = dmin + __builtin_fmaf(jx, jx, __builtin_fmaf(jy, jy, jz * jz));
+      near = d2 < cut_lo;
+      if (exact || (!near && d2 < cut_hi)) {
         // rare: the FP64 test of every member, from positions read again (no integer one is kept for this)
         near = false;
         for (int q = 0; q < nri; ++q) near = near || near64(posfx[icl * M + q], xj);
@@ -2005,9 +2012,8 @@ void vcl_build(Ctx &c) {
       // (one i-cluster per wave below 2048 clusters: latency-bound small builds)
       const int eg = c.prm.build_groups > 0 ? c.prm.build_groups
                                              : (M >= 4 ? (ncl <= 2048 ? 1 : 4) : M == 2 ? 4 : 8);
-      // FP32 member test (lengths in units of ilen): a band of 128 ulps, 2^-17 below 1 and 2^-16 above
-      uint32_t cut_lo = 0, cut_hi = 0;
-      cutoff_band(1.f, std::ldexp(1.0, -16), cut_lo, cut_hi);
+      // FP32 member test: the band around ilen^2 (lengths in units of ilen)
+      const float cut_lo = 1.f - std::ldexp(1.f, -14), cut_hi = 1.f + std::ldexp(1.f, -14);
       const ExpandLimits lim = expand_limits(c.fg, ilen);
 // the staged form when the block's rows fit in 64 KiB of LDS (4 G rows of cap int32)
 #define LJG_EXPAND_LAUNCH(MV, GV)                                                                                 \

@@ -25,8 +25,19 @@ def _box(dims, density, seed, jitter):
                                                ((9, 9, 9), 0.75, 1e9)])
 def test_jrows_exact_in_any_box(oracle, M, dims, density, unit):
     # (20, 7, 7) at density 0.02: clusters longer than 1.5 (rc + skin) take the exact test
-    announce(f"j-rows exact M={M}: lattice {dims} density {density} unit {unit}")
-    n, box, x, y, z = _box(dims, density, 3, 0.2)
+    _check_jrows(oracle, M, dims, density, unit, 0.2)
+
+
+@pytest.mark.parametrize("M", [1, 2, 4, 8])
+@pytest.mark.parametrize("dims,jitter", [((9, 9, 9), 0.0), ((9, 10, 12), 0.0), ((9, 9, 9), 1e-5), ((12, 9, 9), 1e-6)])
+def test_jrows_exact_at_the_edge(oracle, M, dims, jitter):
+    # a lattice of spacing (rc + skin) / 3: six neighbours of every particle are at rc + skin, or next to it
+    _check_jrows(oracle, M, dims, (3.0 / (RC + SKIN)) ** 3, 1.0, jitter)
+
+
+def _check_jrows(oracle, M, dims, density, unit, jitter):
+    announce(f"j-rows exact M={M}: lattice {dims} density {density} unit {unit} jitter {jitter}")
+    n, box, x, y, z = _box(dims, density, 3, jitter)
     box, x, y, z = tuple(b * unit for b in box), x * unit, y * unit, z * unit
     rc, skin = RC * unit, SKIN * unit
     with ap.Engine((0.0, 0.0, 0.0), box, rc, skin, cluster_size=M) as e:
