@@ -1318,10 +1318,10 @@ constexpr int kExpandThreads = 256;
 // round twice each (8 2^-24 of a component, 28 2^-24 of d^2), |q|^2 and |j|^2 three times (60 2^-24), the four sums
 // stay below 39 (156 2^-24): d^2 is off by less than 250 2^-24.  Tests within 2^-14 = 1024 2^-24 of ilen^2 (cut_lo,
 // cut_hi; one wave iteration in ~300) are decided again by the FP64 test, so the rows are its rows.
-// The pass is bound by VALU instructions (90 % of the issue slots; ~1000 candidates of a cluster, one in four
-// kept).  Every member of a non-cubic box tested in FP64: 954 us a pass for 2.0M particles, M 8; the exact integer
+// The pass is bound by the loads of its ~1000 candidates per cluster, one in four of them kept (a fifth of the
+// requests miss L2).  Every member of a non-cubic box tested in FP64: 954 us a pass for 2.0M particles, M 8; the exact integer
 // difference per pair, in cubic ones: 237 us for 10^6; three FP32 subtractions and a square per pair: 591 and 181;
-// now 613 and 178 us.  The same sums by v_mfma_f32_4x4x1, a lane's j against four members: 669 and 205.
+// now 607 and 174 us.  The same sums by v_mfma_f32_4x4x1, a lane's j against four members: 669 and 205.
 constexpr double kExpandSpan = 1.5;
 
 // Limits in fixed-point units, per dimension: j: L/2 - ilen; q: the largest member offset that the FP32 test
@@ -1448,53 +1448,58 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
   // index clamped to the stream's last one every lane, dead groups included, loads a real slot and the
   // prefetches need no guard.
   const int klast = pre[NS] * M - 1;
-  int32_t jsn;
-  int4 xjn;
-  {
-    const uint32_t k0 = (uint32_t)(l < klast ? l : klast);
-    jsn = centry((int)(k0 / M)) * M + (int)(k0 % M);
-    xjn = posfx[jsn];
-  }
-  for (int base = 0; base < nmax; base += LG) {
-    const int32_t js = jsn;
-    const int4 xj = xjn;
-    const bool inrow = base + l < nflat;
-    {
-      const int kn = base + LG + l;
-      const uint32_t kc = (uint32_t)(kn < klast ? kn : klast);
-      jsn = centry((int)(kc / M)) * M + (int)(kc % M);
-      xjn = posfx[jsn];
-    }
-    bool near = false;
-    // the FP64 member test
-    auto near64 = [&](const int4 &pi, const int4 &pj) {
-      const double dx = (double)(int32_t)((uint32_t)pi.x - (uint32_t)pj.x) * f.scale[0];
-      const double dy = (double)(int32_t)((uint32_t)pi.y - (uint32_t)pj.y) * f.scale[1];
-      const double dz = (double)(int32_t)((uint32_t)pi.z - (uint32_t)pj.z) * f.scale[2];
-      return dx * dx + dy * dy + dz * dz <= il2;
-    };
-    if (inrow && xj.w >= 0) {  // padding slots carry type -1
-      const int32_t ox = (int32_t)((uint32_t)xj.x - (uint32_t)xi[0].x);
-      const int32_t oy = (int32_t)((uint32_t)xj.y - (uint32_t)xi[0].y);
-      const int32_t oz = (int32_t)((uint32_t)xj.z - (uint32_t)xi[0].z);
-      const float jx = (float)ox * scx, jy = (float)oy * scy, jz = (float)oz * scz;
-      float dmin = __builtin_inff();
+  // (offsets within these limits, less the rounding of a length, keep the row in the members' frame)
+  const float limx = (float)jlim[0] * scx * 0.999999f, limy = (float)jlim[1] * scy * 0.999999f;
+  const float limz = (float)jlim[2] * scz * 0.999999f;
+  auto slot_of = [&](int k) {
+    const uint32_t kc = (uint32_t)(k < klast ? k : klast);
+    return centry((int)(kc / M)) * M + (int)(kc % M);
+  };
+  // One j per lane.  Conditions are masks, with one branch for the undecided (6000 clusters 27 -> 23 us against a
+  // nested form, whose branches a build of few wavefronts waits for).
+  auto step = [&](int base, int js, const int4 &xj) {
+    const float jx = (float)(int32_t)((uint32_t)xj.x - (uint32_t)xi[0].x) * scx;
+    const float jy = (float)(int32_t)((uint32_t)xj.y - (uint32_t)xi[0].y) * scy;
+    const float jz = (float)(int32_t)((uint32_t)xj.z - (uint32_t)xi[0].z) * scz;
+    float dmin = __builtin_inff();
 #pragma unroll
-      for (int q = 0; q < M; ++q)
-        dmin = fminf(dmin, __builtin_fmaf(fxi[q], jx, __builtin_fmaf(fyi[q], jy, __builtin_fmaf(fzi[q], jz, sqi[q]))));
-      const float d2 = dmin + __builtin_fmaf(jx, jx, __builtin_fmaf(jy, jy, jz * jz));
-      near = d2 < cut_lo;
-      if (exact || (!near && d2 < cut_hi)) {
-        // rare: the FP64 test of every member, from positions read again (no integer one is kept for this)
+    for (int q = 0; q < M; ++q)
+      dmin = fminf(dmin, __builtin_fmaf(fxi[q], jx, __builtin_fmaf(fyi[q], jy, __builtin_fmaf(fzi[q], jz, sqi[q]))));
+    const float d2 = dmin + __builtin_fmaf(jx, jx, __builtin_fmaf(jy, jy, jz * jz));
+    const bool inrow = (base + l < nflat) & (xj.w >= 0);  // padding slots carry type -1
+    bool near = inrow & (d2 < cut_lo);
+    const bool undecided = inrow & (exact | ((d2 < cut_hi) & !near));
+    if (__builtin_amdgcn_ballot_w64(undecided) != 0ull) {
+      // rare: the FP64 test of every member, from positions read again (no integer one is kept for this)
+      if (undecided) {
         near = false;
-        for (int q = 0; q < nri; ++q) near = near || near64(posfx[icl * M + q], xj);
+        for (int q = 0; q < nri; ++q) {
+          const int4 pi = posfx[icl * M + q];
+          const double dx = (double)(int32_t)((uint32_t)pi.x - (uint32_t)xj.x) * f.scale[0];
+          const double dy = (double)(int32_t)((uint32_t)pi.y - (uint32_t)xj.y) * f.scale[1];
+          const double dz = (double)(int32_t)((uint32_t)pi.z - (uint32_t)xj.z) * f.scale[2];
+          near = near | (dx * dx + dy * dy + dz * dz <= il2);
+        }
       }
-      if (near) frame_bad = frame_bad || abs_u32(ox) > jlim[0] || abs_u32(oy) > jlim[1] || abs_u32(oz) > jlim[2];
     }
-    const unsigned long long ball = __ballot(near) & gmask;
-    const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(ball >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ball, 0u));
-    if (near && cnt + below < cap) jrow[cnt + below] = js;
+    frame_bad = frame_bad | (near & ((fabsf(jx) > limx) | (fabsf(jy) > limy) | (fabsf(jz) > limz)));
+    const unsigned long long ball = __builtin_amdgcn_ballot_w64(near) & gmask;
+    const int at = cnt + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(ball >> 32),
+                                                        __builtin_amdgcn_mbcnt_lo((uint32_t)ball, 0u));
+    if (near & (at < cap)) jrow[at] = js;
     cnt += __popcll(ball);
+  };
+  // two steps per trip, each one's positions loaded during the other's (they stay in their registers)
+  int ja = slot_of(l);
+  int4 xa = posfx[ja];
+  for (int base = 0; base < nmax; base += 2 * LG) {
+    const int jb = slot_of(base + LG + l);
+    const int4 xb = posfx[jb];
+    step(base, ja, xa);
+    if (base + LG >= nmax) break;
+    ja = slot_of(base + 2 * LG + l);
+    xa = posfx[ja];
+    step(base + LG, jb, xb);
   }
   if (live && l == 0) count[ic] = cnt;
   if (__ballot(frame_bad) != 0ull && lane == 0) stats[2] = 1ull;  // every writer stores the same value
