@@ -19,28 +19,48 @@ constexpr int kWavesPerBlock = kFThreads / kWave;
 // ---- block-level deterministic partials ------------------------------------------------------------
 // Per-block partial sums (fixed tree, so reproducible); the block's pair count is also added to acc's
 // per-XCD lines when acc is set (integer addition, so the order of the atomics does not matter).
-// They go to entry bid.
+// They go to entry bid.  Without globals only the count is summed, by the wavefronts first: the tree's eight
+// barriers are a tenth of a small launch.
+template <bool GLOB>
 __device__ inline void block_partials(double e, double v, int64_t h, double *pe, double *pv, int64_t *ph,
-                                      bool globals, unsigned long long *acc, int bid) {
-  __shared__ double se[kFThreads], sv[kFThreads];
-  __shared__ int64_t sh[kFThreads];
-  se[threadIdx.x] = globals ? e : 0.;
-  sv[threadIdx.x] = globals ? v : 0.;
-  sh[threadIdx.x] = h;
-  __syncthreads();
-  for (int s = kFThreads / 2; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) {
-      se[threadIdx.x] += se[threadIdx.x + s];
-      sv[threadIdx.x] += sv[threadIdx.x + s];
-      sh[threadIdx.x] += sh[threadIdx.x + s];
-    }
+                                      unsigned long long *acc, int bid) {
+  if constexpr (GLOB) {
+    __shared__ double se[kFThreads], sv[kFThreads];
+    __shared__ int64_t sh[kFThreads];
+    se[threadIdx.x] = e;
+    sv[threadIdx.x] = v;
+    sh[threadIdx.x] = h;
     __syncthreads();
-  }
-  if (threadIdx.x == 0) {
-    pe[bid] = se[0];
-    pv[bid] = sv[0];
-    ph[bid] = sh[0];
-    if (acc) acc_add(acc, (unsigned long long)sh[0]);
+    for (int s = kFThreads / 2; s > 0; s >>= 1) {
+      if ((int)threadIdx.x < s) {
+        se[threadIdx.x] += se[threadIdx.x + s];
+        sv[threadIdx.x] += sv[threadIdx.x + s];
+        sh[threadIdx.x] += sh[threadIdx.x + s];
+      }
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+      pe[bid] = se[0];
+      pv[bid] = sv[0];
+      ph[bid] = sh[0];
+      if (acc) acc_add(acc, (unsigned long long)sh[0]);
+    }
+  } else {
+    __shared__ int32_t sw[kWavesPerBlock];
+    int32_t w = (int32_t)h;  // (a block's pairs number far below 2^31)
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) w += __shfl_xor(w, off, kWave);
+    if ((threadIdx.x & (kWave - 1)) == 0) sw[threadIdx.x / kWave] = w;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      int64_t t = 0;
+#pragma unroll
+      for (int k = 0; k < kWavesPerBlock; ++k) t += sw[k];
+      pe[bid] = 0.;
+      pv[bid] = 0.;
+      ph[bid] = t;
+      if (acc) acc_add(acc, (unsigned long long)t);
+    }
   }
 }
 

@@ -60,7 +60,11 @@ struct MixedBand {
 // xrow[ic * xstride]: the listed j-cluster members within rc + skin of one of its members) instead of
 // every member of every listed entry; the element gives the j slot and its entry directly, so their two
 // loads are issued together one iteration ahead.
-template <int M, int G, bool MIX, bool GLOB, bool INTEG, bool N3, bool XR>
+// S (fused member-row launches): a group of lanes takes M / S of its i-cluster's members, and S groups the cluster.  A
+// launch that leaves the SIMDs a wavefront or two each waits for every instruction and load of one wavefront's walk; S
+// times the wavefronts walk the same rows with 1 / S of the pair terms, the same lanes adding the same j in the same
+// order, so the forces are the same to the bit.  30,011 particles, M8 G4: 15.4 -> 12.8 us per launch.
+template <int MC, int G, bool MIX, bool GLOB, bool INTEG, bool N3, bool XR, int S>
 __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_force_cluster_mixed(
     int64_t nclusters, Segs sg, const float4 *__restrict__ pos32, int32_t row, const int32_t *__restrict__ lcount,
     const int4 *__restrict__ list, const int32_t *__restrict__ xcount, const int2 *__restrict__ xrow,
@@ -70,8 +74,10 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
     SkipIf sk, double *__restrict__ clg, IntegArgs ia, MixedBand bd, Owned own, WorkQueue wq) {
   static_assert(!(N3 && INTEG), "the fused update needs every pair's force first");
   static_assert(!(N3 && XR), "Newton-3 lists stream whole entries");
-  if (skip_launch(sk)) return;
+  static_assert(S == 1 || (XR && INTEG), "only fused member-row launches are split");
+  constexpr int M = MC / S;  // this group's members
   constexpr int LG = kWave / G;
+  if (skip_launch(sk)) return;
   constexpr int NVAL = 3 * M + 1 + (GLOB ? 2 : 0);
   constexpr int NV = pow2_at_least(NVAL);
   constexpr float kW = N3 ? 2.f : 1.f;  // weight of a hit in the pair count, energy and virial sums
@@ -126,15 +132,20 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
       break;
     }
     const int item = tile * G + grp;
-    int ic = item < nclusters ? (int)seg_index(sg, item) : -1;
-    if constexpr (G == 1) ic = __builtin_amdgcn_readfirstlane(ic);
+    int ic = item < nclusters * S ? (int)seg_index(sg, item / S) : -1;
+    int part = S > 1 ? item % S * M : 0;
+    if constexpr (G == 1) {
+      ic = __builtin_amdgcn_readfirstlane(ic);
+      part = __builtin_amdgcn_readfirstlane(part);
+    }
+    const int64_t m0 = (int64_t)ic * MC + part;  // the slot of the group's first member
     if (!wq.ctr) ++tile;
   if (ic >= 0) {
     float xi[M], yi[M], zi[M];
     int ti[M];
 #pragma unroll
     for (int q = 0; q < M; ++q) {
-      const float4 p = pos32[(int64_t)ic * M + q];
+      const float4 p = pos32[m0 + q];
       const bool pad = p.x == kPadPos32;
       xi[q] = pad ? -kPadPos32 : p.x;
       yi[q] = pad ? -kPadPos32 : p.y;
@@ -151,7 +162,7 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
     const int64_t beg = (int64_t)ic * row;
     const int2 *xr = XR ? xrow + (int64_t)ic * xstride : nullptr;
     // >= M without member rows: every list holds its own cluster (a member row at least its real members)
-    const int nj = XR ? xcount[ic] : lcount[ic] * M;
+    const int nj = XR ? xcount[ic] : lcount[ic] * MC;
     // prefetch the first j of this lane (an empty list skips the loop and never loads), and with member
     // rows the element of the next one
     const int kk = l < nj ? l : nj - 1;
@@ -165,8 +176,8 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
         p = pos32[x0.x];
         xq = xr[l + LG < nj ? l + LG : nj - 1];
       } else {
-        e = list[beg + (uint32_t)kk / M];
-        p = pos32[(int64_t)(e.x & kClusterMask) * M + (kk & (M - 1))];
+        e = list[beg + (uint32_t)kk / MC];
+        p = pos32[(int64_t)(e.x & kClusterMask) * MC + (kk & (MC - 1))];
       }
     }
     for (int base = 0; base < nj; base += LG) {
@@ -178,10 +189,10 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
       // Newton-3: this lane's j slot, and whether its entry is the cluster's own (member pairs b > q only)
       int64_t sj_n3 = 0;
       bool own_n3 = false;
-      const int bm = (base + l) & (M - 1);
+      const int bm = (base + l) & (MC - 1);
       if constexpr (N3) {
         const int jc = e.x & kClusterMask;
-        sj_n3 = (int64_t)jc * M + bm;
+        sj_n3 = (int64_t)jc * MC + bm;
         own_n3 = jc == ic && ((uint32_t)e.x >> kShiftBits) == 13u;
       }
       float fjx = 0.f, fjy = 0.f, fjz = 0.f;  // Newton-3: the reaction on j, summed over the i-members
@@ -194,8 +205,8 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
       } else {
         const int kn = base + LG + l;
         const int kc = kn < nj ? kn : nj - 1;
-        e = list[beg + (uint32_t)kc / M];
-        p = pos32[(int64_t)(e.x & kClusterMask) * M + (kc & (M - 1))];
+        e = list[beg + (uint32_t)kc / MC];
+        p = pos32[(int64_t)(e.x & kClusterMask) * MC + (kc & (MC - 1))];
       }
       auto pair_term = [&](int q, float dx, float dy, float dz, float r2, bool m) {
         float eps24 = eps24_1, sig2 = sig2_1, shift6 = shift6_1;
@@ -249,8 +260,8 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
           ec = list[beg + xc.y];
           sj = xc.x;
         } else {
-          ec = list[beg + (uint32_t)kc / M];
-          sj = (int64_t)(ec.x & kClusterMask) * M + (kc & (M - 1));
+          ec = list[beg + (uint32_t)kc / MC];
+          sj = (int64_t)(ec.x & kClusterMask) * MC + (kc & (MC - 1));
         }
         const int sid = (int)((uint32_t)ec.x >> kShiftBits);
         // the box lengths are read here, not held through the loop (six registers the common path needs)
@@ -273,7 +284,7 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
           if (__ballot(inband) == 0ull) continue;
           int32_t qq = q;
           asm volatile("" : "+v"(qq));
-          const double4 pi = bd.posd[(int64_t)ic * M + qq];
+          const double4 pi = bd.posd[m0 + qq];
           const double drx = pi.x - xjd, dry = pi.y - yjd, drz = pi.z - zjd;
           const double dr2 = drx * drx + dry * dry + drz * drz;
           if (inband && dr2 <= bd.rc2 && dr2 > 0.) inside |= 1u << q;
@@ -313,7 +324,7 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
       double se = 0., sv = 0.;
 #pragma unroll
       for (int q = 0; q < M; ++q)
-        if (is_owned(own, (int64_t)ic * M + q)) { se += (double)ae[q]; sv += (double)av[q]; }
+        if (is_owned(own, m0 + q)) { se += (double)ae[q]; sv += (double)av[q]; }
       v[3 * M + 1] = se;
       v[3 * M + 2] = sv;
     }
@@ -322,7 +333,7 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
     constexpr int R = NV >> K;
     const int q0 = group_value_slot<NV, LG>(l) * R;
     if ((l & ((1 << (KL - K)) - 1)) == 0) {
-      const int64_t s0 = (int64_t)ic * M;
+      const int64_t s0 = m0;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         const int q = q0 + r;
@@ -364,7 +375,7 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
       for (int m = l; m < M; m += LG) {
 #pragma clang fp contract(off)
         if (!((real >> m) & 1u)) continue;
-        const int64_t i = (int64_t)ic * M + m;
+        const int64_t i = m0 + m;
         const double Fx = fsh[m], Fy = fsh[M + m], Fz = fsh[2 * M + m];
         const int t = __float_as_int(pos32[i].w);
         fx[i] = Fx;
@@ -390,7 +401,7 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
           if (ex * ex + ey * ey + ez * ez >= ia.half_skin2) {
             ia.flag[0] = ia.stamp;
             ia.hflag[0] = ia.stamp;
-            if (ia.box_flag) ia.box_flag[ia.cluster_box[i / M]] = 1;
+            if (ia.box_flag) ia.box_flag[ia.cluster_box[i / MC]] = 1;
           }
           ia.pos32_next[i] = make_float4((float)(x - cc.x), (float)(y - cc.y), (float)(z - cc.z), __int_as_float(t));
           ia.posd_next[i] = make_double4(x, y, z, 0.);
@@ -412,7 +423,7 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
       __threadfence();
     }
   }
-  block_partials(e_out, v_out, h_out, pe, pv, ph, GLOB, acc, (int)blockIdx.x);
+  block_partials<GLOB>(e_out, v_out, h_out, pe, pv, ph, acc, (int)blockIdx.x);
 }
 
 // FP64 cluster kernel: same tiles (one i-cluster per wave), absolute FP64 positions with the periodic
@@ -541,7 +552,7 @@ __global__ __launch_bounds__(kFThreads) void k_force_cluster_fp64(
       }
     }
   }
-  block_partials(e_out, v_out, h_out, pe, pv, ph, GLOB, acc, (int)blockIdx.x);
+  block_partials<GLOB>(e_out, v_out, h_out, pe, pv, ph, acc, (int)blockIdx.x);
 }
 
 __global__ void k_zero_forces(int64_t n, double *__restrict__ fx, double *__restrict__ fy, double *__restrict__ fz,
@@ -555,6 +566,18 @@ __global__ void k_zero_forces(int64_t n, double *__restrict__ fx, double *__rest
   }
 }
 
+// Groups that share a cluster's members in a fused member-row launch of `blocks` workgroups unsplit (256 are a wavefront
+// per SIMD): four or two while that makes no more than two to three wavefronts per SIMD, us per launch unsplit / 2 / 4 / 8:
+// 22 workgroups (700 particles, M8 G1) 9.5 / - / 7.25 / 7.3, 235 (30,011, M8 G4) 15.4 / 12.8 / 14.4 / -.
+static int member_split(int M, int blocks) {
+  if (M == 8) return blocks <= 128 ? 4 : blocks <= 384 ? 2 : 1;
+  return M == 4 && blocks <= 256 ? 2 : 1;
+}
+template <int G>
+static int plain_blocks(int64_t items) {
+  return blocks_for(items, kWavesPerBlock * G);
+}
+
 template <int M, int G>
 static void launch_mixed(Ctx &c, bool mix, bool glob, const ForceArgs &a, const double *tab, const IntegArgs *integ,
                          const ClusterSubset *sub, bool n3) {
@@ -562,7 +585,8 @@ static void launch_mixed(Ctx &c, bool mix, bool glob, const ForceArgs &a, const 
   const Segs sg = sub ? sub->segs : Segs{nullptr, nullptr, 0};
   const int64_t items = sub ? sub->nitems : c.nclusters;
   if (items == 0) return;
-  const int nb = blocks_for(items, per_block);
+  const int split = integ && c.xrows_valid && !n3 && !glob ? member_split(M, plain_blocks<G>(items)) : 1;
+  const int nb = blocks_for(items * split, per_block);
   // a subset launch writes its block partials after part_offset (reserved beforehand: launches of two
   // subsets may run at once)
   const int64_t off = sub ? sub->part_offset : 0;
@@ -613,8 +637,9 @@ static void launch_mixed(Ctx &c, bool mix, bool glob, const ForceArgs &a, const 
     launch_blocks = persist_blocks;
     c.part_items = launch_blocks;  // the block partials written
   }
-#define LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, XRV)                                                                     \
-  hipLaunchKernelGGL((k_force_cluster_mixed<M, G, MIXV, GLOBV, INTV, N3V, XRV>), dim3(launch_blocks), dim3(kFThreads), \
+#define LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, XRV, SV)                                                                 \
+  hipLaunchKernelGGL((k_force_cluster_mixed<M, G, MIXV, GLOBV, INTV, N3V, XRV, SV>),                                 \
+                     dim3(SV > 1 ? blocks_for(items * SV, per_block) : launch_blocks), dim3(kFThreads),              \
                      0, c.stream, items, sg, c.pos32.p, c.list_row, c.list_count.p, c.list.p, c.xcount.p, c.xrow.p,  \
                      c.xstride, rc2, (float)a.eps24, (float)a.sig2, (float)a.shift6, a.ntypes, tab,                  \
                      c.st[c.cur].fx.p, c.st[c.cur].fy.p, c.st[c.cur].fz.p, c.part_e.p + off, c.part_v.p + off,       \
@@ -622,11 +647,11 @@ static void launch_mixed(Ctx &c, bool mix, bool glob, const ForceArgs &a, const 
 #define LJG_LAUNCH(MIXV, GLOBV, INTV, N3V)                                                                         \
   do {                                                                                                             \
     if constexpr (N3V) {                                                                                           \
-      LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, false);                                                                  \
+      LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, false, 1);                                                               \
     } else if (xr) {                                                                                               \
-      LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, true);                                                                   \
+      LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, true, 1);                                                                \
     } else {                                                                                                       \
-      LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, false);                                                                  \
+      LJG_LAUNCH1(MIXV, GLOBV, INTV, N3V, false, 1);                                                               \
     }                                                                                                              \
   } while (0)
   if (n3) {
@@ -637,6 +662,17 @@ static void launch_mixed(Ctx &c, bool mix, bool glob, const ForceArgs &a, const 
       if (glob) LJG_LAUNCH(true, true, false, true); else LJG_LAUNCH(true, false, false, true);
     } else {
       if (glob) LJG_LAUNCH(false, true, false, true); else LJG_LAUNCH(false, false, false, true);
+    }
+  } else if (integ && xr && split > 1) {
+    if constexpr (M == 8) {
+      if (split == 4) {
+        if (mix) LJG_LAUNCH1(true, false, true, false, true, 4); else LJG_LAUNCH1(false, false, true, false, true, 4);
+      }
+    }
+    if constexpr (M >= 4) {
+      if (split == 2) {
+        if (mix) LJG_LAUNCH1(true, false, true, false, true, 2); else LJG_LAUNCH1(false, false, true, false, true, 2);
+      }
     }
   } else if (integ) {
     if (mix) LJG_LAUNCH(true, false, true, false); else LJG_LAUNCH(false, false, true, false);
@@ -681,9 +717,11 @@ static void launch_fp64(Ctx &c, bool mix, bool glob, const ForceArgs &a, const d
 // i-clusters per wave for the FP32 kernel: the tuned default per cluster size, or the caller's choice.
 int default_groups(int M) { return M >= 8 ? 1 : M == 4 ? 2 : M == 2 ? 4 : 16; }
 
+// (an upper bound: whether the launch is split also depends on its options)
 int64_t cluster_force_blocks(const Ctx &c, int64_t nitems) {
   const int G = c.prm.tile_groups > 0 ? c.prm.tile_groups : default_groups(c.M);
-  return blocks_for(nitems, kWavesPerBlock * G);
+  const int split = member_split(c.M, blocks_for(nitems, kWavesPerBlock * G));
+  return blocks_for(nitems * split, kWavesPerBlock * G);
 }
 
 void cluster_force(Ctx &c, bool mixed, bool globals, const IntegArgs *integ, const ClusterSubset *sub, bool n3) {

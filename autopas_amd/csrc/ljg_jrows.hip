@@ -340,7 +340,7 @@ __global__ __launch_bounds__(kFThreads, GLOB || G < 4 ? 1 : FAST && !MIX ? 5 : 4
       }
     }
   }
-  block_partials(e_out, v_out, lane == 0 ? (int64_t)hits : 0, pe, pv, ph, GLOB, acc, bid);
+  block_partials<GLOB>(e_out, v_out, lane == 0 ? (int64_t)hits : 0, pe, pv, ph, acc, bid);
 }
 
 template <int M, int G>
