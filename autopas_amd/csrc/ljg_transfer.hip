@@ -11,7 +11,6 @@
 #include <cstring>
 #include <memory>
 #include <thread>
-#include <vector>
 
 #include "ljg_internal.h"
 
@@ -247,16 +246,18 @@ const double *stage_positions(Ctx &c, const double *const pos[3], const double *
 // The copy out of a download: `total` doubles on the device, nine arrays of `count` back to back (null outputs
 // are left out), as chunks through the ring.  Chunk k occupies ring slot k mod slots; it is queued once chunk
 // k - slots has been copied out, and is complete when the progress word passes it.  This thread queues the
-// chunks; all threads take chunks in order and copy them out.
+// chunks; all threads take chunks in order and copy them out.  The helpers are not joined but share this object: one
+// that the scheduler lets start late (the caller's own worker threads may be spinning on every core: 2 to 3 ms were
+// seen) finds no chunk left and ends without touching the buffers, and only chunks that were taken are waited for.
 namespace {
 struct Download {
   const double *ring;
   size_t count, chunk, total;
   int nchunks, slots;
-  double *const *outs;
+  double *outs[9];
   volatile unsigned long long *progress;
   unsigned long long base;  // progress holds base + the number of complete chunks
-  std::unique_ptr<std::atomic<char>[]> done;
+  std::unique_ptr<std::atomic<char>[]> done;  // 1: copied out, 2: given up
   std::atomic<int> next{0};
   std::atomic<bool> abort{false};
 
@@ -280,7 +281,10 @@ struct Download {
       const int k = next.fetch_add(1);
       if (k >= nchunks) return;
       for (unsigned spins = 0; !ready(k); ++spins) {
-        if (abort.load(std::memory_order_relaxed)) return;
+        if (abort.load(std::memory_order_relaxed)) {
+          done[k].store(2, std::memory_order_release);
+          return;
+        }
         if (spins > 64) std::this_thread::yield();
       }
       copy_out(k);
@@ -290,14 +294,14 @@ struct Download {
 }  // namespace
 
 // Chunks of an eighth (at least 256 KiB, where a chunk's transfer takes as long as its launch; at most 2 MiB), and
-// from 8 MiB on three helpers: one thread copies about 30 GB/s, the link carries 55.  A thread costs ~20 us
-// to start.  Downloads of 63, 72 and 144 MB: 3.50, 3.74 and 7.36 -> 1.42, 1.55 and 2.95 ms.
+// from 24 MiB on three helpers: one thread copies about 30 GB/s, the link carries 55.  Downloads of 63, 72 and 144 MB: 3.50, 3.74 and 7.36 -> 1.42, 1.55 and 2.95 ms.
 constexpr size_t kMinChunk = (256u << 10) / sizeof(double), kMaxChunk = (2u << 20) / sizeof(double);
-constexpr size_t kHelpedBytes = 8u << 20;
+constexpr size_t kHelpedBytes = 24u << 20;
 constexpr int kHelpers = 3;
 
 void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs[9]) {
-  Download d;
+  const std::shared_ptr<Download> shared = std::make_shared<Download>();
+  Download &d = *shared;
   d.count = count;
   d.total = 9 * count;
   d.chunk = (d.total + 7) / 8;
@@ -307,13 +311,14 @@ void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs
   d.ring = stage_buffer(c, bytes < kRingBytes ? bytes : kRingBytes);
   d.slots = (int)(c.pin_stage_cap / (d.chunk * sizeof(double)));
   d.slots = d.slots < 1 ? 1 : d.slots;  // (a single chunk shorter than kMinChunk)
-  d.outs = outs;
+  std::copy(outs, outs + 9, d.outs);
   d.progress = c.pin_progress;
   d.base = c.progress_seq;
   c.progress_seq += (unsigned long long)d.nchunks + 1;
   d.done.reset(new std::atomic<char>[(size_t)d.nchunks]);
   for (int k = 0; k < d.nchunks; ++k) d.done[k].store(0, std::memory_order_relaxed);
   int queued = 0;  // chunks queued, nchunks + 1 once the last progress write is
+  int mine = -1;   // the chunk this thread has taken last
   auto pump = [&]() {
     while (queued <= d.nchunks &&
            (queued == d.nchunks || queued < d.slots || d.done[queued - d.slots].load(std::memory_order_acquire))) {
@@ -323,30 +328,25 @@ void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs
       ++queued;
     }
   };
-  std::vector<std::thread> threads;
-  auto join = [&]() {
-    for (auto &t : threads) t.join();
-    threads.clear();
-  };
   try {
     pump();
     if (d.total * sizeof(double) >= kHelpedBytes) {
-      threads.reserve(kHelpers);
       for (int k = 0; k < kHelpers; ++k) {
         try {
-          threads.emplace_back([&d]() { d.help(); });
+          std::thread([shared]() { shared->help(); }).detach();
         } catch (const std::exception &) {
           break;  // no more threads to be had: this one copies the rest
         }
       }
     }
     auto t0 = std::chrono::steady_clock::now();
-    auto wait_for = [&](auto &&met) {
+    // (device: only the device is waited for, which a synchronisation of the stream completes)
+    auto wait_for = [&](bool device, auto &&met) {
       for (uint64_t spins = 0; !met(); ++spins) {
         pump();
         if ((spins & 1023) == 1023 && std::chrono::steady_clock::now() - t0 > std::chrono::seconds(2)) {
           LJG_HIP(hipStreamSynchronize(c.stream));  // reports any error
-          if (queued > d.nchunks && !met()) throw HipError{hipErrorUnknown, "download not completed", __LINE__};
+          if (device && queued > d.nchunks && !met()) throw HipError{hipErrorUnknown, "download not completed", __LINE__};
           t0 = std::chrono::steady_clock::now();
         }
       }
@@ -354,17 +354,22 @@ void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs
     for (;;) {
       const int k = d.next.fetch_add(1);
       if (k >= d.nchunks) break;
-      wait_for([&]() { return d.ready(k); });
+      mine = k;
+      wait_for(true, [&]() { return d.ready(k); });
       d.copy_out(k);
     }
-    // the helpers' last chunks may wait for chunks that are not queued yet
-    wait_for([&]() { return queued > d.nchunks; });
+    // every chunk is taken: the helpers finish theirs (which may wait for some that are not queued yet)
+    for (int k = 0; k < d.nchunks; ++k)
+      wait_for(false, [&]() { return d.done[k].load(std::memory_order_acquire) != 0; });
+    wait_for(false, [&]() { return queued > d.nchunks; });
   } catch (...) {
+    // no chunk is taken from here on; those taken end with the abort or with their copy
+    const int taken = std::min(d.next.exchange(d.nchunks), d.nchunks);
     d.abort.store(true);
-    join();
+    for (int k = 0; k < taken; ++k)
+      while (d.done[k].load(std::memory_order_acquire) == 0 && k != mine) std::this_thread::yield();
     throw;
   }
-  join();
 }
 
 }  // namespace ljg

@@ -15,8 +15,8 @@ def _arrays(n, seed, L):
     return [rng.uniform(0.0, L, n) for _ in range(3)] + [rng.standard_normal(n) for _ in range(6)]
 
 
-# one chunk; chunks of 256 KiB; an upload's 4 MiB; helpers from 8 MiB; the ring wraps above 16 MiB
-@pytest.mark.parametrize("n", [1, 2, 3640, 3641, 3643, 29129, 87381, 87382, 116508, 116509, 233017, 500001])
+# one chunk; chunks of 256 KiB; an upload's 4 MiB; the ring wraps above 16 MiB; helpers from 24 MiB
+@pytest.mark.parametrize("n", [1, 2, 3640, 3641, 3643, 29129, 87381, 87382, 116508, 116509, 233017, 349525, 349526, 500001])
 def test_round_trip(n):
     announce(f"upload and download of {n} particles")
     with ap.Engine((0, 0, 0), (50.0,) * 3, 2.5, 0.3, cluster_size=8) as e:
