@@ -1709,6 +1709,10 @@ constexpr int kLaneListsBelow = 24;
 // kernel, ~60 per lane in the group form; above it, by a lane each (the group form scans every visit
 // twice, and a build this large fills the GPU with lanes anyway)
 constexpr int64_t kSplitListsBelow = 1 << 18;
+// ... and also where the towers are fewer than two wavefronts per SIMD, however many clusters each holds: a tower per
+// wavefront leaves the rest idle.  97,001 particles, M 4 (841 towers of 29 clusters): 160 -> 72 us,
+// 300,000 (1785 of 42) 294 -> 192, M 8 (1122 of 34) 136 -> 78.
+constexpr int64_t kSplitTowers = 2048;
 
 // The capacities a build keeps for the next one, with headroom for fluctuations (a melting lattice
 // lengthens its rows by ~10% between rebuilds early on: by default a quarter of headroom keeps the two
@@ -1954,9 +1958,10 @@ void vcl_build(Ctx &c) {
   // cluster-entry lists: a lane per i-cluster when the towers hold few clusters, unless the caller chose
   // (list_mode 3: the lane rows with a group of lanes per i-cluster; the automatic choice takes it for the
   // lane rows of builds of fewer than kSplitListsBelow i-clusters)
+  const bool few_towers = c.prm.list_mode == 0 && ntow <= kSplitTowers && ncl < kSplitListsBelow;
   const bool auto_lane = c.prm.list_mode == 0 && ncl < (int64_t)kLaneListsBelow * ntow;
   const bool split_lists =
-      c.prm.list_mode == 3 || (auto_lane && (partial ? c.seg_nclusters : ncl) < kSplitListsBelow);
+      c.prm.list_mode == 3 || few_towers || (auto_lane && (partial ? c.seg_nclusters : ncl) < kSplitListsBelow);
   const bool lane_lists = c.prm.list_mode == 2 || auto_lane || split_lists;
   // (a partial build starts from the stride the other boxes' rows are stored with)
   int32_t cap = jrows ? (c.jccap > 0 ? c.jccap : kJclSplit * 24)
