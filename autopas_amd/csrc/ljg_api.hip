@@ -88,6 +88,7 @@ static void rebuild_for(Ctx &c, int kernel) {
     if (kernel == LJG_KERNEL_VERLET_MIXED) verlet_build(c);
   }
   c.steps_since_rebuild = 0;  // the rebuild's permutation set the reference positions
+  c.moved_far = c.stepped = false;
   std::fill(c.box_since.begin(), c.box_since.end(), 0);
   c.box_pending.clear();
 }
@@ -747,6 +748,7 @@ ljg_status ljg_update_positions(ljg_ctx *h, const double *x, const double *y, co
   unsigned long long word = 0;  // flag[2] and flag[3]
   stream_wait(c, reinterpret_cast<const unsigned long long *>(c.flag.p + 2), 1, &word);
   const int32_t mv = (int32_t)(uint32_t)word;
+  c.moved_far = c.moved_far || mv != 0;
   c.have_forces = false;
   c.box_glob_valid = false;
   if (moved) *moved = mv != 0;
@@ -939,6 +941,7 @@ static void run_steps(Ctx &c, int32_t kernel, int32_t nsteps, double dt, bool ti
   };
   // the drift of step s (fused with the kick of s - 1); with a fused kernel only that of step 0
   auto drift_step = [&](int32_t step, bool speculative) {
+    c.stepped = true;
     if (fused && step > 0) return;
     const SkipIf sk = speculative && dyn ? SkipIf{c.flag.p, stamp_of(step) - 1} : SkipIf{nullptr, 0};
     md_kick_drift(c, !fused && step > 0, true, dt, stamp_of(step), sk);

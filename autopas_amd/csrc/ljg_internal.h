@@ -338,6 +338,8 @@ struct Ctx {
   DevBuf<int32_t> xcount, xcount_tmp;
   int32_t xstride = 0;
   bool xrows_valid = false;     // the current cluster lists carry member rows
+  // Since the last build: an update of the positions reported a move of skin/2; steps were made.
+  bool moved_far = false, stepped = false;
   DevBuf<unsigned int> queue;   // work-queue counters of persistent force launches (kQueueRegions + 1)
   bool queue_ready = false;     // the counters were cleared once after allocation
   DevBuf<float4> pos32;         // per slot: position - c0 of its cluster, type bits in w
