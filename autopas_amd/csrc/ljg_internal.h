@@ -331,7 +331,7 @@ struct Ctx {
   // List entry: x = j cluster | shift id << 27; y,z,w = FP32 bits of c0_j + shift - c0_i (the offset
   // that turns j's cluster-relative FP32 position into i's frame, formed in FP64 and rounded once).
   DevBuf<int4> list;
-  // Member rows of the FP32 cluster kernel: per i-cluster {j slot, entry} of every listed j-cluster
+  // Member rows of the full-list cluster kernels: per i-cluster {j slot, entry} of every listed j-cluster
   // member within ilen of one of its members, at stride xstride = list_row * M (no row can outgrow it);
   // xcount per i-cluster.
   DevBuf<int2> xrow, xrow_tmp;

@@ -117,14 +117,14 @@ bool region_check(const Ctx &c, int64_t n, const double *const src[3], double *c
 }
 
 // An upload in storage order: x, y, z, velocities, types and ids (vx, type, id null: zero, zero, the index) from the
-// arrays given, which may be pinned memory; forces zero, reference positions as given, positions wrapped into
+// arrays given, which may be pinned memory or the state's own; forces zero, reference positions as given, positions wrapped into
 // the box (not those of an ensemble, whose boxes wrap them).
 template <bool HOST>
-__global__ __launch_bounds__(256) void k_init_upload(int64_t n, StateView s, const double *__restrict__ x,
-                                                     const double *__restrict__ y, const double *__restrict__ z,
-                                                     const double *__restrict__ vx, const double *__restrict__ vy,
-                                                     const double *__restrict__ vz, const int32_t *__restrict__ type,
-                                                     const int64_t *__restrict__ id, int32_t wrap, WrapArgs w) {
+__global__ __launch_bounds__(256) void k_init_upload(int64_t n, StateView s, const double *x,
+                                                     const double *y, const double *z,
+                                                     const double *vx, const double *vy,
+                                                     const double *vz, const int32_t *type,
+                                                     const int64_t *id, int32_t wrap, WrapArgs w) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= n) return;
   const double px = load_from<HOST>(x + i), py = load_from<HOST>(y + i), pz = load_from<HOST>(z + i);

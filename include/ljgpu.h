@@ -82,9 +82,10 @@ typedef struct {
                             * of the previous chunk is updated in place when the launch sequence matches
                             * (hipGraphExecUpdate), else instantiated anew.  Per-launch timing events are
                             * then off (ljg_run_stats.force_ms stays 0). */
-  int32_t whole_cluster_rows; /* FP32 cluster kernel (LJG_KERNEL_CLUSTER_MIXED): 0 = each i-cluster streams
+  int32_t whole_cluster_rows; /* full-list cluster kernels (CLUSTER_MIXED, CLUSTER_FP64): 0 = each i-cluster streams
                                * only the j-cluster members within rc + skin of one of its members (a row of
-                               * (entry, member) pairs filtered at every list build); 1 = every member of
+                               * (entry, member) pairs filtered at every list build; the FP64 kernel
+                               * once a particle may have moved skin/2 since: whole entries); 1 = every member of
                                * every listed j-cluster, as VCLClusterFunctor does (VCLClusterFunctor.h:38-89) */
   int32_t persistent;         /* FP32 cluster kernel in ljg_step: 1 = one persistent launch per step, whose
                                * wavefronts (a few per SIMD) take tiles from a work queue in device memory,
@@ -270,7 +271,7 @@ ljg_status ljg_get_clusters(ljg_ctx *ctx, int64_t *slot_particle, int32_t *clust
                             int32_t *list_j, int32_t *list_shift, double *bbox);
 
 /* After a cluster-entry build with member rows (every one for LJG_KERNEL_CLUSTER_MIXED unless
- * whole_cluster_rows is set): per i-cluster the j-cluster members the FP32 cluster kernel streams, as
+ * whole_cluster_rows is set): per i-cluster the j-cluster members the cluster kernels stream, as
  * entry << 3 | member (entry: position in the cluster's entries of ljg_get_clusters).  offsets has
  * num_clusters + 1 entries; rows may be NULL to query the sizes (offsets[num_clusters] is the total).
  * Inspection entry point of this engine's layout (no AutoPas counterpart). */
