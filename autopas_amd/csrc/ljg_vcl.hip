@@ -934,13 +934,16 @@ __global__ __launch_bounds__(kListThreads) void k_cluster_lists_tower(
 // ncl), and the reach is ilen and a margin above their rounding (jcl_geom).  Every test of a pair of boxes in one image
 // computes the same value wherever it is asked.
 // kJclSplit wavefronts per tower split the neighbour-tower visits (oy, ox) into consecutive ranges, a lane per
-// i-cluster; wavefront w writes its entries for i-cluster ci into sub-row w, [ci*cap + w*cap/NS, ...), with its
+// i-cluster; wavefront w writes its entries for i-cluster ci as sub-row w, entry k at jcl[(w*cap/NS + k) * ncl + ci]
+// (lanes side by side write lines side by side: as rows of cap the entries went to memory as partial lines, 107 MB
+// per pass for 15 MB of entries; 2.0M-particle slab 150 -> 121 us and its
+// expansion 607 -> 583), with its
 // length in count[ci*NS + w], so the sub-rows read in order give the whole traversal's order.  Rows have a
 // fixed capacity; the length is the full one even when it exceeds it, so the host can grow it and build
 // again.  The next visit's boxes are loaded into registers while this one runs from LDS.
 // The pass is bound by LDS: with FP64 boxes in LDS as records of 48 bytes the lanes, each at its own place
-// in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 117 us, the 2.0M
-// particle slab 308 -> 150.  Workgroups are dealt so that an XCD takes neighbouring towers.
+// in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 118 us, the 2.0M
+// particle slab 308 -> 121.  Workgroups are dealt so that an XCD takes neighbouring towers.
 constexpr int kJclChunk = 2 * kWave;
 
 struct JclGeom {
@@ -1001,7 +1004,7 @@ __global__ __launch_bounds__(kWave *kJclSplit) void k_jcl_lists(int32_t ntowers,
     float bi[6];
 #pragma unroll
     for (int k = 0; k < 6; ++k) bi[k] = act ? boxf[k * ncl + ci] : 0.f;
-    int32_t *row = jcl + (int64_t)ci * cap + (int64_t)wv * subcap;
+    int32_t *col = jcl + (int64_t)wv * subcap * ncl + ci;
     int32_t cnt = 0;
     // the visits with work, in order: the neighbour tower of visit v within reach and not empty
     auto next_visit = [&](int v, int &vo, int &oxo, int &oyo, int &sxo, int &syo, int &cbo, int &ceo) {
@@ -1081,7 +1084,7 @@ __global__ __launch_bounds__(kWave *kJclSplit) void k_jcl_lists(int32_t ntowers,
             const float bj[6] = {xl, yl, zl, xh, yh, zh};
             if ((bi[5] - bi[2]) + (zh - zl) >= g.one_image_z && passed_earlier(bi, bj, g, tx, ty, oy, ox, sz, r2))
               continue;
-            if (cnt < subcap) row[cnt] = jb + k;
+            if (cnt < subcap) col[cnt * ncl] = jb + k;
             ++cnt;
           }
         }
@@ -1321,7 +1324,7 @@ constexpr int kExpandThreads = 256;
 // The pass is bound by the loads of its ~1000 candidates per cluster, one in four of them kept (a fifth of the
 // requests miss L2).  Every member of a non-cubic box tested in FP64: 954 us a pass for 2.0M particles, M 8; the exact integer
 // difference per pair, in cubic ones: 237 us for 10^6; three FP32 subtractions and a square per pair: 591 and 181;
-// now 607 and 174 us.  The same sums by v_mfma_f32_4x4x1, a lane's j against four members: 669 and 205.
+// now 583 and 163 us.  The same sums by v_mfma_f32_4x4x1, a lane's j against four members: 669 and 205.
 constexpr double kExpandSpan = 1.5;
 
 // Limits in fixed-point units, per dimension: j: L/2 - ilen; q: the largest member offset that the FP32 test
@@ -1411,7 +1414,7 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
       nmax = o > nmax ? o : nmax;
     }
   }
-  const int32_t *crow = jcl + icl * (int64_t)ccap;
+  auto jentry = [&](int w, int k) { return jcl[(int64_t)(w * subcap + k) * nclusters + icl]; };
   extern __shared__ int32_t s_entries[];
   int32_t *srow = STAGED ? s_entries + (int64_t)(threadIdx.x / LG) * ccap : nullptr;
   if constexpr (STAGED) {
@@ -1420,11 +1423,11 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
     // (the sub-rows' first entries are loaded together: most hold no more than LG)
     int32_t first[NS];
 #pragma unroll
-    for (int w = 0; w < NS; ++w) first[w] = l < pre[w + 1] - pre[w] ? crow[w * subcap + l] : 0;
+    for (int w = 0; w < NS; ++w) first[w] = l < pre[w + 1] - pre[w] ? jentry(w, l) : 0;
 #pragma unroll
     for (int w = 0; w < NS; ++w) {
       if (l < pre[w + 1] - pre[w]) srow[pre[w] + l] = first[w];
-      for (int k = l + LG; k < pre[w + 1] - pre[w]; k += LG) srow[pre[w] + k] = crow[w * subcap + k];
+      for (int k = l + LG; k < pre[w + 1] - pre[w]; k += LG) srow[pre[w] + k] = jentry(w, k);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -1439,7 +1442,7 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
     int off = e;
 #pragma unroll
     for (int k = 1; k < NS; ++k) off -= (w == k) ? pre[k] : 0;
-    return crow[w * subcap + off];
+    return jentry(w, off);
   };
   int32_t *jrow = jrows + icl * (int64_t)cap;
   const unsigned long long gmask = (LG == kWave ? ~0ull : ((1ull << LG) - 1ull)) << (grp * LG);
