@@ -640,6 +640,12 @@ __device__ inline int xcd_block(int n, unsigned block, unsigned grid) {
   return k < n ? k : n;
 }
 
+// The same for work whose share varies along its order (towers and cells of an inhomogeneous system): XCD k takes every
+// eighth chunk of q, of about 256 chunks in all.  Its i-th piece; `len` of them, some beyond n.
+inline __host__ __device__ int xcd_chunk(int n) { return (n + 255) / 256 > 1 ? (n + 255) / 256 : 1; }
+inline __host__ __device__ int xcd_chunk_len(int n, int q) { return ((n + q - 1) / q + 7) / 8 * q; }
+__device__ inline int xcd_dealt(int q, int k, int i) { return (i / q * 8 + k) * q + i % q; }
+
 // The FP32 cluster kernel's two position buffers change roles (its fused integrator wrote the next step's
 // positions into the second): the FP32 and the FP64 copies always together.
 // The ownership the force kernels mask the globals with: none (every particle counts) unless the caller

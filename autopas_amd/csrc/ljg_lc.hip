@@ -99,11 +99,13 @@ __global__ __launch_bounds__(kLcThreads, 4) void k_force_lc_fp64(
   const int no0 = g.nh[0] - 2, no1 = g.nh[1] - 2, no2 = g.nh[2] - 2;
   double e_sum = 0., v_sum = 0.;
   int32_t hits = 0;
-  // Workgroups are dealt to the 8 XCDs in turn: XCD k takes the k-th eighth of the cells, its workgroups
-  // consecutive cells at a time, so that neighbouring cells meet in its L2.
-  const int per = (ncells + 7) / 8, stride = (int)gridDim.x / 8;
-  const int c_end = min(((int)(blockIdx.x & 7) + 1) * per, ncells);
-  for (int c = (int)(blockIdx.x & 7) * per + (int)(blockIdx.x >> 3); c < c_end; c += stride) {
+  // Workgroups are dealt to the 8 XCDs in turn: an XCD takes chunks of consecutive cells, so that neighbouring cells
+  // meet in its L2, and chunks from all over the box, so that a film across it keeps every XCD busy (the 2.0M-particle
+  // slab with an eighth of the cells per XCD 7.6 ms a step, now 3.8; 500,000 in a liquid 385 -> 373 us a call).
+  const int q = xcd_chunk(ncells), len = xcd_chunk_len(ncells, q), stride = (int)gridDim.x / 8;
+  for (int k = (int)(blockIdx.x >> 3); k < len; k += stride) {
+    const int c = xcd_dealt(q, (int)(blockIdx.x & 7), k);
+    if (c >= ncells) continue;
     const int64_t ib = cell_start[c], ie = cell_start[c + 1];
     if (ib == ie) continue;
     // (a halo cell holds particles only if their positions are not numbers: they meet some cell's)

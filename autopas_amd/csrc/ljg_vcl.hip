@@ -943,7 +943,8 @@ __global__ __launch_bounds__(kListThreads) void k_cluster_lists_tower(
 // again.  The next visit's boxes are loaded into registers while this one runs from LDS.
 // The pass is bound by LDS: with FP64 boxes in LDS as records of 48 bytes the lanes, each at its own place
 // in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 118 us, the 2.0M
-// particle slab 308 -> 121.  Workgroups are dealt so that an XCD takes neighbouring towers.
+// particle slab 308 -> 121.  Workgroups are dealt so that an XCD takes chunks of neighbouring
+// towers.
 constexpr int kJclChunk = 2 * kWave;
 
 struct JclGeom {
@@ -990,7 +991,7 @@ __global__ __launch_bounds__(kWave *kJclSplit) void k_jcl_lists(int32_t ntowers,
   __shared__ float s_box[NS][6][kJclChunk];
   const int wv = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   float(&sb)[6][kJclChunk] = s_box[wv];
-  const int t = xcd_block(ntowers, blockIdx.x, gridDim.x);
+  const int t = xcd_dealt(xcd_chunk(ntowers), (int)(blockIdx.x & 7), (int)(blockIdx.x >> 3));
   if (t >= ntowers) return;
   const int tx = t % g.nt[0], ty = t / g.nt[0];
   const int ib = (int)cstart[t], ie = ib + ccount[t];
@@ -1989,7 +1990,7 @@ void vcl_build(Ctx &c) {
     if (n_towers == 0 || n_lane == 0)
       ;  // no box marked
     else if (jrows)
-      hipLaunchKernelGGL(k_jcl_lists, dim3(xcd_grid((int)ntow)), dim3(kWave * kJclSplit), 0, c.stream, (int32_t)ntow,
+      hipLaunchKernelGGL(k_jcl_lists, dim3((unsigned)(8 * xcd_chunk_len((int)ntow, xcd_chunk((int)ntow)))), dim3(kWave * kJclSplit), 0, c.stream, (int32_t)ntow,
                          jcl_geom(g), c.ctow_start.p, c.ctow_count.p, ncl, c.boxf.p, cap, c.list_count.p, c.jcl.p);
     else if (split_lists && ens)
       hipLaunchKernelGGL((k_cluster_lists_split<true>), dim3(blocks_for(n_lane * kSplitLanes, kListSplitThreads)),
