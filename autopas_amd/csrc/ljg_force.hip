@@ -576,6 +576,7 @@ __global__ void k_zero_forces(int64_t n, double *__restrict__ fx, double *__rest
 // Groups that share a cluster's members in a fused member-row launch of `blocks` workgroups unsplit (256 are a wavefront
 // per SIMD): four or two while that makes no more than two to three wavefronts per SIMD, us per launch unsplit / 2 / 4 / 8:
 // 22 workgroups (700 particles, M8 G1) 9.5 / - / 7.25 / 7.3, 235 (30,011, M8 G4) 15.4 / 12.8 / 14.4 / -.
+// M 4 by two, steps with their builds (which got faster too): 6859 particles, G4, 17.6 -> 14.5 us.
 static int member_split(int M, int blocks) {
   if (M == 8) return blocks <= 128 ? 4 : blocks <= 384 ? 2 : 1;
   return M == 4 && blocks <= 256 ? 2 : 1;

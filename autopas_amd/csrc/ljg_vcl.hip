@@ -601,8 +601,8 @@ __device__ inline float cluster_derive(int64_t s, int32_t M, bool mine, bool rea
 // padding slot.  The rebuild reference positions are set to the positions; when posfx is given the slots'
 // 32-bit fixed-point positions are written too (type -1 for padding).  Inside the step loop the force is
 // recomputed right after a rebuild, so it is not carried.  The cluster's box and FP32 positions come from the
-// values this pass holds anyway: passes of their own over the slots cost 21 and (cluster-entry builds) 40 us more at 2.0M slots, and two
-// launches.
+// values this pass holds anyway: passes of their own over the slots cost 21 and (cluster-entry builds) 40 us more
+// at 2.0M slots, and two launches.
 __global__ __launch_bounds__(256) void k_permute_clusters(int64_t nnew, int32_t M, const int32_t *__restrict__ src,
                                                           StateView o, StateView n, int32_t carry_force,
                                                           int4 *__restrict__ posfx, FixGeom f, ClusterOut out) {
