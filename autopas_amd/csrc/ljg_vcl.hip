@@ -7,6 +7,7 @@
 #include <cmath>
 
 #include "ljg_internal.h"
+#include "ljg_order.h"
 
 namespace ljg {
 
@@ -274,7 +275,7 @@ __global__ __launch_bounds__(kLayoutBlock) void k_layout_apply(int64_t ntowers, 
   }
 }
 
-// One workgroup per tower: bitonic sort of (z, id) in LDS, then the tower's slots of the cluster layout
+// One workgroup per tower: bitonic sort by tower_before in LDS, then the tower's slots of the cluster layout
 // are written: src[new slot] = old slot, -1 for padding; cluster_tower for the tower's clusters.  A tower
 // holds count[t] particles, its items from start[t], its clusters [cstart[t], cstart[t] + ccount[t]).
 // It takes the rare towers that are longer than the register sorts reach (min_n), up to kTowerSortCap.
@@ -284,9 +285,7 @@ constexpr int kSortRegisters = 1024;  // towers up to this are sorted in registe
 __device__ inline bool zid_less(double za, int32_t sa, double zb, int32_t sb, const int64_t *__restrict__ id) {
   if (sb < 0) return sa >= 0;  // padding sorts last
   if (sa < 0) return false;
-  if (za < zb) return true;
-  if (za > zb) return false;
-  return id[sa] < id[sb];
+  return tower_before(za, id[sa], sa, zb, id[sb], sb);
 }
 
 template <int CAP>
@@ -344,17 +343,21 @@ __global__ __launch_bounds__(kSortThreads) void k_tower_sort(
 
 // Towers of up to 64 particles: one wavefront per tower sorts (z, id) in registers with a bitonic network
 // over 64 E elements, element e * 64 + lane in slot e of a lane (padding sorts last), and writes the same
-// cluster layout as k_tower_sort.  Keys are distinct (ids are), so every sorter produces the one sorted
+// cluster layout as k_tower_sort.  The order is total (tower_before), so every sorter produces the one sorted
 // order.
 constexpr int kSortWaveThreads = 256;
 
-// The register sort carries two words per element: its z rounded to FP32 and its index k in the tower's
-// item list.  Rounding is monotone, so a smaller FP32 z means a smaller z; equal FP32 z (rare) are
-// ordered by the exact (z, id) read back from the item list, in a branch a wavefront takes only when one
-// of its lanes holds such a pair.  Indices k < 0 are padding and sort last.
+// The register sort carries two words per element: its z rounded to FP32 (tower_key32) and its index k in the
+// tower's item list.  A smaller FP32 z means a smaller z; equal FP32 z (rare) are ordered by the exact (z, id, slot)
+// read back from the item list, in a branch a wavefront takes only when one of its lanes holds such a pair.
+// Indices k < 0 are padding and sort last.
 struct TowerItems {
   const double *z;
   const int64_t *id;
+  const int32_t *slot;
+  __device__ bool before(int32_t a, int32_t b) const {
+    return tower_before(z[a], id[a], slot[a], z[b], id[b], slot[b]);
+  }
 };
 
 __device__ inline void zk_less2(float za, int32_t ka, float zb, int32_t kb, const TowerItems &ti, bool &ab, bool &ba) {
@@ -363,9 +366,7 @@ __device__ inline void zk_less2(float za, int32_t ka, float zb, int32_t kb, cons
   const bool tie = (ka >= 0) & (kb >= 0) & (za == zb);
   if (__builtin_amdgcn_ballot_w64(tie) != 0ull) {
     if (tie) {
-      const double da = ti.z[ka], db = ti.z[kb];
-      const int64_t ia = ti.id[ka], ib = ti.id[kb];
-      ab = (da < db) | ((da == db) & (ia < ib));
+      ab = ti.before(ka, kb);
       ba = !ab;
     }
   }
@@ -437,9 +438,9 @@ __global__ __launch_bounds__(kSortWaveThreads) void k_tower_sort_wave(
   for (int e = 0; e < E; ++e) {
     const int k = e * kWave + lane;
     kv[e] = k < n ? k : -1;
-    zv[e] = k < n ? (float)items_z[b + k] : 0.f;
+    zv[e] = k < n ? tower_key32(items_z[b + k]) : 0.f;
   }
-  const TowerItems ti{items_z + b, items_id + b};
+  const TowerItems ti{items_z + b, items_id + b, items + b};
   bitonic2_sizes<E, 2>(zv, kv, lane, ti);
   const int64_t c0 = cstart[t], c1 = c0 + ccount[t];
   const int nslot = (int)((c1 - c0) * M);
@@ -454,7 +455,7 @@ __global__ __launch_bounds__(kSortWaveThreads) void k_tower_sort_wave(
 // Longer towers of up to 1024 particles: W wavefronts per tower, each sorting one W-th of up to 64 E
 // particles in registers as k_tower_sort_wave does, then a merge by rank: an element's place is its index in
 // its part plus the number of the other parts' elements before it (a binary search in each, held in LDS;
-// equal FP32 z are ordered by the exact z and id).  Two wavefronts with half the network each beat one
+// equal FP32 z are ordered by tower_before).  Two wavefronts with half the network each beat one
 // with the whole, and for 513 to 1024 particles four beat the sort in LDS with its 55 barriers: 2500 towers
 // of 800 particles 173 -> 82 us.  Instances: 65 to 256 particles (E = 2, W = 2), 257 to 512
 // (4, 2), 513 to 1024 (4, 4).
@@ -485,9 +486,9 @@ __global__ __launch_bounds__(W *kWave) void k_tower_sort_parts(
   for (int e = 0; e < E; ++e) {
     const int k = e * kWave + lane;
     kv[e] = k < len ? first + k : -1;
-    zf[e] = k < len ? (float)items_z[b + first + k] : 0.f;
+    zf[e] = k < len ? tower_key32(items_z[b + first + k]) : 0.f;
   }
-  const TowerItems ti{items_z + b, items_id + b};
+  const TowerItems ti{items_z + b, items_id + b, items + b};
   bitonic2_sizes<E, 2>(zf, kv, lane, ti);
 #pragma unroll
   for (int e = 0; e < E; ++e) {
@@ -513,11 +514,7 @@ __global__ __launch_bounds__(W *kWave) void k_tower_sort_parts(
         const int mid = (lo + hi) >> 1;
         const float zo = oz[mid];
         bool before = zo < z;
-        if (zo == z) {
-          const int32_t ko = s_k[op][mid];
-          const double da = ti.z[ko], db = ti.z[k];
-          before = (da < db) | ((da == db) & (ti.id[ko] < ti.id[k]));
-        }
+        if (zo == z) before = ti.before(s_k[op][mid], k);
         if (before) lo = mid + 1;
         else hi = mid;
       }
@@ -664,7 +661,7 @@ __global__ __launch_bounds__(256) void k_copy_box_clusters(int64_t nitems, Segs 
 }
 
 // The first passes of a small build in one workgroup: wrap and towers of the particles, tower and cluster
-// offsets, and each particle's place among its tower's (z, then id) by counting those before it, with the
+// offsets, and each particle's place among its tower's by counting those before it (tower_before), with the
 // tower's z in LDS.  A build of a few hundred to a few thousand particles is bound by its launches (~5 us
 // each with the gap before it), and these were seven: clear, histogram, offsets, their marker, scatter, sort,
 // and a second clear.  The sizes go to the host's marker words as soon as they are known.  Towers longer than
@@ -775,7 +772,8 @@ __global__ __launch_bounds__(kSmallThreads) void k_tower_small(
       for (int m = b; m < e; ++m) {
         const double zm = s_z[m];
         bool less = zm < pz[k];
-        if (zm == pz[k] && s_i[m] != i) less = id[s_i[m]] < id[i];
+        if (!less && !(zm > pz[k]) && s_i[m] != i)  // equal, or not a number
+          less = tower_before(zm, id[s_i[m]], s_i[m], pz[k], id[i], i);
         place += less ? 1 : 0;
       }
       src[(int)((uint32_t)s_off[t[k]] >> 16) * M + place] = i;
