@@ -36,8 +36,9 @@ __global__ void k_cell_scatter(int64_t nslots, const int32_t *__restrict__ cell_
 
 // The atomic histogram hands out ranks in arbitrary order; every cell's members are put in particle-id
 // order so the layout (and with it every floating-point summation order downstream) is reproducible.
-// A thread per member counts the members of its cell with a smaller id (ids are distinct) and writes
-// itself to that place: independent loads of the cell's few entries, instead of a serial sort per cell.
+// A thread per member counts the members of its cell with a smaller id (equal ids: a smaller index, so that no two
+// share a place) and writes itself to that place: independent loads of the cell's few entries, instead of a serial
+// sort per cell.
 __global__ void k_cell_order_by_id(int64_t n, const int32_t *__restrict__ items, const int32_t *__restrict__ cell_of,
                                    const int64_t *__restrict__ start, const int64_t *__restrict__ id,
                                    int32_t *__restrict__ sorted) {
@@ -48,7 +49,11 @@ __global__ void k_cell_order_by_id(int64_t n, const int32_t *__restrict__ items,
   const int64_t b = start[c], e = start[c + 1];
   const int64_t key = id ? id[v] : v;  // without ids: the index
   int64_t r = 0;
-  for (int64_t m = b; m < e; ++m) r += (id ? id[items[m]] : items[m]) < key ? 1 : 0;
+  for (int64_t m = b; m < e; ++m) {
+    const int32_t o = items[m];
+    const int64_t k2 = id ? id[o] : o;
+    r += (k2 < key) | ((k2 == key) & (o < v)) ? 1 : 0;
+  }
   sorted[b + r] = v;
 }
 

@@ -94,3 +94,19 @@ def test_every_particle_is_kept(kernel, n, edge, height, bad):
             f = e.download()
             for k, v in zip("xyz", (x, y, z)):
                 assert np.array_equal(f[k], v, equal_nan=True), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kernel", [ap.KERNEL_LC_FP64, ap.KERNEL_VERLET_MIXED])
+@pytest.mark.parametrize("n,L", [(800, 9.0), (5000, 20.0)])
+def test_cells_keep_particles_of_equal_ids(kernel, n, L):
+    announce(f"cell order, kernel {kernel}: {n} particles whose ids are not distinct")
+    rng = np.random.default_rng(n)
+    p = [rng.uniform(0, L, n) for _ in range(3)]
+    with ap.Engine((0, 0, 0), (L, L, L), 2.5, 0.3) as e:
+        e.upload(*p, id=rng.integers(0, 3, n))
+        for _ in range(2):
+            e.rebuild(kernel)
+            f = e.download()
+            for k, v in zip("xyz", p):
+                assert np.array_equal(f[k], v), k
