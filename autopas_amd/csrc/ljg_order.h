@@ -15,13 +15,11 @@ namespace ljg {
 // after all numbers, and equal ids fall back to the slots, which are distinct.  The sorts that rank (a place is the
 // number of particles before) need that: two particles that are each not before the other would share a place and
 // leave another place of the tower unwritten, which the permutation then reads as an old slot.
+// (Without branches: it stands in every stage of the sorting networks.)
 LJG_HD inline bool tower_before(double za, int64_t ia, int32_t sa, double zb, int64_t ib, int32_t sb) {
-  if (za < zb) return true;
-  if (za > zb) return false;
   const bool na = za != za, nb = zb != zb;
-  if (na != nb) return nb;
-  if (ia != ib) return ia < ib;
-  return sa < sb;
+  const bool same = (za == zb) | (na & nb);
+  return (za < zb) | (nb & !na) | (same & ((ia < ib) | ((ia == ib) & (sa < sb))));
 }
 
 // The FP32 word that the register sorts compare first: monotone in that order (rounding is, and what is not a
