@@ -1079,9 +1079,10 @@ __global__ __launch_bounds__(kWave *kJclSplit) void k_jcl_lists(int32_t ntowers,
             const float xl = sb[0][k], yl = sb[1][k], xh = sb[3][k], yh = sb[4][k];
             if (boxf_dist2(bi, xl, yl, zl, xh, yh, zh, shx, shy, shz) > r2) continue;
             // Two z images of a j-cluster can both pass only if twice the reach and the two clusters' z-extents
-            // together come to the box length: below one_image_z no earlier image needs a look.
+            // together come to the box length: below one_image_z no earlier image needs a look (boxes that are
+            // not numbers pass in every image and need one).
             const float bj[6] = {xl, yl, zl, xh, yh, zh};
-            if ((bi[5] - bi[2]) + (zh - zl) >= g.one_image_z && passed_earlier(bi, bj, g, tx, ty, oy, ox, sz, r2))
+            if (!((bi[5] - bi[2]) + (zh - zl) < g.one_image_z) && passed_earlier(bi, bj, g, tx, ty, oy, ox, sz, r2))
               continue;
             if (cnt < subcap) col[cnt * ncl] = jb + k;
             ++cnt;
@@ -1403,7 +1404,11 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
     const int32_t cw = ccount[icl * NS + w];
     pre[w + 1] = pre[w] + (cw < subcap ? cw : subcap);
   }
-  const int nflat = live ? pre[NS] * M : 0;
+  // The first pass lists no cluster, not even itself, where all members lie outside the box along z (farther than a
+  // wrap brings back): its row is its own members.
+  const bool alone = pre[NS] == 0;
+  const int entries = alone ? 1 : pre[NS];
+  const int nflat = live ? entries * M : 0;
   // the loop runs to the wave's longest stream so that the ballots stay uniform
   int nmax = nflat;
   if constexpr (G > 1) {
@@ -1428,6 +1433,7 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
       if (l < pre[w + 1] - pre[w]) srow[pre[w] + l] = first[w];
       for (int k = l + LG; k < pre[w + 1] - pre[w]; k += LG) srow[pre[w] + k] = jentry(w, k);
     }
+    if (alone && l == 0) srow[0] = (int32_t)icl;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -1435,6 +1441,7 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
   // entry e of the concatenated sub-rows
   auto centry = [&](int e) {
     if constexpr (STAGED) return srow[e];
+    if (alone) return (int32_t)icl;
     int w = 0;
 #pragma unroll
     for (int k = 1; k < NS; ++k) w += e >= pre[k] ? 1 : 0;
@@ -1446,10 +1453,10 @@ __global__ __launch_bounds__(kExpandThreads) void k_jrows_expand(
   int32_t *jrow = jrows + icl * (int64_t)cap;
   const unsigned long long gmask = (LG == kWave ? ~0ull : ((1ull << LG) - 1ull)) << (grp * LG);
   int32_t cnt = 0;
-  // Every row holds at least one entry (the cluster's own, or a full sub-row), so with the element
+  // Every row holds at least one entry (the cluster's own), so with the element
   // index clamped to the stream's last one every lane, dead groups included, loads a real slot and the
   // prefetches need no guard.
-  const int klast = pre[NS] * M - 1;
+  const int klast = entries * M - 1;
   // (offsets within these limits, less the rounding of a length, keep the row in the members' frame)
   const float limx = (float)jlim[0] * scx * 0.999999f, limy = (float)jlim[1] * scy * 0.999999f;
   const float limz = (float)jlim[2] * scz * 0.999999f;
