@@ -1525,10 +1525,15 @@ __global__ void k_zero_u64(int64_t n, unsigned long long *__restrict__ p) {
 // next build (each particle moves less than skin/2).  G i-clusters per wavefront stream their list's
 // (entry, member) pairs and keep those within ilen of a real i-member, compacted in stream order with a
 // ballot and a prefix popcount: xrow[ic * xstride + k] = {j slot, entry}, xcount[ic] of them.  The
-// test is FP32 on the cluster-relative positions (the kernel's own arithmetic) against ilen^2 (1 + 2^-16),
-// whose margin is far above the FP32 error of d^2, so a row holds every member within ilen in FP64 and
-// at most a few more.  The cluster's own members are kept (the force kernel drops the pair of a member
-// with itself).
+// test is FP32 on the cluster-relative positions (the kernel's own arithmetic) against ilen^2 and a margin above
+// its error, so a row holds every member within ilen in FP64 and at most a few more.  With E the largest component
+// of the candidate's and the i-members' offsets from their clusters' reference points, the two offsets round by
+// 2^-24 E each, the entry's offset (up to ilen + 2 E) and the sum of it and j's by 2^-24 of their size, the
+// difference by 2^-24 ilen: 2^-24 (5 E + 3 ilen) per component, sqrt(3) of that in length, a few 2^-24 of d^2 in
+// its sum.  The margin is that, and at least 2^-16 ilen^2, which covers clusters of up to ~14 ilen; in a dilute box
+// they are longer (the fixed margin alone lost 110 of 222 pairs near rc in a box of 3e4 with skin 0).  It comes from
+// the pair's own clusters, so a box's rows do not depend on other boxes of an ensemble.  The cluster's own members are
+// kept (the force kernel drops the pair of a member with itself).
 constexpr int kXrowThreads = 256;
 #ifndef LJG_XROWS_SMALL
 #define LJG_XROWS_SMALL 32768
@@ -1548,7 +1553,7 @@ template <int M, int G>
 __global__ __launch_bounds__(kXrowThreads) void k_cluster_xrows(int64_t nitems, Segs sg,
                                                                 const float4 *__restrict__ pos32, int32_t row,
                                                                 const int32_t *__restrict__ lcount,
-                                                                const int4 *__restrict__ list, float thr,
+                                                                const int4 *__restrict__ list, float ilen, float thr,
                                                                 int32_t xstride, int32_t *__restrict__ xcount,
                                                                 int2 *__restrict__ xrow) {
   constexpr int LG = kWave / G;
@@ -1557,14 +1562,18 @@ __global__ __launch_bounds__(kXrowThreads) void k_cluster_xrows(int64_t nitems, 
   const int64_t item = ((int64_t)blockIdx.x * (kXrowThreads / kWave) + threadIdx.x / kWave) * G + grp;
   const bool live = item < nitems;
   const int64_t ic = seg_index(sg, live ? item : nitems - 1);
-  float xi[M], yi[M], zi[M];
+  float xi[M], yi[M], zi[M], ei = 0.f;
 #pragma unroll
   for (int q = 0; q < M; ++q) {
     const float4 p = pos32[ic * M + q];
     xi[q] = p.x;
     yi[q] = p.y;
     zi[q] = p.z;
+    ei = p.x != kPadPos32 ? fmaxf(ei, fmaxf(fabsf(p.x), fmaxf(fabsf(p.y), fabsf(p.z)))) : ei;
   }
+  asm volatile("" : "+v"(ei));  // one register, not the members' part of it in eight
+  constexpr float kSlope = 1.04e-7f;  // sqrt(3) 2^-24, rounded up
+  const float reach = ilen * (1.f + 3.f * kSlope + 0x1p-20f);  // (2^-20: the roundings of d^2 and of the margin)
   const int nj = live ? min(lcount[ic], row) * M : 0;
   int nmax = nj;  // the loop runs to the wave's longest stream so that the ballots stay uniform
 #pragma unroll
@@ -1596,12 +1605,15 @@ __global__ __launch_bounds__(kXrowThreads) void k_cluster_xrows(int64_t nitems, 
       if (p.x != kPadPos32) {
         const float jx = p.x + __int_as_float(ep.e.y), jy = p.y + __int_as_float(ep.e.z),
                     jz = p.z + __int_as_float(ep.e.w);
+        float dmin = __builtin_inff();  // (a padding i-member, at +3e30, is not near)
 #pragma unroll
         for (int q = 0; q < M; ++q) {
           const float dx = xi[q] - jx, dy = yi[q] - jy, dz = zi[q] - jz;
-          const float d2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
-          near = near || d2 <= thr;  // a padding i-member (at +3e30) is never near
+          dmin = fminf(dmin, __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz)));
         }
+        const float e = fmaxf(ei, fmaxf(fabsf(p.x), fmaxf(fabsf(p.y), fabsf(p.z))));
+        const float far = __builtin_fmaf(5.f * kSlope, e, reach);
+        near = dmin <= fmaxf(thr, far * far);
       }
     }
     const unsigned long long ball = __ballot(near) & gmask;
@@ -1669,7 +1681,7 @@ void vcl_member_rows(Ctx &c, bool partial, const int32_t *active) {
     const int nb = blocks_for(ni, (kXrowThreads / kWave) * (small ? 1 : 4));
 #define LJG_XROWS(MV, GV)                                                                                          \
   hipLaunchKernelGGL((k_cluster_xrows<MV, GV>), dim3(nb), dim3(kXrowThreads), 0, c.stream, ni, sg, c.pos32.p,       \
-                     c.list_row, c.list_count.p, c.list.p, thr, xs, c.xcount.p, c.xrow.p)
+                     c.list_row, c.list_count.p, c.list.p, (float)ilen, thr, xs, c.xcount.p, c.xrow.p)
 #define LJG_XROWS_M(MV)                                                                                            \
   case MV:                                                                                                         \
     if (small) LJG_XROWS(MV, 1); else LJG_XROWS(MV, 4);                                                            \
