@@ -81,6 +81,7 @@ static void rebuild_for(Ctx &c, int kernel) {
   if (is_cluster_kernel(kernel)) {  // the tower histogram wraps the positions
     c.want_jrows = kernel == LJG_KERNEL_CLUSTER_JROWS_MIXED;
     c.want_n3 = is_n3_kernel(kernel);
+    c.want_fp64 = kernel == LJG_KERNEL_CLUSTER_FP64;
     vcl_build(c);
   } else {
     wrap_positions(c);
@@ -183,7 +184,7 @@ static void rebuild_boxes(Ctx &c, int kernel, const std::vector<int32_t> &mark, 
   }
   if (!segments_ready && !prepare_segments(c, mark)) return;
   c.want_jrows = false;
-  c.want_n3 = false;
+  c.want_n3 = c.want_fp64 = false;
   c.build_partial = true;
   try {
     vcl_build(c);

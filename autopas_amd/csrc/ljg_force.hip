@@ -713,8 +713,9 @@ static void launch_fp64(Ctx &c, bool mix, bool glob, const ForceArgs &a, const d
     else LJG_LAUNCH1(MIXV, GLOBV, N3V, false);                                                                     \
   } while (0)
   // Member rows hold every pair that can come within rc while no particle has moved skin/2 since the build: always in
-  // steps that rebuild then, and elsewhere unless an update of the positions reported it.
-  const bool xr = c.xrows_valid && !n3 && !c.moved_far && (c.prm.dynamic_rebuild != 0 || !c.stepped);
+  // steps that rebuild then, and elsewhere unless an update of the positions reported it.  Rows made for the FP32
+  // kernel leave out what is not a number: whole entries then.
+  const bool xr = c.xrows_valid && c.xrows_fp64 && !n3 && !c.moved_far && (c.prm.dynamic_rebuild != 0 || !c.stepped);
   if (n3) {
     hipLaunchKernelGGL(k_zero_forces, dim3(blocks_for(c.nslots, 256)), dim3(256), 0, c.stream, c.nslots, s.fx.p,
                        s.fy.p, s.fz.p, c.skip);

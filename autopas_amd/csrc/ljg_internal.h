@@ -338,6 +338,7 @@ struct Ctx {
   DevBuf<int32_t> xcount, xcount_tmp;
   int32_t xstride = 0;
   bool xrows_valid = false;     // the current cluster lists carry member rows
+  bool xrows_fp64 = false;      // ... and they were made for the FP64 kernel (want_fp64)
   // Since the last build: an update of the positions reported a move of skin/2; steps were made.
   bool moved_far = false, stepped = false;
   DevBuf<unsigned int> queue;   // work-queue counters of persistent force launches (kQueueRegions + 1)
@@ -372,6 +373,7 @@ struct Ctx {
   bool lists_pending = false;    // the current j rows' lengths are not yet checked on the host
   int32_t pend_cap = 0, pend_jcap = 0;
   bool pend_fast = false;        // the vetoed launch used the first member's frame
+  bool want_fp64 = false;        // the next cluster build's member rows are for the FP64 kernel
   bool want_n3 = false;          // the next cluster build emits Newton-3 (forward-only) cluster-entry lists
   bool lists_n3 = false;         // the current cluster-entry lists are Newton-3 lists
   DevBuf<int32_t> vcount;        // neighbours per particle

@@ -1533,8 +1533,11 @@ __global__ void k_zero_u64(int64_t n, unsigned long long *__restrict__ p) {
 // its sum.  The margin is that, and at least 2^-16 ilen^2, which covers clusters of up to ~14 ilen; in a dilute box
 // they are longer (the fixed margin alone lost 110 of 222 pairs near rc in a box of 3e4 with skin 0).  It comes from
 // the pair's own clusters, so a box's rows do not depend on other boxes of an ensemble.  The cluster's own members are
-// kept (the force kernel drops the pair of a member with itself).
+// kept (the force kernel drops the pair of a member with itself).  With keep_odd (rows for the FP64 kernel) so are
+// candidates, and all candidates of i-members, whose position is not a finite number: forces near them are not
+// numbers, as with whole entries, and do not look sound.
 constexpr int kXrowThreads = 256;
+constexpr float kOddAbove = 1e37f;  // (padding slots stay below, at 3 x 3e30)
 #ifndef LJG_XROWS_SMALL
 #define LJG_XROWS_SMALL 32768
 #endif
@@ -1554,7 +1557,7 @@ __global__ __launch_bounds__(kXrowThreads) void k_cluster_xrows(int64_t nitems, 
                                                                 const float4 *__restrict__ pos32, int32_t row,
                                                                 const int32_t *__restrict__ lcount,
                                                                 const int4 *__restrict__ list, float ilen, float thr,
-                                                                int32_t xstride, int32_t *__restrict__ xcount,
+                                                                int32_t keep_odd, int32_t xstride, int32_t *__restrict__ xcount,
                                                                 int2 *__restrict__ xrow) {
   constexpr int LG = kWave / G;
   const int lane = threadIdx.x & (kWave - 1);
@@ -1574,6 +1577,11 @@ __global__ __launch_bounds__(kXrowThreads) void k_cluster_xrows(int64_t nitems, 
   asm volatile("" : "+v"(ei));  // one register, not the members' part of it in eight
   constexpr float kSlope = 1.04e-7f;  // sqrt(3) 2^-24, rounded up
   const float reach = ilen * (1.f + 3.f * kSlope + 0x1p-20f);  // (2^-20: the roundings of d^2 and of the margin)
+  bool odd_i = false;
+  if (keep_odd) {
+#pragma unroll
+    for (int q = 0; q < M; ++q) odd_i = odd_i | !(fabsf(xi[q] + yi[q] + zi[q]) < kOddAbove);
+  }
   const int nj = live ? min(lcount[ic], row) * M : 0;
   int nmax = nj;  // the loop runs to the wave's longest stream so that the ballots stay uniform
 #pragma unroll
@@ -1614,6 +1622,7 @@ __global__ __launch_bounds__(kXrowThreads) void k_cluster_xrows(int64_t nitems, 
         const float e = fmaxf(ei, fmaxf(fabsf(p.x), fmaxf(fabsf(p.y), fabsf(p.z))));
         const float far = __builtin_fmaf(5.f * kSlope, e, reach);
         near = dmin <= fmaxf(thr, far * far);
+        if (keep_odd) near = near | odd_i | !(fabsf(jx + jy + jz) < kOddAbove);
       }
     }
     const unsigned long long ball = __ballot(near) & gmask;
@@ -1681,7 +1690,8 @@ void vcl_member_rows(Ctx &c, bool partial, const int32_t *active) {
     const int nb = blocks_for(ni, (kXrowThreads / kWave) * (small ? 1 : 4));
 #define LJG_XROWS(MV, GV)                                                                                          \
   hipLaunchKernelGGL((k_cluster_xrows<MV, GV>), dim3(nb), dim3(kXrowThreads), 0, c.stream, ni, sg, c.pos32.p,       \
-                     c.list_row, c.list_count.p, c.list.p, (float)ilen, thr, xs, c.xcount.p, c.xrow.p)
+                     c.list_row, c.list_count.p, c.list.p, (float)ilen, thr, (int32_t)c.want_fp64, xs,      \
+                     c.xcount.p, c.xrow.p)
 #define LJG_XROWS_M(MV)                                                                                            \
   case MV:                                                                                                         \
     if (small) LJG_XROWS(MV, 1); else LJG_XROWS(MV, 4);                                                            \
@@ -1695,6 +1705,7 @@ void vcl_member_rows(Ctx &c, bool partial, const int32_t *active) {
     LJG_HIP(hipGetLastError());
   }
   c.xrows_valid = true;
+  c.xrows_fp64 = c.want_fp64;
 }
 
 // What a build starts from at zero, in one launch: the tower counts (n of them), the list statistics, and

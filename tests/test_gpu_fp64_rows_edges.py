@@ -1,5 +1,5 @@
-"""Member rows where clusters are long (dilute boxes, films in vacuum), and after steps without builds: the FP64
-cluster kernel on them against whole entries, the FP32 one on its pairs."""
+"""Member rows where clusters are long (dilute boxes, films in vacuum), with particles that are not numbers, and after
+steps without builds: the FP64 cluster kernel on them against whole entries, the FP32 one on its pairs."""
 import numpy as np
 import pytest
 
@@ -52,6 +52,33 @@ def test_no_pair_is_lost_in_long_clusters(M, box, skin):
             if kernel == ap.KERNEL_CLUSTER_FP64:
                 assert np.max(np.abs(fa[k] - fb[k])) <= TOL * np.max(np.abs(fb[k])), k
             assert np.array_equal(fa[k] != 0.0, fb[k] != 0.0), k
+
+
+@pytest.mark.parametrize("M", [2, 4, 8])
+@pytest.mark.parametrize("bad", [(np.nan, 0.0, 0.0), (0.0, 0.0, np.nan), (np.nan, np.nan, np.nan)])
+def test_not_a_number_is_not_hidden(M, bad):
+    announce(f"FP64 member rows M={M}, one particle displaced by {bad}")
+    n_side, a = 8, 0.7 ** (-1.0 / 3.0)
+    L = n_side * a
+    x, y, z, _, _, _, _ = ap.generate_lattice(5, n_side ** 3, (n_side,) * 3, a, (0, 0, 0), 0.1, 0.9)
+    at = 77
+    for v, b in zip((x, y, z), bad):
+        v[at] += b
+    res = []
+    for whole in (False, True):
+        with ap.Engine((0, 0, 0), (L,) * 3, 2.5, 0.3, cluster_size=M, whole_cluster_rows=whole) as e:
+            e.upload(x, y, z)
+            g = e.force(ap.KERNEL_CLUSTER_FP64, globals=True)
+            res.append((g, e.download()))
+    (ga, fa), (gb, fb) = res
+    for k in ("fx", "fy", "fz"):
+        assert np.array_equal(np.isnan(fa[k]), np.isnan(fb[k])), k
+        ok = ~np.isnan(fb[k])
+        assert np.max(np.abs(fa[k][ok] - fb[k][ok]), initial=0.0) <= TOL * np.max(np.abs(fb[k][ok]), initial=1.0), k
+    if not all(np.isnan(bad)):  # (with no coordinate at all it may stand alone in a cluster without a box)
+        assert any(np.isnan(fa[k][at]) for k in ("fx", "fy", "fz"))
+    assert ga.pair_count == gb.pair_count
+    assert np.isnan(ga.virial) == np.isnan(gb.virial)
 
 
 @pytest.mark.parametrize("M", [4, 8])
