@@ -69,7 +69,7 @@ __device__ inline int lc_test(int t, int npad, int lane, const double *s_x, cons
     }
 #pragma unroll
     for (int q = 0; q < NT; ++q) {
-      const bool hit = dr2[q] <= rc2;
+      const bool hit = !(dr2[q] > rc2);  // (also where it is not a number)
       const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
       int at = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, cnt[q]));
       asm volatile("" : "+v"(at));  // computed by every lane: the select below stays a select
@@ -180,7 +180,8 @@ __global__ __launch_bounds__(kLcThreads, 4) void k_force_lc_fp64(
       const int64_t mi = mine ? i0 + mq : ib;
       const double mx = x[mi], my = y[mi], mz = z[mi];
       const int mt = MIX ? type[mi] : 0;
-      double ax = 0., ay = 0., az = 0., ae = 0., av = 0.;
+      // (not a number where the particle's position is not finite, as the sums over its pairs then are)
+      double ax = mx - mx, ay = my - my, az = mz - mz, ae = 0., av = ax + ay + az;
       // the queued hits through the pair term
       auto flush = [&]() {
         lds_wave_sync();
@@ -213,7 +214,7 @@ __global__ __launch_bounds__(kLcThreads, 4) void k_force_lc_fp64(
           az += drz * fac;
           if (globals) {
             ae += pair ? eps24 * (lj6 * lj6 - lj6) + shift6 : 0.;
-            av += pair ? dr2 * fac : 0.;
+            av += dr2 * fac;
           }
           hits += pair ? 1 : 0;
         }
@@ -236,7 +237,10 @@ __global__ __launch_bounds__(kLcThreads, 4) void k_force_lc_fp64(
             if (MIX) s_t[pre + k] = type[b + k];
           }
         }
-        if (stage && tid < npad - nj) s_x[nj + tid] = s_y[nj + tid] = s_z[nj + tid] = kLcFar;
+        if (stage && tid < npad - nj) {
+          s_x[nj + tid] = s_y[nj + tid] = s_z[nj + tid] = kLcFar;
+          if (MIX) s_t[nj + tid] = 0;  // (a hit of a particle whose position is not a number)
+        }
         if (stage) __syncthreads();
         int t = 0;
         while (t < npad && nt > 0) {
