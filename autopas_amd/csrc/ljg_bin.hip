@@ -38,23 +38,28 @@ __global__ void k_cell_scatter(int64_t nslots, const int32_t *__restrict__ cell_
 // order so the layout (and with it every floating-point summation order downstream) is reproducible.
 // A thread per member counts the members of its cell with a smaller id (equal ids: a smaller index, so that no two
 // share a place) and writes itself to that place: independent loads of the cell's few entries, instead of a serial
-// sort per cell.
+// sort per cell.  The first member of a cell of more than `above` also reports their number.
 __global__ void k_cell_order_by_id(int64_t n, const int32_t *__restrict__ items, const int32_t *__restrict__ cell_of,
                                    const int64_t *__restrict__ start, const int64_t *__restrict__ id,
-                                   int32_t *__restrict__ sorted) {
+                                   int32_t *__restrict__ sorted, int32_t *__restrict__ longest, int32_t above) {
   const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const int32_t v = items[k];
   const int32_t c = cell_of[v];
   const int64_t b = start[c], e = start[c + 1];
-  const int64_t key = id ? id[v] : v;  // without ids: the index
   int64_t r = 0;
-  for (int64_t m = b; m < e; ++m) {
-    const int32_t o = items[m];
-    const int64_t k2 = id ? id[o] : o;
-    r += (k2 < key) | ((k2 == key) & (o < v)) ? 1 : 0;
+  if (id) {
+    const int64_t key = id[v];
+    for (int64_t m = b; m < e; ++m) {
+      const int32_t o = items[m];
+      const int64_t k2 = id[o];
+      r += (k2 < key) | ((k2 == key) & (o < v)) ? 1 : 0;
+    }
+  } else {  // the index
+    for (int64_t m = b; m < e; ++m) r += items[m] < v ? 1 : 0;
   }
   sorted[b + r] = v;
+  if (r == 0 && e - b > above && e - b > *static_cast<volatile int32_t *>(longest)) atomicMax(longest, (int32_t)(e - b));
 }
 
 // Cell of each particle in upload order (inspection).
@@ -102,10 +107,10 @@ void lc_bin(Ctx &c) {
   c.cell_of.ensure(ns);
   c.rank.ensure(ns);
   c.perm.ensure(ns);
-  c.cell_count.ensure(ncells + 1);
+  c.cell_count.ensure(ncells + 2);  // and the fullest cell's
   c.cell_start.ensure(ncells + 1);
   StateView s = view(c.st[c.cur]);
-  LJG_HIP(hipMemsetAsync(c.cell_count.p, 0, (ncells + 1) * sizeof(int32_t), c.stream));
+  LJG_HIP(hipMemsetAsync(c.cell_count.p, 0, (ncells + 2) * sizeof(int32_t), c.stream));
   hipLaunchKernelGGL(k_cell_hist, dim3(blocks_for(ns, 256)), dim3(256), 0, c.stream, ns, s.x, s.y, s.z, s.orig, g,
                      c.cell_of.p, c.rank.p, c.cell_count.p);
   LJG_HIP(hipGetLastError());
@@ -115,7 +120,7 @@ void lc_bin(Ctx &c) {
   LJG_HIP(hipGetLastError());
   c.cell_sorted.ensure((size_t)c.n);
   hipLaunchKernelGGL(k_cell_order_by_id, dim3(blocks_for(c.n, 256)), dim3(256), 0, c.stream, c.n, c.perm.p,
-                     c.cell_of.p, c.cell_start.p, s.id, c.cell_sorted.p);
+                     c.cell_of.p, c.cell_start.p, s.id, c.cell_sorted.p, c.cell_count.p + ncells + 1, kLcWholeCell);
   LJG_HIP(hipGetLastError());
   std::swap(c.perm, c.cell_sorted);
   c.cell_of_particle.ensure(c.n);
@@ -134,14 +139,14 @@ void lc_bin(Ctx &c) {
 
 void cell_bin_launch(hipStream_t st, int64_t n, const double *x, const double *y, const double *z, const CellGeom &g,
                      int32_t *cell_of, int32_t *rank, int32_t *count, const int64_t *start, int32_t *items,
-                     const int64_t *id, int32_t *sorted, int phase) {
+                     const int64_t *id, int32_t *sorted, int32_t *longest, int phase) {
   if (phase == 0) {
     hipLaunchKernelGGL(k_cell_hist, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, x, y, z,
                        (const int32_t *)nullptr, g, cell_of, rank, count);
   } else {
     hipLaunchKernelGGL(k_cell_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, cell_of, rank, start, items);
     hipLaunchKernelGGL(k_cell_order_by_id, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, items, cell_of, start, id,
-                       sorted);
+                       sorted, longest, kLcWholeCell);
   }
   LJG_HIP(hipGetLastError());
 }

@@ -302,7 +302,7 @@ struct Ctx {
   CellGeom cg{};
   int64_t ncells = 0;
   DevBuf<int32_t> cell_of;      // per slot
-  DevBuf<int32_t> cell_count;   // ncells (+1)
+  DevBuf<int32_t> cell_count;   // ncells + 1, then what the fullest cell holds if that is above kLcWholeCell
   DevBuf<int64_t> cell_start;   // ncells + 1
   DevBuf<int32_t> rank;         // per slot, rank inside cell/tower from the atomic histogram
   DevBuf<int32_t> perm;         // gather map new slot -> old slot
@@ -484,15 +484,17 @@ void lc_bin(Ctx &c);                       // ljg_bin.hip
 CellGeom make_cell_geom(const double lo[3], const double hi[3], double ilen, int64_t *ncells);
 // LinkedCells binning of n particles on explicit buffers (ljg_bin.hip): phase 0 = cell and rank of every
 // particle (count must be zero), phase 1 = scatter into the cells by rank and order each cell by id (index
-// when id is null) into sorted.
+// when id is null) into sorted; *longest (zero before): the fullest cell's number, if above kLcWholeCell.
+constexpr int32_t kLcWholeCell = 40;
 void cell_bin_launch(hipStream_t st, int64_t n, const double *x, const double *y, const double *z, const CellGeom &g,
                      int32_t *cell_of, int32_t *rank, int32_t *count, const int64_t *start, int32_t *items,
-                     const int64_t *id, int32_t *sorted, int phase);
+                     const int64_t *id, int32_t *sorted, int32_t *longest, int phase);
 // The plain FP64 linked-cells kernel on explicit buffers in cell order (ljg_lc.hip); block partials into
-// pe/pv/ph (lc_force_blocks(g) of them).
-int64_t lc_force_blocks(const CellGeom &g);
-void lc_force_launch(hipStream_t st, const double *x, const double *y, const double *z, const int32_t *type,
-                     const int64_t *cell_start, const CellGeom &g, double rc2, int32_t ntypes, const double *tab,
+// pe/pv/ph (lc_force_blocks(n, g) of them).
+int64_t lc_force_blocks(int64_t n, const CellGeom &g);
+void lc_force_launch(hipStream_t st, int64_t n, const double *x, const double *y, const double *z,
+                     const int32_t *type, const int32_t *cell_of, const int64_t *cell_start,
+                     const int32_t *longest, const CellGeom &g, double rc2, int32_t ntypes, const double *tab,
                      double eps24, double sig2, double shift6, double *fx, double *fy, double *fz, double *pe,
                      double *pv, int64_t *ph, bool globals, unsigned long long *acc, SkipIf skip,
                      Owned owned = Owned{nullptr, 0});

@@ -47,7 +47,7 @@ ScratchLayout layout_for(int64_t n, int64_t ncells, int32_t ntypes, int64_t scan
   l.type = take(4 * un);
   l.xw = take(24 * un);  // wrapped positions in caller order, later the forces in cell order
   l.xs = take(24 * un);  // positions in cell order
-  l.count = take(4 * (size_t)(ncells + 1));
+  l.count = take(4 * (size_t)(ncells + 2));  // of the cells, and the fullest one's
   l.start = take(8 * (size_t)(ncells + 1));
   l.scan = take(8 * (size_t)scan_len);
   l.pe = take(8 * (size_t)nblocks);
@@ -144,7 +144,7 @@ ljg_status ljg_force_lc_noalloc(const ljg_params *params, int32_t ntypes, const 
   int64_t ncells = 0;
   const CellGeom g = make_cell_geom(params->box_min, params->box_max, ilen, &ncells);
   if (ncells > LJG_NOALLOC_MAX_CELLS) return LJG_ERR_CAPACITY;
-  const int64_t nblocks = lc_force_blocks(g);
+  const int64_t nblocks = lc_force_blocks(n, g);
   const int64_t slen = scan_tmp_len(ncells);
   const ScratchLayout l = layout_for(n, ncells, ntypes, slen, nblocks);
   if (l.total > (size_t)LJG_NOALLOC_SCRATCH_BYTES) return LJG_ERR_CAPACITY;
@@ -204,18 +204,20 @@ ljg_status ljg_force_lc_noalloc(const ljg_params *params, int32_t ntypes, const 
     }
     // every counter that must start at zero is cleared here by a kernel (the array keeps the last call's
     // contents)
-    hipLaunchKernelGGL(k_na_fill, dim3(blocks_for(ncells + 1, 256)), dim3(256), 0, st, ncells + 1, count);
+    hipLaunchKernelGGL(k_na_fill, dim3(blocks_for(ncells + 2, 256)), dim3(256), 0, st, ncells + 2, count);
     hipLaunchKernelGGL(k_na_wrap, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, x, y, z, wrap_args(*params), xw);
     LJG_HIP(hipGetLastError());
-    cell_bin_launch(st, n, xw, xw + n, xw + 2 * n, g, cell_of, rank, count, nullptr, nullptr, nullptr, nullptr, 0);
+    cell_bin_launch(st, n, xw, xw + n, xw + 2 * n, g, cell_of, rank, count, nullptr, nullptr, nullptr, nullptr,
+                    nullptr, 0);
     exclusive_scan_i32_to_i64_on(st, count, start, ncells, scan, slen);
-    cell_bin_launch(st, n, nullptr, nullptr, nullptr, g, cell_of, rank, count, start, items, id, sorted, 1);
+    cell_bin_launch(st, n, nullptr, nullptr, nullptr, g, cell_of, rank, count, start, items, id, sorted,
+                    count + ncells + 1, 1);
     hipLaunchKernelGGL(k_na_gather, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, sorted, xw, type, ntypes, cell_of, xs,
                        ts, cells);
     LJG_HIP(hipGetLastError());
     // the forces in cell order go where the wrapped caller-order positions were
     double *fs = xw;
-    lc_force_launch(st, xs, xs + n, xs + 2 * n, ts, start, g, rc2, ntypes, tab, e24[0], s2[0], sh6[0], fs, fs + n,
+    lc_force_launch(st, n, xs, xs + n, xs + 2 * n, ts, cells, start, count + ncells + 1, g, rc2, ntypes, tab, e24[0], s2[0], sh6[0], fs, fs + n,
                     fs + 2 * n, pe, pv, ph, globals != nullptr, nullptr, SkipIf{nullptr, 0});
     hipLaunchKernelGGL(k_na_scatter, dim3(blocks_for(n, 256)), dim3(256), 0, st, n, sorted, fs, fx, fy, fz);
     LJG_HIP(hipGetLastError());
