@@ -298,9 +298,9 @@ ljg_status ljg_create(const ljg_params *p, ljg_ctx **out) {
     LJG_HIP(hipHostMalloc((void **)&c.host_flag, 4 * sizeof(int32_t), hipHostMallocMapped | hipHostMallocCoherent));
     std::memset(c.host_flag, 0, 4 * sizeof(int32_t));
     LJG_HIP(hipHostGetDevicePointer((void **)&c.host_flag_dev, c.host_flag, 0));
-    LJG_HIP(hipHostMalloc((void **)&c.pin_mark, (1 + kMarkWords) * sizeof(unsigned long long),
+    LJG_HIP(hipHostMalloc((void **)&c.pin_mark, (1 + kMarkProgress) * sizeof(unsigned long long),
                           hipHostMallocMapped | hipHostMallocCoherent));
-    std::memset(c.pin_mark, 0, (1 + kMarkWords) * sizeof(unsigned long long));
+    std::memset(c.pin_mark, 0, (1 + kMarkProgress) * sizeof(unsigned long long));
     LJG_HIP(hipHostGetDevicePointer((void **)&c.pin_mark_dev, c.pin_mark, 0));
     c.flag.ensure(4);
     hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(64), 0, c.stream, (int64_t)4, c.flag.p);

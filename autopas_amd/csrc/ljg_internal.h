@@ -453,11 +453,10 @@ struct Ctx {
   size_t pin_seg_cap = 0;
   int32_t *pin_flags = nullptr;
   size_t pin_flags_cap = 0;
-  // Pinned, device-mapped staging of uploads and downloads (bytes pin_stage_cap), and a download's progress
-  // word.  stage_mark: kernels may read the staging buffer until a marker of at least this number was seen.
+  // Pinned, device-mapped staging of uploads and downloads (bytes pin_stage_cap; a download's progress word is
+  // pin_mark[kMarkProgress]).  stage_mark: kernels may read the staging buffer until a marker of at least this number was seen.
   double *pin_stage = nullptr, *pin_stage_dev = nullptr;
   size_t pin_stage_cap = 0;
-  unsigned long long *pin_progress = nullptr, *pin_progress_dev = nullptr;
   unsigned long long progress_seq = 0, stage_mark = 0, mark_seen = 0;
   // second buffers an edit of the ensemble writes the moved layout into, then swaps in
   DevBuf<float4> pos32_alt, pos32n_alt;
@@ -568,6 +567,7 @@ void md_set_positions(Ctx &c, const double *pos, const double *vel);
 // which the host spins (a stream synchronisation wakes the host tens of microseconds after the work
 // ends).  After 2 s of spinning it synchronises the stream instead.  ljg_md.hip
 constexpr int kMarkWords = 63;                          // words one marker read returns at most
+constexpr int kMarkProgress = 1 + kMarkWords;           // the word behind them: a download's progress
 constexpr int kMarkFlagBoxes = 2 * (kMarkWords - 1);    // ensembles up to this size read box flags with it
 // Waits for the work queued on the stream and reads n words of src, then n2 words of src2 (device
 // memory), into out, with one marker kernel whose pinned word the host polls.

@@ -13,10 +13,10 @@
 #include <thread>
 
 #include "ljg_internal.h"
+#include "ljg_stage.h"
 
 namespace ljg {
 
-constexpr size_t kRingBytes = 16u << 20;
 constexpr int kMoveThreads = 256;
 
 // Pinned memory is read and written at system scope: kernels that follow each other in a stream meet at the
@@ -64,29 +64,20 @@ static double *stage_buffer(Ctx &c, size_t bytes) {
   }
   c.stage_mark = 0;
   if (c.pin_stage_cap < bytes) {
+    const size_t cap = stage_capacity(bytes, c.pin_stage_cap);
     if (c.pin_stage) LJG_HIP(hipHostFree(c.pin_stage));
     c.pin_stage = nullptr;
     c.pin_stage_cap = 0;
-    size_t cap = 64u << 10;
-    while (cap < bytes) cap <<= 1;
     LJG_HIP(hipHostMalloc((void **)&c.pin_stage, cap, hipHostMallocMapped | hipHostMallocCoherent));
     c.pin_stage_cap = cap;
     LJG_HIP(hipHostGetDevicePointer((void **)&c.pin_stage_dev, c.pin_stage, 0));
-    if (!c.pin_progress) {
-      LJG_HIP(hipHostMalloc((void **)&c.pin_progress, sizeof(unsigned long long),
-                            hipHostMallocMapped | hipHostMallocCoherent));
-      *c.pin_progress = 0;
-      LJG_HIP(hipHostGetDevicePointer((void **)&c.pin_progress_dev, c.pin_progress, 0));
-    }
   }
   return c.pin_stage;
 }
 
 void release_stage(Ctx &c) {
   if (c.pin_stage) (void)hipHostFree(c.pin_stage);
-  if (c.pin_progress) (void)hipHostFree(c.pin_progress);
   c.pin_stage = nullptr;
-  c.pin_progress = nullptr;
 }
 
 // dst (may be null) = src; whether every value lies in [lo, hi] (NaN does not).  Without an early exit, so that the
@@ -293,9 +284,7 @@ struct Download {
 };
 }  // namespace
 
-// Chunks of an eighth (at least 256 KiB, where a chunk's transfer takes as long as its launch; at most 2 MiB), and
-// from 24 MiB on three helpers: one thread copies about 30 GB/s, the link carries 55.  Downloads of 63, 72 and 144 MB: 3.50, 3.74 and 7.36 -> 1.42, 1.55 and 2.95 ms.
-constexpr size_t kMinChunk = (256u << 10) / sizeof(double), kMaxChunk = (2u << 20) / sizeof(double);
+// From 24 MiB on with three helpers: one thread copies about 30 GB/s, the link carries 55.  Downloads of 63, 72 and 144 MB: 3.50, 3.74 and 7.36 -> 1.42, 1.55 and 2.95 ms.
 constexpr size_t kHelpedBytes = 24u << 20;
 constexpr int kHelpers = 3;
 
@@ -304,15 +293,14 @@ void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs
   Download &d = *shared;
   d.count = count;
   d.total = 9 * count;
-  d.chunk = (d.total + 7) / 8;
-  d.chunk = d.chunk < kMinChunk ? kMinChunk : d.chunk > kMaxChunk ? kMaxChunk : d.chunk;
+  d.chunk = download_chunk(d.total);
   d.nchunks = (int)((d.total + d.chunk - 1) / d.chunk);
   const size_t bytes = (d.nchunks > 1 ? (size_t)d.nchunks * d.chunk : d.total) * sizeof(double);
   d.ring = stage_buffer(c, bytes < kRingBytes ? bytes : kRingBytes);
   d.slots = (int)(c.pin_stage_cap / (d.chunk * sizeof(double)));
   d.slots = d.slots < 1 ? 1 : d.slots;  // (a single chunk shorter than kMinChunk)
   std::copy(outs, outs + 9, d.outs);
-  d.progress = c.pin_progress;
+  d.progress = c.pin_mark + kMarkProgress;
   d.base = c.progress_seq;
   c.progress_seq += (unsigned long long)d.nchunks + 1;
   d.done.reset(new std::atomic<char>[(size_t)d.nchunks]);
@@ -324,7 +312,7 @@ void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs
            (queued == d.nchunks || queued < d.slots || d.done[queued - d.slots].load(std::memory_order_acquire))) {
       const size_t b = (size_t)queued * d.chunk, n = queued == d.nchunks ? 0 : std::min(d.chunk, d.total - b);
       move_launch<true>(c, dev + (n ? b : 0), c.pin_stage_dev + (n ? (size_t)(queued % d.slots) * d.chunk : 0), n,
-                  queued > 0 ? c.pin_progress_dev : nullptr, d.base + (unsigned long long)queued);
+                  queued > 0 ? c.pin_mark_dev + kMarkProgress : nullptr, d.base + (unsigned long long)queued);
       ++queued;
     }
   };
