@@ -325,6 +325,7 @@ ljg_status ljg_destroy(ljg_ctx *h) {
   (void)hipSetDevice(c.device);
   if (c.stream) (void)hipStreamSynchronize(c.stream);
   if (c.side) (void)hipStreamSynchronize(c.side);
+  release_stage(c);
   for (auto &s : c.st) s.release();
   c.cell_of.release(); c.cell_count.release(); c.cell_start.release(); c.rank.release(); c.perm.release();
   c.cell_of_particle.release(); c.tower_of.release(); c.tower_count.release(); c.tower_start.release();
@@ -342,7 +343,6 @@ ljg_status ljg_destroy(ljg_ctx *h) {
   if (c.host_flag) (void)hipHostFree(c.host_flag);
   if (c.pin_mark) (void)hipHostFree(c.pin_mark);
   if (c.pin_seg) (void)hipHostFree(c.pin_seg);
-  release_stage(c);
   if (c.pin_flags) (void)hipHostFree(c.pin_flags);
   for (auto e : c.event_pool) (void)hipEventDestroy(e);
   if (c.ev0) (void)hipEventDestroy(c.ev0);

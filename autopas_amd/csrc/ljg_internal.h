@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "../../include/ljgpu.h"
+#include "ljg_ring.h"
 
 namespace ljg {
 
@@ -457,6 +458,7 @@ struct Ctx {
   // pin_mark[kMarkProgress]).  stage_mark: kernels may read the staging buffer until a marker of at least this number was seen.
   double *pin_stage = nullptr, *pin_stage_dev = nullptr;
   size_t pin_stage_cap = 0;
+  Helpers helpers;                    // of downloads
   unsigned long long progress_seq = 0, stage_mark = 0, mark_seen = 0;
   // second buffers an edit of the ensemble writes the moved layout into, then swaps in
   DevBuf<float4> pos32_alt, pos32n_alt;

@@ -6,11 +6,8 @@
 // buffer, which the kernels read directly, and downloads run as a ring of chunks: the device writes a chunk
 // into the buffer while the host copies earlier ones out, from a few threads when there is much to copy.
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 #include <cstring>
-#include <memory>
-#include <thread>
 
 #include "ljg_internal.h"
 #include "ljg_stage.h"
@@ -76,6 +73,7 @@ static double *stage_buffer(Ctx &c, size_t bytes) {
 }
 
 void release_stage(Ctx &c) {
+  c.helpers.join();
   if (c.pin_stage) (void)hipHostFree(c.pin_stage);
   c.pin_stage = nullptr;
 }
@@ -234,57 +232,8 @@ const double *stage_positions(Ctx &c, const double *const pos[3], const double *
   return dev;
 }
 
-// The copy out of a download: `total` doubles on the device, nine arrays of `count` back to back (null outputs
-// are left out), as chunks through the ring.  Chunk k occupies ring slot k mod slots; it is queued once chunk
-// k - slots has been copied out, and is complete when the progress word passes it.  This thread queues the
-// chunks; all threads take chunks in order and copy them out.  The helpers are not joined but share this object: one
-// that the scheduler lets start late (the caller's own worker threads may be spinning on every core: 2 to 3 ms were
-// seen) finds no chunk left and ends without touching the buffers, and only chunks that were taken are waited for.
-namespace {
-struct Download {
-  const double *ring;
-  size_t count, chunk, total;
-  int nchunks, slots;
-  double *outs[9];
-  volatile unsigned long long *progress;
-  unsigned long long base;  // progress holds base + the number of complete chunks
-  std::unique_ptr<std::atomic<char>[]> done;  // 1: copied out, 2: given up
-  std::atomic<int> next{0};
-  std::atomic<bool> abort{false};
-
-  bool ready(int k) const {
-    const unsigned long long p = *progress;
-    return p > base + (unsigned long long)k && p <= base + (unsigned long long)nchunks;
-  }
-  void copy_out(int k) {
-    std::atomic_thread_fence(std::memory_order_acquire);
-    const size_t b = (size_t)k * chunk, e = b + chunk < total ? b + chunk : total;
-    const double *src = ring + (size_t)(k % slots) * chunk;
-    for (size_t i = b; i < e;) {
-      const size_t a = i / count, stop = (a + 1) * count < e ? (a + 1) * count : e;
-      if (outs[a]) std::memcpy(outs[a] + (i - a * count), src + (i - b), (stop - i) * sizeof(double));
-      i = stop;
-    }
-    done[k].store(1, std::memory_order_release);
-  }
-  void help() {
-    for (;;) {
-      const int k = next.fetch_add(1);
-      if (k >= nchunks) return;
-      for (unsigned spins = 0; !ready(k); ++spins) {
-        if (abort.load(std::memory_order_relaxed)) {
-          done[k].store(2, std::memory_order_release);
-          return;
-        }
-        if (spins > 64) std::this_thread::yield();
-      }
-      copy_out(k);
-    }
-  }
-};
-}  // namespace
-
-// From 24 MiB on with three helpers: one thread copies about 30 GB/s, the link carries 55.  Downloads of 63, 72 and 144 MB: 3.50, 3.74 and 7.36 -> 1.42, 1.55 and 2.95 ms.
+// From 24 MiB on with three helpers: one thread copies about 30 GB/s, the link carries 55.  Downloads of 63, 72 and
+// 144 MB: 3.50, 3.74 and 7.36 -> 1.42, 1.55 and 2.95 ms.
 constexpr size_t kHelpedBytes = 24u << 20;
 constexpr int kHelpers = 3;
 
@@ -321,7 +270,7 @@ void download_arrays(Ctx &c, const double *dev, size_t count, double *const outs
     if (d.total * sizeof(double) >= kHelpedBytes) {
       for (int k = 0; k < kHelpers; ++k) {
         try {
-          std::thread([shared]() { shared->help(); }).detach();
+          c.helpers.start([shared]() { shared->help(); });
         } catch (const std::exception &) {
           break;  // no more threads to be had: this one copies the rest
         }
