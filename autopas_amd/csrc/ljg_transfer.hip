@@ -94,11 +94,11 @@ static bool copy_checked(double *__restrict__ dst, const double *__restrict__ sr
 }
 
 bool region_check(const Ctx &c, int64_t n, const double *const src[3], double *const dst[3]) {
-  const double inf = __builtin_inf(), ilen = c.prm.cutoff + c.prm.skin;
+  const double ilen = c.prm.cutoff + c.prm.skin;
   for (int d = 0; d < 3; ++d) {
     if (!c.open) {
       if (dst[d]) std::memcpy(dst[d], src[d], (size_t)n * sizeof(double));
-    } else if (!copy_checked(dst[d], src[d], (size_t)n, c.open ? c.open_min[d] - ilen : -inf, c.open_max[d] + ilen)) {
+    } else if (!copy_checked(dst[d], src[d], (size_t)n, c.open_min[d] - ilen, c.open_max[d] + ilen)) {
       return false;
     }
   }
