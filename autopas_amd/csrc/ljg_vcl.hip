@@ -666,11 +666,13 @@ __global__ __launch_bounds__(256) void k_copy_box_clusters(int64_t nitems, Segs 
 // each with the gap before it), and these were seven: clear, histogram, offsets, their marker, scatter, sort,
 // and a second clear.  The sizes go to the host's marker words as soon as they are known.  Towers longer than
 // kSmallTower are left to the sorts of the general path, which find the histogram's results in place.
-// A job of 700 particles with 150 steps and 15 builds: 2805 -> 2385 us with the other launches saved.
+// A job of 700 particles with 150 steps and 15 builds: 2805 -> 2385 us with the other launches saved.  Counting takes as
+// long as the launches it saves in towers of about 150 (3900 particles in 9 x 9 x 64, M 8, 156 to a tower: 114 us a build,
+// with the general path's sorts 85; 12 x 12 x 36, 108 on average: 97 and 81).
 constexpr int kSmallThreads = 1024;
 constexpr int kSmallSlots = 4096;   // old slots (padding included); also bounds the offsets below 2^16
 constexpr int kSmallTowers = kSmallThreads;
-constexpr int kSmallTower = 256;
+constexpr int kSmallTower = 128;
 
 __global__ __launch_bounds__(kSmallThreads) void k_tower_small(
     int32_t nslots, double *__restrict__ x, double *__restrict__ y, double *__restrict__ z,

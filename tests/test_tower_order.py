@@ -110,3 +110,27 @@ def test_cells_keep_particles_of_equal_ids(kernel, n, L):
             f = e.download()
             for k, v in zip("xyz", p):
                 assert np.array_equal(f[k], v), k
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 4, 8])
+@pytest.mark.parametrize("column", [127, 128, 129])
+def test_small_build_where_it_leaves_the_sorts_to_others(oracle, M, column):
+    announce(f"small build, M={M}: a column of {column} particles and more in its tower")
+    rng = np.random.default_rng(M + column)
+    box, n = (9.0, 9.0, 60.0), 700
+    x, y, z = (rng.uniform(-0.5 * b, 1.5 * b, n) for b in box)
+    z[1::3] = z[::3][:len(z[1::3])]
+    x[:column], y[:column] = 0.1, 0.1
+    x[column:] = 3.5 + 0.4 * (x[column:] % 9.0) / 9.0 * 10.0  # the others: not in that tower
+    ids = rng.permutation(n).astype(np.int64)
+    wx, wy, wz = oracle.wrap(x, y, z, (0, 0, 0), box)
+    r = oracle.vcl_periodic(wx, wy, wz, ids, (0, 0, 0), box, 2.8, M)
+    assert np.max(np.bincount(r["cluster_tower"])) * M >= column
+    with ap.Engine((0.0, 0.0, 0.0), box, 2.5, 0.3, cluster_size=M) as e:
+        e.upload(x, y, z, id=ids)
+        for _ in range(2):
+            e.build_pairs()
+            g = e.clusters()
+            for k in ("slot_particle", "cluster_tower", "list_offsets", "list_j", "list_shift", "bbox"):
+                assert np.array_equal(g[k], r[k]), k
