@@ -138,9 +138,11 @@ __global__ __launch_bounds__(kFThreads, (XR && !MIX && !GLOB) ? 4 : 1) void k_fo
       ic = __builtin_amdgcn_readfirstlane(ic);
       part = __builtin_amdgcn_readfirstlane(part);
     }
-    // The slot of the group's member q.  (Formed from ic where it is used: one 64-bit first slot kept from here took
-    // two registers more than five wavefronts per SIMD have, M 4: 1024 boxes of an ensemble 913 -> 970 us a step.)
-    auto slot = [&](int q) { return (int64_t)ic * MC + (S > 1 ? part + q : q); };
+    // The slot of the group's member q.  (Unsplit it is formed from ic where it is used: one 64-bit first slot kept from
+    // here took two registers more than five wavefronts per SIMD have, M 4: 1024 boxes of an ensemble 913 -> 970 us a
+    // step.)
+    const int64_t m0 = (int64_t)ic * MC + part;
+    auto slot = [&](int q) { return S > 1 ? m0 + q : (int64_t)ic * MC + q; };
     if (!wq.ctr) ++tile;
   if (ic >= 0) {
     float xi[M], yi[M], zi[M];
