@@ -390,8 +390,8 @@ __device__ __forceinline__ void lc_slice(const LcIn &in, LcShared<MIX> &sh, int6
 
 // Workgroups are dealt to the 8 XCDs in turn: an XCD takes chunks of consecutive cells or ranges, so that neighbouring
 // cells meet in its L2, and chunks from all over the box, so that a film across it keeps every XCD busy (the
-// 2.0M-particle slab with an eighth of the cells per XCD 7.6 ms a step, now 3.8; 500,000 in a liquid 385 -> 373 us a
-// call).
+// 2.0M-particle slab with an eighth of the cells per XCD 7.6 ms a step, then 3.8 (with lanes for the gas 2.1); 500,000
+// in a liquid 385 -> 373 us a call).
 template <bool MIX>
 __global__ __launch_bounds__(kLcThreads, 4) void k_force_lc_cells(LJG_LC_ARGS, LcCells cells) {
   if (skip_launch(sk)) return;

@@ -942,9 +942,9 @@ __global__ __launch_bounds__(kListThreads) void k_cluster_lists_tower(
 // fixed capacity; the length is the full one even when it exceeds it, so the host can grow it and build
 // again.  The next visit's boxes are loaded into registers while this one runs from LDS.
 // The pass is bound by LDS: with FP64 boxes in LDS as records of 48 bytes the lanes, each at its own place
-// in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 118 us, the 2.0M
-// particle slab 308 -> 121.  Workgroups are dealt so that an XCD takes chunks of neighbouring
-// towers.
+// in the tower, met in few banks and every test moved twice the bytes: 10^6 particles 151 -> 106 us, the 2.0M
+// particle slab 308 -> 150; with the columns as well 95 and 121 to 126.  Workgroups are dealt so that an XCD takes
+// chunks of neighbouring towers.
 constexpr int kJclChunk = 2 * kWave;
 
 struct JclGeom {
